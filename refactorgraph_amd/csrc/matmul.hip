@@ -8,22 +8,13 @@
 // F64) in an order that differs from the CPU loop, so results agree to rounding, not bit for bit.
 // The bias is read through strides inside the epilogue instead of being expanded into Y first.
 //
-// Fast path (FP16 / BF16, A not transposed, m and n multiples of 256, k multiple of 64): one
-// 256x256 tile of Y per workgroup of four wavefronts (128x128 each, 4x4 blocks of
-// v_mfma_f32_32x32x16), k-tiles of 64 copied from global memory straight into two LDS buffers
-// with global_load_lds_dwordx4, fragments double buffered by k-step, one MFMA per scheduling slot:
-// the structure of the MatMulInteger kernel with 16-bit operands.
-//   A tile (and B given as [n,k]): rows of 128 bytes, chunk c of row r at chunk position
-//           c ^ (r & 7) ^ ((r >> 3) & 1); fragments by 128-bit reads.
-//   B given as [k,n]: 64 k-rows of 512 bytes, chunk c of k-row r at c ^ swz(r & 3); the operand
-//           (8 consecutive k of one column per lane) is formed by two ds_read_b64_tr_b16, which
-//           transpose 16-bit elements inside 16 lanes (lane i receives element i % 4 of the 8-byte
-//           pieces addressed by lanes i / 4, i / 4 + 4, i / 4 + 8, i / 4 + 12).
+// FP16 / BF16, A not transposed, k a multiple of 64: mm_ring, tiles of 64 x 64 to 256 x 256 of Y whose operands are copied
+// straight into a ring of LDS stages; a cost model picks the shape, or two of them for one product.
 // Few rows of A with the weights as [n, k] (a decode step) are bound by reading the weights once: one row goes
 // through a matrix-vector kernel on the vector ALUs, 2 to 16 rows through 4x4x4 block products whose operands
 // come straight from global memory, up to 255 rows through 32x32x16 products with the tiles passed through LDS.
 // With the weights as [k, n] the block products sit behind a transposition in registers (32 rows a pass).  Where
-// those passes would take longer than one launch of the 256 x 256 tiles, fewer than 256 rows run on one row of tiles.
+// those passes would take longer than the tiles, fewer than 256 rows go to the tiles too.
 // F32 (A not transposed) has 128 x 128 tiles of 32x32x2 products and the block-product kernels for few rows.
 // Everything else (F64, transposed A, other shapes) goes through a plain tiled kernel.
 #include <hip/hip_bf16.h>
@@ -230,250 +221,10 @@ template <> struct Mfma<__hip_bfloat16> {
     }
 };
 
-constexpr int BM = 256, BN = 256, BK = 64;   // BK in elements: 128 bytes
-constexpr int M_TILE = 32768;                // one A or B tile in LDS
-constexpr int M_STAGE = 2 * M_TILE;
-
-__device__ __forceinline__ uint32_t n_swizzle(uint32_t r) { return 4 * (r & 1) + 10 * ((r >> 1) & 1); }  // r < 4
-
-// A, B: byte pointers to this workgroup's first row / first column; pitches in bytes.  SHORT_M: A has only
-// a_rows < 256 rows; the tile's rows beyond them are copied from the last one (their results are not stored).
-template <class T, bool TRANS_B, bool SHORT_M>
-__device__ __forceinline__ void mm_tile_loop(f16v (&acc)[4][4], uint8_t *lds0, uint8_t *lds1, const uint8_t *A,
-                                             const uint8_t *B, uint32_t k, uint32_t pitch_a, uint32_t pitch_b,
-                                             uint32_t a_rows) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave >> 1, wn = wave & 1, h = lane >> 5;
-    // copy q < 8: A rows 8 (8 wave + q) .. + 7, this lane row + lane / 8, chunk position lane % 8.
-    // copy 8 + p, B as [n,k]: the same for B's rows (columns of Y); B as [k,n]: k-rows
-    // 2 (8 wave + p) and the next, this lane k-row + lane / 32, chunk position lane % 32.
-    const uint8_t *a_wave = A + static_cast<uint64_t>(wave * 64) * pitch_a;
-    const uint32_t a_lane = (lane >> 3) * pitch_a + 16 * ((lane & 7) ^ (lane >> 3));
-    const uint8_t *b_wave = B + static_cast<uint64_t>(wave * (TRANS_B ? 64 : 16)) * pitch_b;
-    uint32_t b_lane[2];
-    if constexpr (TRANS_B) {
-        b_lane[0] = b_lane[1] = (lane >> 3) * pitch_b + 16 * ((lane & 7) ^ (lane >> 3));
-    } else {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) b_lane[p] = (lane >> 5) * pitch_b + 16 * ((lane & 31) ^ n_swizzle(2 * p + (lane >> 5)));
-    }
-    auto copy = [&](uint8_t *base, uint32_t kt, int q) {
-        const uint8_t *src;
-        uint8_t *dst;
-        if (q < 8) {
-            if constexpr (SHORT_M) {
-                const uint32_t row = wave * 64 + 8 * q + (lane >> 3);
-                src = A + ((row < a_rows ? row : a_rows - 1) * pitch_a + kt * 128 + (16 * ((lane & 7) ^ (lane >> 3) ^ (q & 1))));
-            } else {
-                src = a_wave + (kt * 128 + 8 * q * pitch_a) + (a_lane ^ (16 * (q & 1)));
-            }
-            dst = base + (wave * 8 + q) * 1024;
-        } else if constexpr (TRANS_B) {
-            src = b_wave + (kt * 128 + 8 * (q - 8) * pitch_b) + (b_lane[0] ^ (16 * (q & 1)));
-            dst = base + M_TILE + (wave * 8 + (q - 8)) * 1024;
-        } else {
-            src = b_wave + static_cast<uint64_t>(kt * BK + 2 * (q - 8)) * pitch_b + b_lane[q & 1];
-            dst = base + M_TILE + (wave * 8 + (q - 8)) * 1024;
-        }
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                         (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-    };
-    // A fragment i of k-step ks: row wm 128 + 32 i + lane % 32, chunk 2 ks + h
-    const uint32_t a_off = (wm * 128 + (lane & 31)) * 128 + 16 * (h ^ (lane & 7) ^ ((lane >> 3) & 1));
-    auto read_a = [&](const uint8_t *base, int ks, int i) -> u32x4 {
-        return *reinterpret_cast<const u32x4 *>(base + (a_off ^ (32 * ks)) + i * 4096);
-    };
-    // B fragment j of k-step ks, B as [n,k]: like A with row wn 128 + 32 j + lane % 32.
-    // B as [k,n]: column wn 128 + 32 j + lane % 32, k 16 ks + 8 h .. + 7 in two transposing reads:
-    // lane a of a group of 16 addresses k-row + a / 4, columns 4 (a % 4) .. + 3 of the group's 16.
-    uint32_t b_off;
-    if constexpr (TRANS_B) {
-        b_off = M_TILE + (wn * 128 + (lane & 31)) * 128 + 16 * (h ^ (lane & 7) ^ ((lane >> 3) & 1));
-    } else {
-        const uint32_t a16 = lane & 15, r = a16 >> 2;
-        const uint32_t chunk = wn * 16 + 2 * ((lane >> 4) & 1) + ((a16 & 3) >> 1);  // + 4 j: bits 6-7 of the byte offset
-        b_off = M_TILE + (8 * h + r) * 512 + 16 * (chunk ^ n_swizzle(r)) + 8 * (a16 & 1);
-    }
-    auto read_b = [&](const uint8_t *base, int ks, int j, int half, u32x4 &f) {
-        if constexpr (TRANS_B) {
-            if (half == 0) f = *reinterpret_cast<const u32x4 *>(base + (b_off ^ (32 * ks)) + j * 4096);
-        } else {
-            const s4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (s4 __attribute__((address_space(3))) *)(base + (b_off ^ (64 * j)) + (16 * ks + 4 * half) * 512));
-            const u32x2 w = __builtin_bit_cast(u32x2, v);
-            f[2 * half] = w[0];
-            f[2 * half + 1] = w[1];
-        }
-    };
-
-    const uint32_t k_tiles = k / BK;
-    u32x4 fa[2][4], fb[2][4];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) copy(lds0, 0, q);
-#pragma unroll
-    for (int q = 0; q < 16; ++q) copy(lds1, k_tiles > 1 ? 1 : 0, q);  // k_tiles == 1: tile 0 again, never multiplied
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");  // tile 0 (the 16 older copies)
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fa[0][i] = read_a(lds0, 0, i);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        read_b(lds0, 0, j, 0, fb[0][j]);
-        read_b(lds0, 0, j, 1, fb[0][j]);
-    }
-
-    // Tile kt is in buffer RB, tile kt+1 arrives in WB.
-    auto step = [&](uint32_t kt_, uint8_t *RB, const uint8_t *WB) __attribute__((always_inline)) {
-        const bool more = kt_ + 2 < k_tiles;  // uniform
-        auto slot = [&]<int s>() __attribute__((always_inline)) {
-            // rows walk the columns back and forth, so that only one operand changes between MFMAs
-            constexpr int ks = s / 16, o = s % 16, row = o / 4, col = (row & 1) ? 3 - o % 4 : o % 4;
-            constexpr int cur = ks & 1, nxt = cur ^ 1;
-            if constexpr (s == 48) {
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's part of tile kt+1
-                __syncthreads();                                  // tile kt+1 complete, RB no longer read
-            }
-            acc[row][col] = Mfma<T>::run(fa[cur][row], fb[cur][col], acc[row][col]);
-            const uint8_t *src = ks == 3 ? WB : RB;
-            constexpr int nks = (ks + 1) % 4;
-            if constexpr (o < 4) fa[nxt][o] = read_a(src, nks, o);
-            else if constexpr (o < 12) read_b(src, nks, (o - 4) / 2, (o - 4) % 2, fb[nxt][(o - 4) / 2]);
-            if constexpr (s >= 48) if (more) copy(RB, kt_ + 2, s - 48);
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
-            (slot.template operator()<I>(), ...);
-        }(std::make_integer_sequence<int, 64>{});
-    };
-    uint32_t kt = 0;
-    for (; kt + 2 <= k_tiles; kt += 2) {
-        step(kt, lds0, lds1);
-        step(kt + 1, lds1, lds0);
-    }
-    if (kt < k_tiles) step(kt, lds0, lds1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land after the workgroup's LDS is released
-}
-
-template <class T, bool TRANS_B, bool SHORT_M = false>  // SHORT_M: fewer than 256 rows of A, one row of tiles
-__global__ __launch_bounds__(256, 1) void mm_mfma_256x256(T *__restrict__ y, const T *__restrict__ a,
-                                                          const T *__restrict__ b, Bias bias, uint32_t m, uint32_t k,
-                                                          uint32_t n, float alpha, float beta, uint32_t a_matrix0,
-                                                          uint32_t b_matrix0, uint32_t y_matrix0) {
-    __shared__ __align__(1024) uint8_t lds0[M_STAGE];
-    __shared__ __align__(1024) uint8_t lds1[M_STAGE];
-
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t bz = blockIdx.z;
-    const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
-
-    // XCD-aware tile order: consecutive workgroup ids are dealt round-robin to the 8 XCDs, so
-    // give each XCD a contiguous block of tiles (they then share A row-panels / B column-panels
-    // in that XCD's L2); within it walk tiles in column-major groups of 4 rows to keep panels hot.
-    const uint32_t tiles_n = (n + BN - 1) / BN, tiles_m = (m + BM - 1) / BM, n_tiles = tiles_m * tiles_n;
-    uint32_t t = blockIdx.x;
-    if (n_tiles % 8 == 0) t = (t % 8) * (n_tiles / 8) + t / 8;
-    const uint32_t group = 4 * tiles_n;
-    const uint32_t g = t / group, r = t % group;
-    const uint32_t rows_here = tiles_m - g * 4 < 4 ? tiles_m - g * 4 : 4;
-    const uint32_t tile_m = g * 4 + r % rows_here, tile_n = r / rows_here;
-
-    // m and n need not be multiples of the tile: the last tile of a row or column of tiles is moved back
-    // so that it ends with the matrix (m, n >= 256); the outputs it shares with its neighbour are
-    // computed twice, to the same values
-    const uint32_t tile_row0 = SHORT_M ? 0 : tile_m * BM + BM <= m ? tile_m * BM : m - BM;
-    const uint32_t tile_col0 = tile_n * BN + BN <= n ? tile_n * BN : n - BN;
-    const uint8_t *A = reinterpret_cast<const uint8_t *>(a + (am * m + tile_row0) * k);
-    const T *b_matrix = b + bm * static_cast<uint64_t>(k) * n;
-    const uint8_t *B = reinterpret_cast<const uint8_t *>(
-        TRANS_B ? b_matrix + static_cast<uint64_t>(tile_col0) * k : b_matrix + tile_col0);
-
-    f16v acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-    mm_tile_loop<T, TRANS_B, SHORT_M>(acc, lds0, lds1, A, B, k, 2 * k, TRANS_B ? 2 * k : 2 * n, m);
-
-    // 32x32 accumulator layout: lane holds column (lane % 32); register e holds row
-    // 8*(e/4) + 4*(lane/32) + e%4.  The 128x128 block of a wavefront is transposed through LDS (its
-    // own 32 KiB of the tile buffers, free now) so that Y is written with 128-bit row-contiguous
-    // stores: neighbouring lanes first exchange two of their four rows, so that every lane writes
-    // two adjacent columns (one dword) of two rows; chunk c of row r sits at chunk position c ^ (r & 15).
-    const uint32_t wm = wave >> 1, wn = wave & 1;
-    const uint32_t row0 = tile_row0 + wm * 128, col0 = tile_col0 + wn * 128;
-    const T *C = static_cast<const T *>(bias.ptr);
-    __syncthreads();  // every wavefront has read its last fragments
-    uint8_t *stage = (wave & 2 ? lds1 : lds0) + (wave & 1) * 32768;
-    const bool odd = lane & 1;
-    const uint32_t col_pair = (lane & 31) & ~1u;  // first of the two columns this lane writes
-    // a bias per column (the usual one of a linear layer) is the same for every row: four loads per lane instead
-    // of one per output (4096^3: 133 -> 118 us)
-    const bool column_bias = C && bias.sm == 0;
-    float cb[4] = {0.f, 0.f, 0.f, 0.f};
-    if (column_bias) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cb[j] = beta * up(C[ym * bias.sb + (col0 + j * 32 + (lane & 31)) * bias.sn]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            // any other bias: the sixteen values of a block are requested together, ahead of their use (one at a
-            // time each addition waited for its own load: 4096^3 with a bias per output 160 us)
-            T bv[16];
-            const bool other_bias = C && !column_bias;
-            if (other_bias) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    uint32_t row = row0 + i * 32 + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
-                    if (SHORT_M && row >= m) row = m - 1;
-                    bv[e] = C[ym * bias.sb + row * bias.sm + (col0 + j * 32 + (lane & 31)) * bias.sn];
-                }
-            }
-#pragma unroll
-            for (int eg = 0; eg < 4; ++eg) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = alpha * acc[i][j][4 * eg + e];
-                    if (column_bias) v[e] += cb[j];
-                    else if (other_bias) v[e] += beta * up(bv[4 * eg + e]);
-                }
-                // even lanes keep rows 0 and 1, odd lanes rows 2 and 3 of the group of four
-                const float give0 = odd ? v[0] : v[2], give1 = odd ? v[1] : v[3];
-                const float got0 = __shfl_xor(give0, 1, kWave), got1 = __shfl_xor(give1, 1, kWave);
-                const float lo0 = odd ? got0 : v[0], hi0 = odd ? v[2] : got0;
-                const float lo1 = odd ? got1 : v[1], hi1 = odd ? v[3] : got1;
-                const uint32_t r_first = i * 32 + 8 * eg + 4 * (lane >> 5) + (odd ? 2 : 0);
-                const uint32_t byte_col = 2 * (j * 32 + col_pair);
-                auto put = [&](uint32_t row, float lo, float hi) {
-                    const T pair[2] = {down<T>(lo), down<T>(hi)};
-                    *reinterpret_cast<uint32_t *>(stage + row * 256 + (byte_col ^ (16 * (row & 15)))) =
-                        __builtin_bit_cast(uint32_t, pair);
-                };
-                put(r_first, lo0, hi0);
-                put(r_first + 1, lo1, hi1);
-            }
-        }
-    // (each wavefront reads back only what it wrote itself: no barrier)
-    T *Y = y + (ym * m + row0) * n + col0;
-#pragma unroll
-    for (int it = 0; it < 32; ++it) {
-        const uint32_t idx = lane + 64 * it, row = idx / 16, chunk = idx % 16;
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + row * 256 + 16 * (chunk ^ (row & 15)));
-        if (!SHORT_M || row0 + row < m)
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(Y + static_cast<uint64_t>(row) * n + chunk * 8));
-    }
-}
-
 // ---------------------------------------------------------------- FP16 / BF16: any shape on the matrix cores
 //
-// What the kernels above do not take (fewer than 256 columns, column counts that are no multiple of 8, k that is
-// no multiple of 64, ...) as long as A is not transposed and k is a multiple of 8: 128 x 128 outputs per workgroup
+// What mm_ring does not take (B as [k, n] with a column count that is no multiple of 8, k that is no multiple of 64) as
+// long as A is not transposed and k is a multiple of 8: 128 x 128 outputs per workgroup
 // of four wavefronts (64 x 64 each, 2 x 2 blocks of v_mfma_f32_32x32x16), k in tiles of 64 through two LDS
 // buffers filled from registers that are loaded three tiles ahead.  Both tiles are kept as [row or column][k] with a
 // pitch of 72 elements, so every fragment is one 128-bit read; B as [k, n] is turned on its way into LDS (two k-rows
@@ -483,8 +234,64 @@ __global__ __launch_bounds__(256, 1) void mm_mfma_256x256(T *__restrict__ y, con
 // elements come from five aligned words.
 constexpr int HT = 128, HK = 64, HP = 72, HF = 3;
 constexpr size_t kHalfTiles = 128;   // tiles of 128 rows up to which tiles of 64 rows are launched instead
-constexpr size_t kSmallGrid = 384;  // workgroups up to which these tiles replace the 256 x 256 ones
-constexpr size_t kSkinnyPassesSmall = 12000, kRowsKnPassesSmall = 10500;
+constexpr size_t kSmallGrid = 384;  // workgroups up to which these tiles are weighed against the few-rows kernels
+constexpr size_t kFewRows = 256;     // rows of A below which those kernels are considered
+
+// Stores the MI x NJ blocks of 32 x 32 accumulators of a wavefront, whose first output is (row0, col0) of matrix ym.
+template <class T, int MI, int NJ>
+__device__ __forceinline__ void store_blocks(const f16v (&acc)[MI][NJ], T *__restrict__ y, const Bias &bias, uint64_t ym, uint32_t row0,
+                                             uint32_t col0, uint32_t m, uint32_t n, float alpha, float beta) {
+    const uint32_t lane = threadIdx.x & 63, l32 = lane & 31, kh = lane >> 5;
+    // accumulator: column lane % 32 of the block, register e holds row 8 (e / 4) + 4 (lane / 32) + e % 4
+    const T *C = static_cast<const T *>(bias.ptr);
+    // (a bias per column is the same for every row: one load per column block instead of one per output)
+    const bool column_bias = C && bias.sm == 0;
+    float cb[NJ] = {};
+    if (column_bias) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t col = col0 + 32 * j + l32;
+            cb[j] = beta * up(C[ym * bias.sb + (col < n ? col : n - 1) * bias.sn]);
+        }
+    }
+    // with an even n (and Y on a 4-byte boundary) neighbouring lanes exchange two of their four rows, so that a lane
+    // stores two adjacent columns of two rows with 32-bit stores; otherwise element by element
+    const bool pairs = n % 2 == 0 && (reinterpret_cast<uintptr_t>(y) & 3u) == 0;
+    const bool odd = lane & 1;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int eg = 0; eg < 4; ++eg) {
+                const uint32_t row_eg = row0 + 32 * i + 8 * eg + 4 * kh;
+                const uint32_t col = col0 + 32 * j + l32;
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = alpha * acc[i][j][4 * eg + e];
+                    if (column_bias) v[e] += cb[j];
+                    else if (C && row_eg + e < m && col < n) v[e] += beta * up(C[ym * bias.sb + (row_eg + e) * bias.sm + col * bias.sn]);
+                }
+                if (pairs) {
+                    // even lanes keep rows 0 and 1, odd lanes rows 2 and 3 of the group of four
+                    const float give0 = odd ? v[0] : v[2], give1 = odd ? v[1] : v[3];
+                    const float got0 = __shfl_xor(give0, 1, kWave), got1 = __shfl_xor(give1, 1, kWave);
+                    const float lo0 = odd ? got0 : v[0], hi0 = odd ? v[2] : got0;
+                    const float lo1 = odd ? got1 : v[1], hi1 = odd ? v[3] : got1;
+                    const uint32_t row = row_eg + (odd ? 2 : 0), col_pair = col & ~1u;
+                    if (col_pair < n) {  // (n is even: both columns are in or out)
+                        const T p0[2] = {down<T>(lo0), down<T>(hi0)}, p1[2] = {down<T>(lo1), down<T>(hi1)};
+                        if (row < m) *reinterpret_cast<uint32_t *>(y + (ym * m + row) * n + col_pair) = __builtin_bit_cast(uint32_t, p0);
+                        if (row + 1 < m) *reinterpret_cast<uint32_t *>(y + (ym * m + row + 1) * n + col_pair) = __builtin_bit_cast(uint32_t, p1);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (row_eg + e < m && col < n) y[(ym * m + row_eg + e) * n + col] = down<T>(v[e]);
+                }
+            }
+}
 
 // TM: rows of a tile, 128 or 64 (a wavefront then has 32 rows of 64 columns: twice the workgroups for few tiles)
 template <class T, bool TRANS_B, bool B_VEC, int TM>  // B_VEC: rows of B as [k, n] start on 16-byte boundaries, n >= 8
@@ -631,55 +438,346 @@ __global__ __launch_bounds__(256, 2) void mm_tiles16(T *__restrict__ y, const T 
     }
     if (t < tiles) step(s0, s1, t);
     if (t + 1 < tiles) step(s1, s2, t + 1);
-    // accumulator: column lane % 32 of the block, register e holds row 8 (e / 4) + 4 (lane / 32) + e % 4
+    store_blocks<T, MI, 2>(acc, y, bias, ym, row0 + wm * (TM / 2), col0 + wn * 64, m, n, alpha, beta);
+}
+
+// A wave-uniform pointer, moved to scalar registers (so that what is added to it later is scalar arithmetic).
+__device__ __forceinline__ const uint8_t *uniform_pointer(const uint8_t *p) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits)));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32)));
+    return reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// ---------------------------------------------------------------- FP16 / BF16: middle-sized products
+//
+// 64 MI x 64 NJ outputs per workgroup of four wavefronts (32 MI x 32 NJ each, blocks of v_mfma_f32_32x32x16), k in tiles
+// of 64 copied straight into a ring of NS stages of LDS, up to NS - 1 tiles ahead of the one being multiplied.
+// A stage is a row of 8 KiB panels, 64 lines of 128 bytes each, A's MI panels first:
+//   A, and B as [n, k]: a line is a row of the tile (64 k); chunk c (16 bytes) of row r at position c ^ (r & 7) ^ ((r >> 3) & 1)
+//   B as [k, n]: a line is a k-row of 64 columns; chunk c of k-row r at position c ^ 4 ((r >> 1) & 1) ^ 2 ((r >> 3) & 1), read
+//   by ds_read_b64_tr_b16 (four k-rows of 16 columns per 16 lanes); both patterns meet every LDS bank once.
+// Tile t lives in stage t % NS.  Its fragments are read two k-steps (of four) ahead of their products, so that the last
+// of them are on their way in the second k-step; the barrier behind that k-step frees the stage for tile t + NS, whose copies
+// are dealt over the following four k-steps, and makes tile t + 1 visible.
+// Eight wavefronts (but for the smallest tile): two on a SIMD, so that the products of one fill the clocks in which the
+// other issues its copies (with four of twice the size 128 x 128 takes 44.5 us at [1000, 4096] x [4096, 4096]^T instead of
+// 40.8, 128 x 256 71 instead of 64 at 2048 rows).  k-tiles of 32 in twice the stages are slower (51 us: lines are fetched in
+// halves), a fifth stage changes nothing.  Bound by what the CUs together take from L2 and the memory-side cache: a
+// workgroup with the chip to itself needs 24 us for 128 x 128 x 4096, 256 of them 41 us (13 TB/s of operands; the products
+// alone would be 14 us).  FP16 / BF16, k = 4096, device time before (registers filled three tiles ahead for 128 x 128, two
+// LDS buffers for 256 x 256) and now: [1000, 4096] x [4096, 4096]^T 62 -> 41 us (825 TFLOP/s), 6144 columns 78 -> 53,
+// [2048, 4096] x [4096, 4096]^T 110 -> 64 us (1,070 TFLOP/s), 11008 columns 210 -> 169, 64 rows as [k, n] 47 -> 17 us.
+template <class T, bool TRANS_B, int WM, int WN, int MI, int NJ, int NS>
+struct Ring {
+    static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, WAVES = WM * WN, LINE = 128, STAGE = (TM + TN) * LINE, LDS = NS * STAGE;
+    static constexpr int COPIES_A = TM * LINE / 1024 / WAVES, COPIES_B = TN * LINE / 1024 / WAVES, COPIES = COPIES_A + COPIES_B;  // of a wavefront and tile
+};
+
+template <class T, bool TRANS_B, int WM, int WN, int MI, int NJ, int NS>
+__device__ __forceinline__ void ring_loop(f16v (&acc)[MI][NJ], uint8_t *lds, const uint8_t *A, const uint8_t *B, uint32_t row0,
+                                          uint32_t col0, uint32_t m, uint32_t k, uint32_t n) {
+    typedef Ring<T, TRANS_B, WM, WN, MI, NJ, NS> R;
+    constexpr int LINE = R::LINE, KS = 4, D = 2;  // k-steps of a tile, k-steps from a fragment's read to its product
+    constexpr int C = R::COPIES, CA = R::COPIES_A, CB = R::COPIES_B;
+    constexpr int HALF = NS == 2 ? C : (C + 1) / 2;  // copies of a tile that are issued in the second half of a step, right behind the barrier
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave / WN, wn = wave % WN, h = lane >> 5;
+    // copy q < CA of this wavefront: rows 8 (CA wave + q) .. + 7 of A's tile, this lane row + lane / 8, position lane % 8;
+    // copy CA + q: lines 8 (CB wave + q) .. + 7 of B's panels.  Rows and columns beyond the matrix are copied from
+    // inside it (not stored).
+    auto swizzle = [](uint32_t r) -> uint32_t { return (r & 7) ^ ((r >> 3) & 1); };
+    uint32_t voff[C];
+#pragma unroll
+    for (int q = 0; q < CA; ++q) {
+        const uint32_t r = 8 * (CA * wave + q) + (lane >> 3), row = row0 + r < m ? row0 + r : m - 1;
+        voff[q] = (row - row0) * (2 * k) + 16 * ((lane & 7) ^ swizzle(r));
+    }
+#pragma unroll
+    for (int q = 0; q < CB; ++q) {
+        if constexpr (TRANS_B) {
+            const uint32_t r = 8 * (CB * wave + q) + (lane >> 3);
+            const uint32_t col = col0 + r < n ? col0 + r : n - 1;
+            voff[CA + q] = (col - col0) * (2 * k) + 16 * ((lane & 7) ^ swizzle(r));
+        } else {
+            const uint32_t r = 8 * (CB * wave + q) + (lane >> 3), kr = r & 63, chunk = (lane & 7) ^ (4 * ((kr >> 1) & 1)) ^ (2 * ((kr >> 3) & 1));
+            const uint32_t col = col0 + 64 * (r >> 6) + 8 * chunk;
+            voff[CA + q] = 2 * (kr * n + (col + 8 <= n ? col : n - 8));
+        }
+    }
+    const uint8_t *a_base = uniform_pointer(A + static_cast<uint64_t>(row0) * (2 * k));
+    const uint8_t *b_base = uniform_pointer(TRANS_B ? B + static_cast<uint64_t>(col0) * (2 * k) : B);
+    const uint64_t b_step = TRANS_B ? LINE : static_cast<uint64_t>(LINE) * n;  // bytes from one tile of B to the next
+    const uint32_t lds0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds))));
+    // The copies are assembly (a scalar base plus a 32-bit lane offset), so that the compiler adds no waits for them:
+    // the waits are the explicit ones in front of the barriers.
+    auto copy = [&]<int Q>(const uint8_t *a_from, const uint8_t *b_from, uint32_t stage) __attribute__((always_inline)) {
+        const uint32_t to = lds0 + stage + 1024 * (Q < CA ? CA * wave + Q : R::TM * LINE / 1024 + CB * wave + (Q - CA));
+        const uint8_t *from = Q < CA ? a_from : b_from;
+        const uint32_t lane_off = voff[Q];
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(lane_off), "s"(from), "s"(to)
+                     : "memory", "m0");
+    };
+    const uint32_t a_off = (wm * 32 * MI + (lane & 31)) * LINE + 16 * (h ^ swizzle(lane & 31));
+    auto read_a = [&](uint32_t stage, int ks, int i) -> u32x4 {
+        return *reinterpret_cast<const u32x4 *>(lds + stage + (a_off ^ (32 * ks)) + i * 32 * LINE);
+    };
+    uint32_t b_off[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        if constexpr (TRANS_B) {
+            b_off[j] = R::TM * LINE + (wn * 32 * NJ + 32 * j + (lane & 31)) * LINE + 16 * (h ^ swizzle(lane & 31));
+        } else {
+            const uint32_t a16 = lane & 15, r = a16 >> 2, block = wn * NJ + j;
+            const uint32_t chunk = 4 * (block & 1) + 2 * ((lane >> 4) & 1) + ((a16 & 3) >> 1);
+            b_off[j] = R::TM * LINE + 64 * LINE * (block >> 1) + (8 * h + r) * 128 + 16 * (chunk ^ (4 * ((r >> 1) & 1)) ^ (2 * h)) + 8 * (a16 & 1);
+        }
+    }
+    auto read_b = [&](uint32_t stage, int ks, int j, u32x4 &f) {
+        if constexpr (TRANS_B) {
+            f = *reinterpret_cast<const u32x4 *>(lds + stage + (b_off[j] ^ (32 * ks)));
+        } else {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const s4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (s4 __attribute__((address_space(3))) *)(lds + stage + b_off[j] + (16 * ks + 4 * half) * 128));
+                const u32x2 w = __builtin_bit_cast(u32x2, v);
+                f[2 * half] = w[0];
+                f[2 * half + 1] = w[1];
+            }
+        }
+    };
+
+    const uint32_t k_tiles = k / 64;
+    auto a_tile = [&](uint32_t t) { return uniform_pointer(a_base + (t < k_tiles ? t : 0) * static_cast<uint64_t>(LINE)); };
+    auto b_tile = [&](uint32_t t) { return uniform_pointer(b_base + (t < k_tiles ? t : 0) * b_step); };
+    // tiles 0 .. NS - 2 and the first half of tile NS - 1's copies (behind the end: tile 0 again, never multiplied)
+    auto fill = [&]<int COUNT>(uint32_t tile, uint32_t stage) __attribute__((always_inline)) {
+        const uint8_t *a_from = a_tile(tile), *b_from = b_tile(tile);
+        [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
+            (copy.template operator()<Q>(a_from, b_from, stage), ...);
+        }(std::make_integer_sequence<int, COUNT>{});
+    };
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s) fill.template operator()<C>(s, s * R::STAGE);
+    fill.template operator()<HALF>(NS - 1, (NS - 1) * R::STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * C + HALF) : "memory");  // tile 0
+    __syncthreads();
+    u32x4 fa[KS][MI], fb[KS][NJ];
+#pragma unroll
+    for (int ks = 0; ks < D; ++ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[ks][i] = read_a(0, ks, i);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) read_b(0, ks, j, fb[ks][j]);
+    }
+    // MODE 0: tile t + NS exists; 1: tile t + NS - 1 is the last one; 2: nothing is left to copy
+    auto step = [&]<int MODE>(uint32_t t, uint32_t stage, uint32_t next, uint32_t prev) __attribute__((always_inline)) {
+        constexpr int P = MI * NJ, SLOTS = KS * P;
+        const uint8_t *a_old = a_tile(t + NS - 1), *b_old = b_tile(t + NS - 1), *a_new = a_tile(t + NS), *b_new = b_tile(t + NS);
+        auto slot = [&]<int s>() __attribute__((always_inline)) {
+            // rows walk the columns back and forth, so that only one operand changes between products
+            constexpr int ks = s / P, o = s % P, row = o / NJ, col = (row & 1) ? NJ - 1 - o % NJ : o % NJ;
+            if constexpr (s == D * P) {
+                // tile t + 1 has landed and this wavefront's reads of tile t are done
+                if constexpr (MODE == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * C) : "memory");
+                __syncthreads();
+            }
+            acc[row][col] = Mfma<T>::run(fa[ks][row], fb[ks][col], acc[row][col]);
+            constexpr int nks = (ks + D) % KS;
+            const uint32_t src = ks < D ? stage : next;
+            // MI + NJ fragments in the first slots of the k-step, two a slot
+            [&]<int... F>(std::integer_sequence<int, F...>) __attribute__((always_inline)) {
+                ([&] {
+                    if constexpr (F / 2 == o || (o == P - 1 && F / 2 >= P)) {
+                        if constexpr (F < NJ) read_b(src, nks, F, fb[nks][F]);
+                        else fa[nks][F - NJ] = read_a(src, nks, F - NJ);
+                    }
+                }(), ...);
+            }(std::make_integer_sequence<int, MI + NJ>{});
+            [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
+                ([&] {
+                    if constexpr (MODE < 2 && s < D * P && Q < C - HALF && Q * D * P / HALF == s) copy.template operator()<HALF + Q>(a_old, b_old, prev);
+                    if constexpr (MODE < 1 && s >= D * P && Q * D * P / HALF == s - D * P) copy.template operator()<Q>(a_new, b_new, stage);
+                }(), ...);
+            }(std::make_integer_sequence<int, HALF>{});
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+            (slot.template operator()<I>(), ...);
+        }(std::make_integer_sequence<int, SLOTS>{});
+    };
+    uint32_t t = 0, stage = 0, prev = (NS - 1) * R::STAGE;
+    auto advance = [&] {
+        ++t;
+        prev = stage;
+        stage = stage + R::STAGE == static_cast<uint32_t>(R::LDS) ? 0 : stage + R::STAGE;
+    };
+    auto next = [&] { return stage + R::STAGE == static_cast<uint32_t>(R::LDS) ? 0u : stage + R::STAGE; };
+    for (; t + NS < k_tiles; advance()) step.template operator()<0>(t, stage, next(), prev);
+    if (t + NS == k_tiles) {
+        step.template operator()<1>(t, stage, next(), prev);
+        advance();
+    }
+    for (; t < k_tiles; advance()) step.template operator()<2>(t, stage, next(), prev);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land after the workgroup's LDS is released
+}
+
+// The same outputs in 128-bit stores (n a multiple of 8, Y on a 16-byte boundary): a wavefront's blocks pass through
+// 2 KiB MI NJ of LDS of its own, a row of them in 64 NJ bytes.
+template <class T, int MI, int NJ>
+__device__ __forceinline__ void store_rows(const f16v (&acc)[MI][NJ], uint8_t *stage, T *__restrict__ y, const Bias &bias, uint64_t ym,
+                                           uint32_t row0, uint32_t col0, uint32_t m, uint32_t n, float alpha, float beta) {
+    const uint32_t lane = threadIdx.x & 63, l32 = lane & 31, kh = lane >> 5;
     const T *C = static_cast<const T *>(bias.ptr);
-    // (a bias per column is the same for every row: one load per column block instead of one per output)
+    // a bias per column (the usual one of a linear layer) is the same for every row: one load per column block
     const bool column_bias = C && bias.sm == 0;
-    float cb[2] = {0.f, 0.f};
+    float cb[NJ] = {};
     if (column_bias) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t col = col0 + wn * 64 + 32 * j + l32;
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t col = col0 + 32 * j + l32;
             cb[j] = beta * up(C[ym * bias.sb + (col < n ? col : n - 1) * bias.sn]);
         }
     }
-    // with an even n (and Y on a 4-byte boundary) neighbouring lanes exchange two of their four rows, so that a lane
-    // stores two adjacent columns of two rows with 32-bit stores; otherwise element by element
-    const bool pairs = n % 2 == 0 && (reinterpret_cast<uintptr_t>(y) & 3u) == 0;
+    auto at = [](uint32_t row, uint32_t byte) -> uint32_t {  // NJ = 2: rows 2 apart go to different halves of a line
+        return row * 64 * NJ + (NJ == 2 ? byte ^ (64 * ((row >> 1) & 1)) : byte);
+    };
     const bool odd = lane & 1;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j) {
+            // any other bias: the sixteen values of a block are requested together, ahead of their use
+            T bv[16];
+            const bool other_bias = C && !column_bias;
+            if (other_bias) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const uint32_t row = row0 + 32 * i + 8 * (e / 4) + 4 * kh + e % 4, col = col0 + 32 * j + l32;
+                    bv[e] = C[ym * bias.sb + (row < m ? row : m - 1) * bias.sm + (col < n ? col : n - 1) * bias.sn];
+                }
+            }
 #pragma unroll
             for (int eg = 0; eg < 4; ++eg) {
-                const uint32_t row_eg = row0 + wm * (TM / 2) + 32 * i + 8 * eg + 4 * kh;
-                const uint32_t col = col0 + wn * 64 + 32 * j + l32;
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     v[e] = alpha * acc[i][j][4 * eg + e];
                     if (column_bias) v[e] += cb[j];
-                    else if (C && row_eg + e < m && col < n) v[e] += beta * up(C[ym * bias.sb + (row_eg + e) * bias.sm + col * bias.sn]);
+                    else if (other_bias) v[e] += beta * up(bv[4 * eg + e]);
                 }
-                if (pairs) {
-                    // even lanes keep rows 0 and 1, odd lanes rows 2 and 3 of the group of four
-                    const float give0 = odd ? v[0] : v[2], give1 = odd ? v[1] : v[3];
-                    const float got0 = __shfl_xor(give0, 1, kWave), got1 = __shfl_xor(give1, 1, kWave);
-                    const float lo0 = odd ? got0 : v[0], hi0 = odd ? v[2] : got0;
-                    const float lo1 = odd ? got1 : v[1], hi1 = odd ? v[3] : got1;
-                    const uint32_t row = row_eg + (odd ? 2 : 0), col_pair = col & ~1u;
-                    if (col_pair < n) {  // (n is even: both columns are in or out)
-                        const T p0[2] = {down<T>(lo0), down<T>(hi0)}, p1[2] = {down<T>(lo1), down<T>(hi1)};
-                        if (row < m) *reinterpret_cast<uint32_t *>(y + (ym * m + row) * n + col_pair) = __builtin_bit_cast(uint32_t, p0);
-                        if (row + 1 < m) *reinterpret_cast<uint32_t *>(y + (ym * m + row + 1) * n + col_pair) = __builtin_bit_cast(uint32_t, p1);
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (row_eg + e < m && col < n) y[(ym * m + row_eg + e) * n + col] = down<T>(v[e]);
-                }
+                // even lanes keep rows 0 and 1, odd lanes rows 2 and 3 of the group of four
+                const float give0 = odd ? v[0] : v[2], give1 = odd ? v[1] : v[3];
+                const float got0 = __shfl_xor(give0, 1, kWave), got1 = __shfl_xor(give1, 1, kWave);
+                const T p0[2] = {down<T>(odd ? got0 : v[0]), down<T>(odd ? v[2] : got0)};
+                const T p1[2] = {down<T>(odd ? got1 : v[1]), down<T>(odd ? v[3] : got1)};
+                const uint32_t row = 32 * i + 8 * eg + 4 * kh + (odd ? 2 : 0), byte = 2 * (32 * j + (l32 & ~1u));
+                *reinterpret_cast<uint32_t *>(stage + at(row, byte)) = __builtin_bit_cast(uint32_t, p0);
+                *reinterpret_cast<uint32_t *>(stage + at(row + 1, byte)) = __builtin_bit_cast(uint32_t, p1);
             }
+        }
+    // (each wavefront reads back only what it wrote itself: no barrier)
+#pragma unroll
+    for (int it = 0; it < 2 * MI * NJ; ++it) {
+        const uint32_t idx = lane + 64 * it, row = idx / (4 * NJ), chunk = idx % (4 * NJ);
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + at(row, 16 * chunk));
+        if (row0 + row < m && col0 + 8 * chunk < n)
+            *reinterpret_cast<u32x4 *>(y + (ym * m + row0 + row) * n + col0 + 8 * chunk) = v;
+    }
+}
+
+template <class T, bool TRANS_B, int WM, int WN, int MI, int NJ, int NS>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void mm_ring(T *__restrict__ y, const T *__restrict__ a, const T *__restrict__ b, Bias bias,
+                                                  uint32_t m, uint32_t k, uint32_t n, uint32_t col_first, uint32_t columns,
+                                                  float alpha, float beta, uint32_t a_matrix0, uint32_t b_matrix0, uint32_t y_matrix0) {
+    typedef Ring<T, TRANS_B, WM, WN, MI, NJ, NS> R;
+    __shared__ __align__(1024) uint8_t lds[R::LDS];
+    const uint32_t bz = blockIdx.z;
+    const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
+    // consecutive workgroup ids go round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, walked down the
+    // rows of one column panel after the other
+    const uint32_t row_tiles = (m + R::TM - 1) / R::TM, n_tiles = row_tiles * ((columns + R::TN - 1) / R::TN);
+    const uint32_t xcd = blockIdx.x % 8, share = n_tiles / 8, more = n_tiles % 8;
+    const uint32_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / 8;
+    const uint32_t row0 = (tile % row_tiles) * R::TM, col0 = col_first + (tile / row_tiles) * R::TN;
+    f16v acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    ring_loop<T, TRANS_B, WM, WN, MI, NJ, NS>(acc, lds, reinterpret_cast<const uint8_t *>(a + am * m * static_cast<uint64_t>(k)),
+                                      reinterpret_cast<const uint8_t *>(b + bm * static_cast<uint64_t>(k) * n), row0, col0, m, k, n);
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t wave_row = row0 + (wave / WN) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
+    if (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0) {
+        __syncthreads();  // every wavefront has read its last fragments
+        store_rows<T, MI, NJ>(acc, lds + wave * (32 * MI * 64 * NJ), y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
+    } else {
+        store_blocks<T, MI, NJ>(acc, y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
+    }
+}
+
+// The tile shapes and what a launch of them takes: `fixed` us a round of 256 workgroups (a CU holds one), and per 64 of
+// k `alone` ns while few CUs have a tile, `full` ns while all have one (they then share what L2 and the memory-side cache
+// deliver, 30 to 40 % of the time of every shape).  Measured at k = 512 to 4096, FP16 and BF16, both layouts of B.
+struct RingShape {
+    uint32_t rows, cols;
+    double fixed, alone, full;
+};
+constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 180, 260},  {64, 128, 3, 235, 405},  {128, 128, 4.5, 300, 560},
+                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 11, 1000, 1660}};
+constexpr int kRingShapeCount = 6;
+constexpr uint32_t kCus = 256;
+
+struct RingPlan {
+    int first, rest;   // shape of the first `columns` columns and of those behind them
+    uint32_t columns;  // 0: all on `rest`
+    double us;
+};
+
+inline double ring_us(const RingShape &t, double tiles, double steps) {
+    const double rounds = static_cast<double>(static_cast<uint64_t>(tiles / kCus)), left = tiles / kCus - rounds;
+    return rounds * (t.fixed + 1e-3 * steps * t.full) + (left > 0 ? t.fixed + 1e-3 * steps * (t.alone + (t.full - t.alone) * left) : 0);
+}
+
+// One shape for the whole product, or whole rounds of one shape and another one for the columns that are left: 344 tiles of
+// 256 x 256 ([2048, 4096] x [4096, 11008]) would be a full round and one with two thirds of the CUs idle (208 us); a full
+// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.
+inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t batch) {
+    RingPlan best{0, 0, 0, 1e30};
+    const double steps = static_cast<double>(k / 64);
+    auto single = [&](size_t columns) {
+        std::pair<int, double> one{0, 1e30};
+        for (int i = 0; i < kRingShapeCount; ++i) {
+            const RingShape &t = kRingShapes[i];
+            const double us = ring_us(t, static_cast<double>((m + t.rows - 1) / t.rows) * static_cast<double>((columns + t.cols - 1) / t.cols) *
+                                             static_cast<double>(batch), steps);
+            if (us < one.second) one = {i, us};
+        }
+        return one;
+    };
+    const auto whole = single(n);
+    best.rest = whole.first;
+    best.us = whole.second;
+    if (batch != 1) return best;
+    for (int i = 0; i < kRingShapeCount; ++i) {
+        const RingShape &t = kRingShapes[i];
+        const size_t row_tiles = (m + t.rows - 1) / t.rows, tiles = row_tiles * (n / t.cols);
+        const size_t wide = tiles / kCus * kCus / row_tiles;  // columns of tiles in whole rounds
+        if (wide == 0 || wide * t.cols >= n) continue;
+        const auto rest = single(n - wide * t.cols);
+        const double us = ring_us(t, static_cast<double>(row_tiles * wide), steps) + rest.second;
+        if (us < 0.97 * best.us) best = {i, rest.first, static_cast<uint32_t>(wide * t.cols), us};
+    }
+    return best;
 }
 
 // ---------------------------------------------------------------- few rows of A (decode): weight streaming
@@ -1941,14 +2039,8 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     typedef typename Acc<T>::type A_t;
     const A_t al = through<T>(alpha), be = bias.ptr ? through<T>(beta) : A_t(0);
     constexpr bool narrow = sizeof(T) == 2;
-    // rows of B as [k, n] and of Y start on 16-byte boundaries when n is a multiple of 8; tiles that are moved
-    // back overlap their neighbours, which a bias that is the output itself does not allow
-    const bool ragged = m % BM != 0 || n % BN != 0;
-    const bool fast = narrow && !trans_a && m >= BM && n >= BN && n % 8 == 0 && k % BK == 0 && k > 0 && aligned16(a) &&
-                      aligned16(b) && aligned16(y_) && !(ragged && bias.ptr == y_);
-
-    // fewer rows than a tile, weights as [n, k]: stream W once per slab of 32 rows of A
-    const bool skinny = narrow && !fast && !trans_a && trans_b && m < BM && n % 32 == 0 && k % SK_TK == 0 &&
+    // fewer than 256 rows, weights as [n, k]: stream W once per slab of 32 rows of A
+    const bool skinny = narrow && !trans_a && trans_b && m < kFewRows && n % 32 == 0 && k % SK_TK == 0 &&
                         aligned16(a) && aligned16(b);
 
     // one row (and up to four where the block-product kernel below does not apply): matrix-vector products on the
@@ -1972,46 +2064,39 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
 
     // fewer than 256 rows, weights as [k, n]: the same block products behind a transposition in registers, 32 rows a
     // pass (one to four rows against a wide B stay with the matrix-vector kernel, which is a little faster there)
-    const bool rows_kn = narrow && !trans_a && !trans_b && m < BM && !(m <= 4 && n >= 8192) && n % 16 == 0 && k % 128 == 0 &&
+    const bool rows_kn = narrow && !trans_a && !trans_b && m < kFewRows && !(m <= 4 && n >= 8192) && n % 16 == 0 && k % 128 == 0 &&
                          k > 0 && static_cast<uint64_t>(k) * n < (1ull << 31) && k < (1u << 26) && aligned16(a) && aligned16(b);
 
-    // fewer than 256 rows on the 256 x 256 tiles (one row of tiles, A's missing rows repeated, their results not
-    // stored): a launch costs what a full tile costs, about 93 us at k = 4096, whatever m is, so it is taken where
-    // the passes of the few-rows kernels would take longer (measured per pass at k = 4096: 5.5 ns per column for 32
-    // rows with B as [k, n], 3.4 to 4.7 ns for 64 rows with B as [n, k]) and where the plain kernel is the alternative
-    const bool short_ok = narrow && !trans_a && m < BM && n >= BN && n % 8 == 0 && k % BK == 0 && k > 0 && aligned16(a) &&
-                          aligned16(b) && aligned16(y_) && !(n % BN != 0 && bias.ptr == y_) &&
-                          k < (1u << 22);  // a lane's offset into A (up to 255 rows) stays below 2^31
-    // FP16 / BF16 shapes that none of the kernels above takes, more than 8 rows: 128 x 128 tiles, any m and n.
-    // They also take the shapes of the 256 x 256 tiles when those are few: a workgroup's walk through k is a chain
-    // of dependent steps (1.33 us per 64 of k on the large tile, 0.83 us on the small one), so while the small tiles
-    // find a CU each, or nearly, the launch ends earlier (k = 4096: 85 -> 53 us up to 64 large tiles, 85 -> 78 at 86,
-    // level at 128)
+    // FP16 / BF16 on the tiles, any m: the ring kernel where k is in whole tiles and rows of B as [k, n] start on 16-byte
+    // boundaries (its lane offsets, up to 256 rows of A or B or 64 k-rows of B, stay below 2^32), mm_tiles16 for the rest.
     // Up to 8 rows only where the plain kernel is expected to take longer (it needs 2.9 ns per thousand elements of B,
     // 596 us for [8, 4096] x [4096, 50257]; a tile launch about 4 us and 0.83 us per 64 of k).
+    const size_t side_by_side = a_index || b_index ? 1 : batch;  // matrices that are tiles of one launch
     const bool tiles16_rows = m > 8 || static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k);
     const bool tiles16 = narrow && !trans_a && k % 8 == 0 && k > 0 && tiles16_rows && aligned16(a) && (!trans_b || aligned16(b));
-    const bool small_grid = tiles16 && ((m + HT - 1) / HT) * ((n + HT - 1) / HT) * (a_index || b_index ? 1 : batch) <= kSmallGrid;
-    bool short_tile = false;
-    if (short_ok || small_grid) {
-        // (the tile launch that the passes of the few-rows kernels are weighed against is cheaper on the small tiles;
-        // there the matrices of a batch count too, all of them being tiles of one launch that find a CU each)
-        // (one to four rows against W as [n, k] read W once at the speed of the memory whatever n is: never a tile)
-        const uint64_t columns = small_grid ? n * (a_index || b_index ? 1 : batch) : n;
-        // passes of four rows over B as [k, n] against one launch of small tiles (a pass: 4.3 us or B at 5 TB/s)
-        const double b_us = 2.0 * static_cast<double>(k) * static_cast<double>(columns) / 5.0e6;
-        const double gemv_kn_us = static_cast<double>((m + 3) / 4) * (b_us > 4.3 ? b_us : 4.3);
-        const bool gemv_kn_slow = small_grid && m > 4 && 4.0 + 0.83 * static_cast<double>((k + HK - 1) / HK) < gemv_kn_us;
-        if (trans_b) short_tile = rows || gemv ? false : skinny ? ((m + 63) / 64) * columns > (small_grid ? kSkinnyPassesSmall : 23000u) : true;
-        else short_tile = rows_kn ? ((m + 31) / 32) * columns > (small_grid ? kRowsKnPassesSmall : 17000u)
-                                  : gemv_kn ? (short_ok && m > 16) || gemv_kn_slow : true;
-    }
+    const size_t tiles128 = ((m + HT - 1) / HT) * ((n + HT - 1) / HT) * side_by_side;
+    const bool ring = tiles16 && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
+    const RingPlan plan = ring ? ring_plan(m, k, n, side_by_side) : RingPlan{0, 0, 0, 0};
     // A short k leaves a tile little to do between fetching its operands and storing its results, and two small tiles
-    // per CU overlap the one's stores with the other's loads: with k <= 128 the small tiles take a full grid too
-    // ([4096, 128] x [128, 4096] 24.7 -> 22.9 us, [8192, 128] x [128, 8192] 93 -> 76 us, 32 products of
-    // [512, 128] x [512, 128]^T 21 -> 13.5 us; at k = 256 they lose, 28 -> 31 us), and with k <= 512 every short tile
-    // is a small one and taken before the few-rows kernels (32 products [128, 128] x [4096, 128]^T 110 -> 25 us)
-    const bool short_k = tiles16 && m > 16 && ((fast && k <= 128) || (short_ok && k <= 512));
+    // per CU overlap the one's stores with the other's loads: with k <= 128 (k <= 512 below 256 rows) more tiles than CUs
+    // are mm_tiles16's ([8192, 128] x [128, 8192] 76 us, 32 products [128, 128] x [4096, 128]^T 25 us).
+    const bool short_k = tiles16 && m > 16 && n >= 256 && n % 8 == 0 && k % 64 == 0 && aligned16(b) && aligned16(y_) &&
+                         k <= (m < kFewRows ? 512u : 128u) && tiles128 > kCus;
+    // Fewer than 256 rows: the tiles, or the passes of the few-rows kernels where those end earlier (us, from
+    // measurements at k = 4096: mm_skinny 13.5 for 32 and 19 for 64 rows of 4096 columns, 38 for 11008 columns;
+    // mm_rows_kn 22 for 32 rows of 4096 columns; a pass of four rows of mm_gemv_kn 4.3, or B at 5 TB/s).  One to 16 rows
+    // that mm_gemv and mm_rows take read W as [n, k] once at the speed of the memory whatever n is: never a tile.
+    bool tiles_first = tiles16 && m >= kFewRows;
+    if (tiles16 && !tiles_first && (ring || tiles128 <= kSmallGrid)) {
+        const double tile_us = ring ? plan.us : 4.0 + 0.83 * static_cast<double>((k + HK - 1) / HK);
+        const double columns = static_cast<double>(n * side_by_side), k4096 = static_cast<double>(k) / 4096;
+        const double skinny_us = static_cast<double>((m + 63) / 64) * (3.0 + columns * (m <= 32 ? 2.6e-3 : 3.4e-3) * k4096);
+        const double rows_kn_us = static_cast<double>((m + 31) / 32) * (2.0 + columns * (m <= 16 ? 3.5e-3 : 5.0e-3) * k4096);
+        const double b_us = 2.0 * static_cast<double>(k) * columns / 5.0e6;
+        const double gemv_kn_us = static_cast<double>((m + 3) / 4) * (b_us > 4.3 ? b_us : 4.3);
+        if (trans_b) tiles_first = rows || gemv ? false : !skinny || tile_us < skinny_us;
+        else tiles_first = rows_kn ? tile_us < rows_kn_us : !gemv_kn || (m > 4 && tile_us < gemv_kn_us);
+    }
 
     // F32 on the matrix cores.  A launch of the 128 x 128 tiles walks all of k in every workgroup and takes about
     // 300 us at k = 4096 however few tiles there are; up to that cost few rows go through the block products of
@@ -2056,6 +2141,41 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
         }
     };
 
+    auto launch_ring = [&](uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
+        if constexpr (narrow) {
+            const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
+            auto part = [&](int shape, uint32_t first, uint32_t columns) -> int {
+                const RingShape &t = kRingShapes[shape];
+                const uint64_t tiles = ((m + t.rows - 1) / t.rows) * static_cast<uint64_t>((columns + t.cols - 1) / t.cols);
+                if (tiles > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
+                const dim3 grid(static_cast<unsigned>(tiles), 1, count);
+#define RG_RING(WM, WN, MI, NJ, NS)                                                                                          \
+    do {                                                                                                                     \
+        static_assert(Ring<T, true, WM, WN, MI, NJ, NS>::LDS <= 163840);                                                     \
+        if (trans_b) mm_ring<T, true, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a, b, bias, m32, k32, n32, first, columns, al, be, am0, bm0, ym0); \
+        else mm_ring<T, false, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a, b, bias, m32, k32, n32, first, columns, al, be, am0, bm0, ym0);        \
+    } while (0)
+                switch (shape) {
+                    case 0: RG_RING(2, 2, 1, 1, 8); break;
+                    case 1: RG_RING(2, 4, 1, 1, 6); break;
+                    case 2: RG_RING(2, 4, 2, 1, 4); break;
+                    case 3: RG_RING(4, 2, 1, 3, 4); break;
+                    case 4: RG_RING(2, 4, 2, 2, 3); break;
+                    default: RG_RING(2, 4, 4, 2, 2);
+                }
+#undef RG_RING
+                return launch_status();
+            };
+            if (plan.columns) {
+                const int rc = part(plan.first, 0, plan.columns);
+                if (rc) return rc;
+            }
+            return part(plan.rest, plan.columns, n32 - plan.columns);
+        } else {
+            return RG_HIP_E_UNSUPPORTED;
+        }
+    };
+
     auto launch = [&](uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
         if constexpr (narrow) {
             // five to 32 rows against weights as [k, n] with a workspace at hand: the same sharing on the matrix cores
@@ -2079,17 +2199,8 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                                               b + static_cast<uint64_t>(bm0) * k * n, bias, static_cast<uint32_t>(m),
                                               static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, workspace, plan, s);
             }
-            if ((small_grid && (short_tile || fast)) || short_k) return launch_tiles16(am0, bm0, ym0, count);
-            if (short_tile) {
-                const dim3 grid(static_cast<unsigned>((n + BN - 1) / BN), 1, count);
-                if (trans_b)
-                    mm_mfma_256x256<T, true, true><<<grid, 256, 0, s>>>(y, a, b, bias, static_cast<uint32_t>(m), static_cast<uint32_t>(k),
-                                                                        static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                else
-                    mm_mfma_256x256<T, false, true><<<grid, 256, 0, s>>>(y, a, b, bias, static_cast<uint32_t>(m), static_cast<uint32_t>(k),
-                                                                         static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                return launch_status();
-            }
+            if (short_k) return launch_tiles16(am0, bm0, ym0, count);
+            if (tiles_first) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
             if (rows_kn) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 const bool wide = n % 32 == 0 && n >= 8192;
@@ -2153,19 +2264,9 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                 }
                 return 0;
             }
-            if (fast) {
-                const dim3 grid(static_cast<unsigned>(((m + BM - 1) / BM) * ((n + BN - 1) / BN)), 1, count);
-                if (trans_b)
-                    mm_mfma_256x256<T, true><<<grid, 256, 0, s>>>(y, a, b, bias, static_cast<uint32_t>(m), static_cast<uint32_t>(k),
-                                                                  static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                else
-                    mm_mfma_256x256<T, false><<<grid, 256, 0, s>>>(y, a, b, bias, static_cast<uint32_t>(m), static_cast<uint32_t>(k),
-                                                                   static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                return launch_status();
-            }
         }
         if constexpr (narrow) {
-            if (tiles16) return launch_tiles16(am0, bm0, ym0, count);
+            if (tiles16) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
         }
         if constexpr (std::is_same<T, float>::value) {
             if (rows_f32) {

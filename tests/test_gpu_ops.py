@@ -1546,6 +1546,37 @@ def test_matmul_groups_of_matrices_that_share_one_b(S, T, D):
     assert np.array_equal(got, want_s)
 
 
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("m,k,n", [
+    (9, 64, 4096), (17, 128, 264), (64, 192, 520), (65, 320, 1000), (130, 448, 2056), (255, 512, 1032),   # 64-row tiles
+    (300, 576, 4000), (513, 640, 4104), (1025, 256, 6152), (1000, 320, 6144),                             # wider ones
+    (2048, 1024, 4096), (4000, 512, 4104), (2049, 1024, 11016), (256, 64, 256)])                          # 256 rows, two shapes
+def test_matmul_ring_tiles_exact_on_small_integers(m, k, n, tb):
+    """Edges of the tiles and fewer k-tiles than the ring has stages: sums of small integers are exact in float, so the
+    result is the exact product rounded once, whatever the order of the sum."""
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + k * 3 + n)
+    rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda")
+    for n_, dt in ((n, torch.float16), (n + 1 if tb else n, torch.bfloat16)):
+        a, b = rand(m, k), rand(n_, k) if tb else rand(k, n_)
+        exact = a.double() @ (b.double().t().contiguous() if tb else b.double())
+        for c in (None, rand(n_), rand(m, 1), rand(m, n_)):
+            y = ops.matmul(a.to(dt), b.to(dt), None if c is None else c.to(dt), trans_b=tb)
+            ref = exact if c is None else exact + c.double()
+            assert torch.equal(y, ref.to(dt)), (n_, dt, None if c is None else tuple(c.shape))
+
+
+def test_matmul_ring_tiles_bias_in_place_and_batch():
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda")
+    a, b, y = rand(700, 320), rand(1032, 320), rand(700, 1032).half()
+    ref = (a.double() @ b.double().t().contiguous() + y.double()).half()
+    ops.matmul(a.half(), b.half(), y, trans_b=True, out=y)  # the bias is the output itself
+    assert torch.equal(y, ref)
+    a, b = rand(5, 130, 192), rand(5, 192, 264)
+    ref = torch.stack([a[i].double() @ b[i].double() for i in range(5)]).half()
+    assert torch.equal(ops.matmul(a.half(), b.half()), ref)
+
+
 def test_matmul_fp16_exact_on_small_integers_full_tile_grid():
     # integer-valued operands with |sum| < 2048: every fp16 result is exact, so the MFMA path must
     # reproduce numpy's integer product bit for bit over a 3 x 2 grid of tiles and 5 k-tiles
