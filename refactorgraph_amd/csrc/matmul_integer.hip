@@ -570,6 +570,228 @@ __global__ __launch_bounds__(256, 1) void mmi_mfma_256x256(int32_t *__restrict__
             }
 }
 
+// ---------------------------------------------------------------- middle-sized products: a ring of LDS stages
+//
+// 32 MI WM x 32 NJ WN outputs per workgroup of WM WN wavefronts, k in tiles of 128 copied straight into a ring of NS
+// stages, up to NS - 1 tiles ahead of the one being multiplied.  A stage holds A's rows (lines of 128 bytes, chunk c of row r
+// at position c ^ (r & 7) ^ ((r >> 3) & 1)), then panels of PW columns of B: 128 k-rows of PW bytes as in memory, turned by
+// ds_read_b64_tr_b8 (eight k-rows of 32 columns per 32 lanes: chunk c of k-row r at position c ^ 2 (r / (256 / PW) % 4, or % 2
+// for PW = 64) ^ ((r >> 4) & 1), every LDS bank once).  Fragments are read two k-steps (of four) ahead of their products and
+// have their zero point subtracted one k-step ahead; the barrier behind the second k-step frees the stage of tile t for
+// tile t + NS and makes tile t + 1 visible.  Where k ends with half a tile, the last tile starts 64 earlier and its first
+// two k-steps are not multiplied.
+// Eight wavefronts for the larger tiles: two on a SIMD, one of which issues products while the other issues its copies or
+// subtracts zero points (four vector instructions per word of A: with 1 x 2 blocks per wavefront they fit behind the products,
+// with 2 x 1 blocks a launch takes 8 % longer).  Bound by what the CUs together take from L2 and the memory-side cache.
+// uint8 activations with an arbitrary zero point, k = 4096, before (mmi_tiles, 256 x 256 tiles with k shared) and now:
+// [1000, 4096] x [4096, 4096] 43.6 -> 31.6 us (1,060 TOP/s), 2048 rows 61 -> 46, 512 rows 44 -> 20.5, 100 rows 27 -> 17 us.
+template <int WM, int WN, int MI, int NJ, int NS>
+struct Ring {
+    static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, WAVES = WM * WN, STAGE = (TM + TN) * 128, LDS = NS * STAGE;
+    static constexpr int COPIES_A = TM / 8 / WAVES, COPIES_B = TN / 8 / WAVES, COPIES = COPIES_A + COPIES_B;  // of a wavefront and tile
+    static constexpr int PW = TN % 128 == 0 ? 128 : 64;  // columns of a panel of B
+    static_assert(TM % (8 * WAVES) == 0 && TN % (8 * WAVES) == 0 && LDS <= 163840 && (NS - 2) * COPIES + (COPIES + 1) / 2 < 64);
+};
+
+template <bool B_ZP, int WM, int WN, int MI, int NJ, int NS>
+__device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, const uint8_t *A, const uint8_t *B, uint32_t row0,
+                                          uint32_t col0, uint32_t m, uint32_t k, uint32_t n, const uint32_t (&za)[MI], uint32_t zb) {
+    typedef Ring<WM, WN, MI, NJ, NS> R;
+    constexpr int KS = 4, D = 2, PW = R::PW, C = R::COPIES, CA = R::COPIES_A, CB = R::COPIES_B;
+    constexpr int HALF = (C + 1) / 2;  // copies of a tile that are issued in the second half of a step, right behind the barrier
+    constexpr int LINES = 1024 / PW;   // lines of B per copy
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave / WN, wn = wave % WN, h = lane >> 5;
+    auto swizzle_a = [](uint32_t r) -> uint32_t { return (r & 7) ^ ((r >> 3) & 1); };
+    auto swizzle_b = [](uint32_t r) -> uint32_t { return (PW == 128 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1)) ^ ((r >> 4) & 1); };
+    // copy q < CA of this wavefront: rows 8 (CA wave + q) .. + 7 of A's tile; copy CA + q: lines LINES (CB wave + q) .. of B's
+    // panels.  Rows and columns beyond the matrix are copied from inside it (not stored).
+    uint32_t voff[C];
+#pragma unroll
+    for (int q = 0; q < CA; ++q) {
+        const uint32_t r = 8 * (CA * wave + q) + (lane >> 3), row = row0 + r < m ? row0 + r : m - 1;
+        voff[q] = (row - row0) * k + 16 * ((lane & 7) ^ swizzle_a(r));
+    }
+#pragma unroll
+    for (int q = 0; q < CB; ++q) {
+        const uint32_t r = LINES * (CB * wave + q) + lane / (PW / 16), kr = r & 127;
+        const uint32_t col = col0 + PW * (r >> 7) + 16 * ((lane % (PW / 16)) ^ swizzle_b(kr));
+        voff[CA + q] = kr * n + (col + 16 <= n ? col : n - 16);
+    }
+    const uint8_t *a_base = scalar_pointer(A + static_cast<uint64_t>(row0) * k);
+    const uint8_t *b_base = scalar_pointer(B);
+    const uint32_t lds0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds))));
+    auto copy = [&]<int Q>(const uint8_t *a_from, const uint8_t *b_from, uint32_t stage) __attribute__((always_inline)) {
+        const uint32_t to = lds0 + stage + 1024 * (Q < CA ? CA * wave + Q : R::TM / 8 + CB * wave + (Q - CA));
+        const uint8_t *from = Q < CA ? a_from : b_from;
+        const uint32_t lane_off = voff[Q];
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(lane_off), "s"(from), "s"(to)
+                     : "memory", "m0");
+    };
+    const uint32_t a_off = (wm * 32 * MI + (lane & 31)) * 128 + 16 * (h ^ swizzle_a(lane & 31));
+    auto read_a = [&](uint32_t stage, int ks, int i) -> v4i {
+        return *reinterpret_cast<const v4i *>(lds + stage + (a_off ^ (32 * ks)) + i * 4096);
+    };
+    uint32_t b_off[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t a16 = lane & 15, r = 16 * h + (a16 >> 1), col = 32 * (wn * NJ + j);
+        const uint32_t chunk = (col % PW) / 16 + ((lane >> 4) & 1);
+        b_off[j] = R::TM * 128 + (col / PW) * 128 * PW + r * PW + 16 * (chunk ^ swizzle_b(r)) + 8 * (a16 & 1);
+    }
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    auto read_b = [&](uint32_t stage, int ks, int j, v4i &f) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            // (8 or 32 k-rows further a chunk's position is the same)
+            const v2i w = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                (__attribute__((address_space(3))) v2i *)(lds + stage + b_off[j] + (32 * ks + 8 * half) * PW));
+            f[2 * half] = w[0];
+            f[2 * half + 1] = w[1];
+        }
+    };
+
+    const uint32_t k_tiles = (k + 127) / 128;
+    const bool half_tile = k % 128 != 0;  // k is a multiple of 64, at least 128
+    auto tile_k = [&](uint32_t t) -> uint32_t { return t + 1 < k_tiles ? t * 128 : t + 1 == k_tiles ? k - 128 : 0; };
+    auto a_tile = [&](uint32_t t) { return scalar_pointer(a_base + tile_k(t)); };
+    auto b_tile = [&](uint32_t t) { return scalar_pointer(b_base + static_cast<uint64_t>(tile_k(t)) * n); };
+    // tiles 0 .. NS - 2 and the first half of tile NS - 1's copies (behind the end: tile 0 again, never multiplied)
+    auto fill = [&]<int COUNT>(uint32_t tile, uint32_t stage) __attribute__((always_inline)) {
+        const uint8_t *a_from = a_tile(tile), *b_from = b_tile(tile);
+        [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
+            (copy.template operator()<Q>(a_from, b_from, stage), ...);
+        }(std::make_integer_sequence<int, COUNT>{});
+    };
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s) fill.template operator()<C>(s, s * R::STAGE);
+    fill.template operator()<HALF>(NS - 1, (NS - 1) * R::STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * C + HALF) : "memory");  // tile 0
+    __syncthreads();
+    v4i fa[KS][MI], fb[KS][NJ];
+#pragma unroll
+    for (int ks = 0; ks < D; ++ks) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[ks][i] = read_a(0, ks, i);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) read_b(0, ks, j, fb[ks][j]);
+    }
+    auto fix = [&](int ks, int w) {  // word w of the fragments of k-step ks
+        if (w < 4 * MI) fa[ks][w / 4][w % 4] = static_cast<int>(sub_bytes(static_cast<uint32_t>(fa[ks][w / 4][w % 4]), za[w / 4]));
+        else if (B_ZP) fb[ks][w / 4 - MI][w % 4] = static_cast<int>(sub_bytes(static_cast<uint32_t>(fb[ks][w / 4 - MI][w % 4]), zb));
+    };
+    constexpr int WORDS = 4 * (MI + (B_ZP ? NJ : 0));
+#pragma unroll
+    for (int w = 0; w < WORDS; ++w) fix(0, w);
+    // MODE 0: tile t + NS exists; 1: tile t + NS - 1 is the last one; 2: nothing is left to copy.  SKIP: of the tile's four
+    // k-steps only the last two are multiplied.
+    auto step = [&]<int MODE, bool SKIP>(uint32_t t, uint32_t stage, uint32_t next, uint32_t prev) __attribute__((always_inline)) {
+        constexpr int P = MI * NJ, SLOTS = KS * P;
+        const uint8_t *a_old = a_tile(t + NS - 1), *b_old = b_tile(t + NS - 1), *a_new = a_tile(t + NS), *b_new = b_tile(t + NS);
+        auto slot = [&]<int s>() __attribute__((always_inline)) {
+            constexpr int ks = s / P, o = s % P, row = o / NJ, col = (row & 1) ? NJ - 1 - o % NJ : o % NJ;
+            if constexpr (s == D * P) {
+                // tile t + 1 has landed and this wavefront's reads of tile t are done
+                if constexpr (MODE == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * C) : "memory");
+                __syncthreads();
+            }
+            if constexpr (!SKIP || ks >= 2)
+                acc[row][col] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks][row], fb[ks][col], acc[row][col], 0, 0, 0);
+            constexpr int nks = (ks + D) % KS;
+            const uint32_t src = ks < D ? stage : next;
+            [&]<int... F>(std::integer_sequence<int, F...>) __attribute__((always_inline)) {
+                ([&] {
+                    if constexpr (F / 2 == o || (o == P - 1 && F / 2 >= P)) {
+                        if constexpr (F < NJ) read_b(src, nks, F, fb[nks][F]);
+                        else fa[nks][F - NJ] = read_a(src, nks, F - NJ);
+                    }
+                }(), ...);
+            }(std::make_integer_sequence<int, MI + NJ>{});
+#pragma unroll
+            for (int w = 0; w < WORDS; ++w)
+                if (w * P / WORDS == o) fix((ks + 1) % KS, w);
+            [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
+                ([&] {
+                    if constexpr (MODE < 2 && s < D * P && Q < C - HALF && Q * D * P / HALF == s) copy.template operator()<HALF + Q>(a_old, b_old, prev);
+                    if constexpr (MODE < 1 && s >= D * P && Q * D * P / HALF == s - D * P) copy.template operator()<Q>(a_new, b_new, stage);
+                }(), ...);
+            }(std::make_integer_sequence<int, HALF>{});
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+            (slot.template operator()<I>(), ...);
+        }(std::make_integer_sequence<int, SLOTS>{});
+    };
+    uint32_t t = 0, stage = 0, prev = (NS - 1) * R::STAGE;
+    auto next = [&] { return stage + R::STAGE == static_cast<uint32_t>(R::LDS) ? 0u : stage + R::STAGE; };
+    auto advance = [&] {
+        ++t;
+        prev = stage;
+        stage = next();
+    };
+    for (; t + NS < k_tiles; advance()) step.template operator()<0, false>(t, stage, next(), prev);
+    if (t + NS == k_tiles) {
+        step.template operator()<1, false>(t, stage, next(), prev);
+        advance();
+    }
+    const uint32_t whole = half_tile ? k_tiles - 1 : k_tiles;
+    for (; t < whole; advance()) step.template operator()<2, false>(t, stage, next(), prev);
+    if (half_tile) step.template operator()<2, true>(t, stage, next(), prev);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land after the workgroup's LDS is released
+}
+
+template <bool DEQ, int WM, int WN, int MI, int NJ, int NS>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 2 : 1) void mmi_ring(
+    int32_t *__restrict__ y, const uint8_t *__restrict__ a, const uint8_t *__restrict__ b, ZeroPoint za, ZeroPoint zb, Dequant dq,
+    uint32_t m, uint32_t k, uint32_t n, uint32_t a_matrix0, uint32_t b_matrix0, uint32_t y_matrix0) {
+    typedef Ring<WM, WN, MI, NJ, NS> R;
+    __shared__ __align__(1024) uint8_t lds[R::LDS];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, bz = blockIdx.z;
+    const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
+    // consecutive workgroup ids go round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, walked down the
+    // rows of one column panel after the other
+    const uint32_t row_tiles = (m + R::TM - 1) / R::TM, n_tiles = row_tiles * ((n + R::TN - 1) / R::TN);
+    const uint32_t xcd = blockIdx.x % 8, share = n_tiles / 8, more = n_tiles % 8;
+    const uint32_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / 8;
+    const uint32_t row0 = (tile % row_tiles) * R::TM, col0 = (tile / row_tiles) * R::TN;
+    const uint32_t wave_row = row0 + (wave / WN) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
+    uint32_t za_f[MI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const uint32_t row = wave_row + 32 * i + (lane & 31);
+        za_f[i] = splat(zp_byte(za, am * m + (row < m ? row : m - 1)));
+    }
+    const uint32_t zb_f = splat(zp_byte(zb, 0));  // (none or a scalar)
+    v16i acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
+    const uint8_t *A = a + am * m * static_cast<uint64_t>(k), *B = b + bm * static_cast<uint64_t>(k) * n;
+    if (zb_f == 0) ring_loop<false, WM, WN, MI, NJ, NS>(acc, lds, A, B, row0, col0, m, k, n, za_f, 0);
+    else ring_loop<true, WM, WN, MI, NJ, NS>(acc, lds, A, B, row0, col0, m, k, n, za_f, zb_f);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t col = wave_col + 32 * j + (lane & 31);
+        if (col >= n) continue;
+        const float scale = DEQ ? dq.scale[dq.per_column ? col : 0] : 0.f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t row = wave_row + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
+                if (row < m) y[(ym * m + row) * n + col] = finish<DEQ>(acc[i][j][e], scale);
+            }
+    }
+}
+
 }  // namespace
 }  // namespace rg
 
@@ -1059,6 +1281,22 @@ int launch_gemv(int32_t *y, const uint8_t *a, const uint8_t *b, ZeroPoint za, Ze
     return launch_status();
 }
 
+// The shapes of mmi_ring and what a launch takes: `fixed` us a round of 256 workgroups (a CU holds one), and per 128 of k
+// `alone` ns while few CUs have a tile, `full` ns while all have one.
+struct RingShape {
+    uint32_t rows, cols;
+    double fixed, alone, full;
+};
+constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 410, 430}, {64, 128, 3.5, 420, 535}, {128, 128, 6, 530, 800}, {128, 256, 9, 660, 1140}};
+constexpr int kRingShapeCount = 4;
+constexpr RingShape kLargeShape = {256, 256, 12, 1250, 1800};  // mmi_mfma_256x256
+
+inline double ring_us(const RingShape &t, size_t m, size_t n, double steps, size_t count) {
+    const double tiles = static_cast<double>((m + t.rows - 1) / t.rows) * static_cast<double>((n + t.cols - 1) / t.cols) * static_cast<double>(count);
+    const double rounds = static_cast<double>(static_cast<uint64_t>(tiles / 256)), left = tiles / 256 - rounds;
+    return rounds * (t.fixed + 1e-3 * steps * t.full) + (left > 0 ? t.fixed + 1e-3 * steps * (t.alone + (t.full - t.alone) * left) : 0);
+}
+
 template <bool DEQ>
 int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const void *b_zp, unsigned flags,
                size_t batch, size_t m, size_t k, size_t n, const uint32_t *a_index, const uint32_t *b_index,
@@ -1108,6 +1346,43 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
                       (!zb.ptr || !zb.per_row || (reinterpret_cast<uintptr_t>(zb.ptr) & 3u) == 0);
 
     const bool short_tile = short_ok && !gemv && (skinny ? m > 64 : true);
+
+    // the ring tiles, any number of rows from five on: no zero points of B or one for all of it
+    const bool ring = !gemv && k % 64 == 0 && k >= BK && k < (1u << 23) && n % 16 == 0 && n < (1u << 24) && aligned16(a) && aligned16(b) &&
+                      !(zb.ptr && zb.per_row);
+    // Shape with the earliest expected end (us, from measurements at k = 1024 and 4096 like those in kRingShapes), or -1 where
+    // that is one of the other kernels: 256 x 256 tiles, or up to 32 rows mmi_skinny's three launches.
+    auto ring_shape = [&](uint32_t count) -> int {
+        const double steps = static_cast<double>((k + BK - 1) / BK);
+        int best = -1;
+        double us = 1e30;
+        for (int i = 0; i < kRingShapeCount; ++i) {
+            const double t = ring_us(kRingShapes[i], m, n, steps, count);
+            if (t < us) us = t, best = i;
+        }
+        if (fast && ring_us(kLargeShape, m, n, steps, count) < us) return -1;
+        if (skinny && m <= 32 && 8.5 + (DEQ ? 3.5 : 0) + 0.85e-3 * static_cast<double>(n) * count * steps / 32 < us) return -1;
+        return best;
+    };
+    auto launch_ring = [&](int shape, uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
+        const RingShape &t = kRingShapes[shape];
+        const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
+        if (tiles > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
+        const dim3 grid(static_cast<unsigned>(tiles), 1, count);
+        const auto *a8 = static_cast<const uint8_t *>(a);
+        const auto *b8 = static_cast<const uint8_t *>(b);
+        const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
+#define RG_RING(WM, WN, MI, NJ, NS) \
+    mmi_ring<DEQ, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a8, b8, za, zb, dq, m32, k32, n32, am0, bm0, ym0)
+        switch (shape) {
+            case 0: RG_RING(2, 2, 1, 1, 8); break;
+            case 1: RG_RING(2, 4, 1, 1, 6); break;
+            case 2: RG_RING(4, 2, 1, 2, 4); break;
+            default: RG_RING(4, 2, 1, 4, 3);
+        }
+#undef RG_RING
+        return launch_status();
+    };
 
     // the 256 x 256 tiles, with k split between workgroups when the tiles are few
     auto launch_tiles = [&](auto short_m, uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
@@ -1182,6 +1457,11 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
     const bool small_tiles_ok = k % 16 == 0 && k > 0 && small_tiles_rows && aligned16(a) && ((m + GT - 1) / GT) * ((n + GT - 1) / GT) <= 0x7fffffffu;
 
     auto launch = [&](uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
+        if (ring) {
+            const int shape = ring_shape(count);
+            if (shape >= 0) return launch_ring(shape, am0, bm0, ym0, count);
+            if (fast) return launch_tiles(std::false_type{}, am0, bm0, ym0, count);
+        }
         if (small_tiles_ok && (short_tile || (fast && !gemv && !skinny)) && small_tiles_pay(short_tile, count))
             return launch_small_tiles(am0, bm0, ym0, count);
         if (short_tile) return launch_tiles(std::true_type{}, am0, bm0, ym0, count);

@@ -663,6 +663,24 @@ def test_matmul_integer_one_to_four_rows_matrix_vector(m, k, n):
     assert np.all(ye == k * 16384)
 
 
+@pytest.mark.parametrize("m,k,n", [(5, 128, 16), (33, 192, 80), (64, 704, 1040), (100, 1088, 4096), (130, 960, 272), (300, 640, 4112),
+                                   (513, 576, 4096), (1000, 1088, 4096), (2048, 448, 4096), (1025, 320, 6160)])
+def test_matmul_integer_ring_tiles(m, k, n):
+    """Edges of the tiles, k that ends with half a tile, fewer k-tiles than the ring has stages, every zero point form."""
+    rng = np.random.default_rng(m + k + n)
+    a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(-128, 128, (k, n), dtype=np.int8)
+    s = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
+    wrap = lambda t: t.astype(np.int8).astype(np.float64)
+    for az, bz in ((None, None), (121, None), (128, 0), (rng.integers(0, 256, m, dtype=np.uint8), -77)):
+        za = None if az is None else np.atleast_1d(np.asarray(az, np.uint8))
+        zb = None if bz is None else np.array([bz], np.int8)
+        A = wrap(a.astype(np.int64) - (0 if za is None else za.astype(np.int64).reshape(-1, 1)))
+        ref = (A @ wrap(b.astype(np.int64) - (bz or 0))).astype(np.int32)
+        t = [None if z is None else dev(z) for z in (za, zb)]
+        assert np.array_equal(host(ops.matmul_integer(dev(a), dev(b), *t)), ref)
+        assert np.array_equal(host(ops.matmul_integer(dev(a), dev(b), *t, dequant_scale=dev(s))), ref.astype(np.float32) * s)
+
+
 def test_matmul_integer_extremes():
     a = np.zeros((256, 4096), np.uint8)
     b = np.full((4096, 256), -128, np.int8)
