@@ -2072,11 +2072,14 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     // Up to 8 rows only where the plain kernel is expected to take longer (it needs 2.9 ns per thousand elements of B,
     // 596 us for [8, 4096] x [4096, 50257]; a tile launch about 4 us and 0.83 us per 64 of k).
     const size_t side_by_side = a_index || b_index ? 1 : batch;  // matrices that are tiles of one launch
-    const bool tiles16_rows = m > 8 || static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k);
-    const bool tiles16 = narrow && !trans_a && k % 8 == 0 && k > 0 && tiles16_rows && aligned16(a) && (!trans_b || aligned16(b));
+    const bool tile_operands = narrow && !trans_a && k % 8 == 0 && k > 0 && aligned16(a) && (!trans_b || aligned16(b));
     const size_t tiles128 = ((m + HT - 1) / HT) * ((n + HT - 1) / HT) * side_by_side;
-    const bool ring = tiles16 && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
-    const RingPlan plan = ring ? ring_plan(m, k, n, side_by_side) : RingPlan{0, 0, 0, 0};
+    const bool ring_ok = tile_operands && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
+    const RingPlan plan = ring_ok ? ring_plan(m, k, n, side_by_side) : RingPlan{0, 0, 0, 1e30};
+    // (the plain kernel's own chain of steps is 0.54 us per 16 of k: [8, 3648] x [2376, 3648]^T 123 us, 14 on the ring)
+    const bool tiles16_rows = m > 8 || static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k) ||
+                              plan.us < 0.034 * static_cast<double>(k);
+    const bool tiles16 = tile_operands && tiles16_rows, ring = ring_ok && tiles16_rows;
     // A short k leaves a tile little to do between fetching its operands and storing its results, and two small tiles
     // per CU overlap the one's stores with the other's loads: with k <= 128 (k <= 512 below 256 rows) more tiles than CUs
     // are mm_tiles16's ([8192, 128] x [128, 8192] 76 us, 32 products [128, 128] x [4096, 128]^T 25 us).
