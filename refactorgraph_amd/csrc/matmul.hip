@@ -2075,10 +2075,14 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     const bool tile_operands = narrow && !trans_a && k % 8 == 0 && k > 0 && aligned16(a) && (!trans_b || aligned16(b));
     const size_t tiles128 = ((m + HT - 1) / HT) * ((n + HT - 1) / HT) * side_by_side;
     const bool ring_ok = tile_operands && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
-    const RingPlan plan = ring_ok ? ring_plan(m, k, n, side_by_side) : RingPlan{0, 0, 0, 1e30};
+    RingPlan plan{0, 0, 0, 0};
+    auto tiles_plan = [&]() -> const RingPlan & {  // (worked out for the launches that look at it)
+        if (plan.us == 0) plan = ring_plan(m, k, n, side_by_side);
+        return plan;
+    };
     // (the plain kernel's own chain of steps is 0.54 us per 16 of k: [8, 3648] x [2376, 3648]^T 123 us, 14 on the ring)
     const bool tiles16_rows = m > 8 || static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k) ||
-                              plan.us < 0.034 * static_cast<double>(k);
+                              (ring_ok && !gemv && !rows && !gemv_kn && tiles_plan().us < 0.034 * static_cast<double>(k));
     const bool tiles16 = tile_operands && tiles16_rows, ring = ring_ok && tiles16_rows;
     // A short k leaves a tile little to do between fetching its operands and storing its results, and two small tiles
     // per CU overlap the one's stores with the other's loads: with k <= 128 (k <= 512 below 256 rows) more tiles than CUs
@@ -2089,17 +2093,19 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     // measurements at k = 4096: mm_skinny 13.5 for 32 and 19 for 64 rows of 4096 columns, 38 for 11008 columns;
     // mm_rows_kn 22 for 32 rows of 4096 columns; a pass of four rows of mm_gemv_kn 4.3, or B at 5 TB/s).  One to 16 rows
     // that mm_gemv and mm_rows take read W as [n, k] once at the speed of the memory whatever n is: never a tile.
-    bool tiles_first = tiles16 && m >= kFewRows;
-    if (tiles16 && !tiles_first && (ring || tiles128 <= kSmallGrid)) {
-        const double tile_us = ring ? plan.us : 4.0 + 0.83 * static_cast<double>((k + HK - 1) / HK);
+    auto tiles_first = [&]() -> bool {
+        if (!tiles16 || m >= kFewRows) return tiles16;
+        if (!ring && tiles128 > kSmallGrid) return false;
+        if (trans_b && (rows || gemv)) return false;
+        const double tile_us = ring ? tiles_plan().us : 4.0 + 0.83 * static_cast<double>((k + HK - 1) / HK);
         const double columns = static_cast<double>(n * side_by_side), k4096 = static_cast<double>(k) / 4096;
         const double skinny_us = static_cast<double>((m + 63) / 64) * (3.0 + columns * (m <= 32 ? 2.6e-3 : 3.4e-3) * k4096);
         const double rows_kn_us = static_cast<double>((m + 31) / 32) * (2.0 + columns * (m <= 16 ? 3.5e-3 : 5.0e-3) * k4096);
         const double b_us = 2.0 * static_cast<double>(k) * columns / 5.0e6;
         const double gemv_kn_us = static_cast<double>((m + 3) / 4) * (b_us > 4.3 ? b_us : 4.3);
-        if (trans_b) tiles_first = rows || gemv ? false : !skinny || tile_us < skinny_us;
-        else tiles_first = rows_kn ? tile_us < rows_kn_us : !gemv_kn || (m > 4 && tile_us < gemv_kn_us);
-    }
+        if (trans_b) return !skinny || tile_us < skinny_us;
+        return rows_kn ? tile_us < rows_kn_us : !gemv_kn || (m > 4 && tile_us < gemv_kn_us);
+    };
 
     // F32 on the matrix cores.  A launch of the 128 x 128 tiles walks all of k in every workgroup and takes about
     // 300 us at k = 4096 however few tiles there are; up to that cost few rows go through the block products of
@@ -2169,11 +2175,12 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
 #undef RG_RING
                 return launch_status();
             };
-            if (plan.columns) {
-                const int rc = part(plan.first, 0, plan.columns);
+            const RingPlan &p = tiles_plan();
+            if (p.columns) {
+                const int rc = part(p.first, 0, p.columns);
                 if (rc) return rc;
             }
-            return part(plan.rest, plan.columns, n32 - plan.columns);
+            return part(p.rest, p.columns, n32 - p.columns);
         } else {
             return RG_HIP_E_UNSUPPORTED;
         }
@@ -2203,7 +2210,7 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                                               static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, workspace, plan, s);
             }
             if (short_k) return launch_tiles16(am0, bm0, ym0, count);
-            if (tiles_first) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
+            if (tiles_first()) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
             if (rows_kn) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 const bool wide = n % 32 == 0 && n >= 8192;

@@ -6,6 +6,7 @@ stream.  Argument meaning follows include/rg_hip.h; outputs are allocated with t
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import math
 
 import numpy as np
@@ -25,12 +26,17 @@ for _name, _code in (("uint16", abi.U16), ("uint32", abi.U32), ("uint64", abi.U6
         _T2CODE[getattr(torch, _name)] = _code
 
 
+# A call's host work is what a decode step of one sequence waits for (seven calls of 13 us each against 40 us of kernels
+# before): addresses go to ctypes as integers, what depends on shapes alone is worked out once per shape (bounded caches of
+# pure functions), two-dimensional products skip the broadcasting of batches.
+
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """Address of torch's current stream of the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _need_gpu(*ts):
@@ -102,7 +108,7 @@ def dequantize_linear(x, scale, zp=None, axis=1, out=None):
         assert scale.numel() == axis_len
     else:
         outer, axis_len, inner = 1, 1, x.numel()
-    y = torch.empty(x.shape, dtype=torch.float32, device=x.device) if out is None else out
+    y = torch.empty_like(x, dtype=torch.float32) if out is None else out
     check(lib().rg_hip_dequantize_linear(_ptr(y), _ptr(x), _ptr(scale), _ptr(zp), outer, axis_len, inner,
                                          _T2CODE[x.dtype], per_axis, _stream()), "rg_hip_dequantize_linear")
     return y
@@ -113,12 +119,11 @@ def dynamic_quantize_linear(x, out=None, workspace=None):
     _need_gpu(x)
     assert x.dtype == torch.float32 and x.is_contiguous()
     n = x.numel()
-    y = torch.empty(x.shape, dtype=torch.uint8, device=x.device) if out is None else out
+    y = torch.empty_like(x, dtype=torch.uint8) if out is None else out
     assert y.dtype == torch.uint8 and y.numel() == n and y.is_contiguous()
-    scale = torch.empty(1, dtype=torch.float32, device=x.device)
-    zp = torch.empty(1, dtype=torch.uint8, device=x.device)
-    nbytes = lib().rg_hip_dynamic_quantize_linear_workspace(n)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if workspace is None else workspace
+    scale = x.new_empty(1)
+    zp = x.new_empty(1, dtype=torch.uint8)
+    ws = x.new_empty(lib().rg_hip_dynamic_quantize_linear_workspace(n), dtype=torch.uint8) if workspace is None else workspace
     check(lib().rg_hip_dynamic_quantize_linear(_ptr(y), _ptr(scale), _ptr(zp), _ptr(x), n, _ptr(ws), ws.numel(),
                                                _stream()), "rg_hip_dynamic_quantize_linear")
     return y, scale, zp
@@ -134,6 +139,26 @@ def cast(x, dtype, out=None):
     return y
 
 
+def _batches(a, b):
+    """(batch dimensions of a product, their count, indices of a's and of b's matrices or None): the index arrays are
+    needed where the batch dimensions of the operands differ."""
+    if a.dim() == 2 and b.dim() == 2:
+        return (), 1, None, None
+    ab, bb = tuple(a.shape[:-2]), tuple(b.shape[:-2])
+    if ab == bb:
+        return ab, math.prod(ab), None, None
+    ob = tuple(np.broadcast_shapes(ab, bb))
+    ia = np.arange(math.prod(ab), dtype=np.uint32).reshape(ab)
+    ib = np.arange(math.prod(bb), dtype=np.uint32).reshape(bb)
+    oa, obb = np.broadcast_arrays(ia, ib)
+    return ob, math.prod(ob), np.ascontiguousarray(oa.reshape(-1)), np.ascontiguousarray(obb.reshape(-1))
+
+
+@functools.lru_cache(maxsize=4096)
+def _matmul_workspace(*shape):
+    return lib().rg_hip_matmul_workspace(*shape)
+
+
 def matmul(a, b, c=None, trans_a=False, trans_b=False, alpha=1.0, beta=1.0, out=None, workspace=None):
     """Y = alpha * op(A) @ op(B) + beta * C.  a [..., m, k] ([..., k, m] when trans_a), b [..., k, n]
     ([..., n, k] when trans_b), batch dimensions broadcast; c broadcasts to [m, n] (any leading
@@ -143,16 +168,7 @@ def matmul(a, b, c=None, trans_a=False, trans_b=False, alpha=1.0, beta=1.0, out=
     m, k = (a.shape[-1], a.shape[-2]) if trans_a else (a.shape[-2], a.shape[-1])
     n = b.shape[-2] if trans_b else b.shape[-1]
     assert k == (b.shape[-1] if trans_b else b.shape[-2])
-    ab, bb = tuple(a.shape[:-2]), tuple(b.shape[:-2])
-    ob = tuple(np.broadcast_shapes(ab, bb))
-    batch = math.prod(ob)
-    a_idx = b_idx = None
-    if ab != bb:
-        ia = np.arange(math.prod(ab), dtype=np.uint32).reshape(ab)
-        ib = np.arange(math.prod(bb), dtype=np.uint32).reshape(bb)
-        oa, obb = np.broadcast_arrays(ia, ib)
-        a_idx = np.ascontiguousarray(oa.reshape(-1))
-        b_idx = np.ascontiguousarray(obb.reshape(-1))
+    ob, batch, a_idx, b_idx = _batches(a, b)
     sb = sm = sn = 0
     if c is not None:
         assert c.dtype == a.dtype and c.is_contiguous()
@@ -166,10 +182,10 @@ def matmul(a, b, c=None, trans_a=False, trans_b=False, alpha=1.0, beta=1.0, out=
         sn = 1 if cs[-1] == n else 0
         if cs[-2] == 1:
             sm = 0
-    y = torch.empty(ob + (m, n), dtype=a.dtype, device=a.device) if out is None else out
+    y = a.new_empty(ob + (m, n)) if out is None else out
     if workspace is None:
         # what the routine's lowering would ask the allocator for (a uint8 tensor passed as `workspace` is used as is)
-        need = lib().rg_hip_matmul_workspace(_T2CODE[a.dtype], int(trans_a), int(trans_b), batch, m, k, n)
+        need = _matmul_workspace(_T2CODE[a.dtype], int(trans_a), int(trans_b), batch, m, k, n)
         workspace = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
     check(lib().rg_hip_matmul_ws(
         _ptr(y), _ptr(a), _ptr(b), _ptr(c), _T2CODE[a.dtype], int(trans_a), int(trans_b), float(alpha), float(beta),
@@ -218,12 +234,16 @@ def transpose(x, perm, out=None):
     """Contiguous x with its dimensions permuted (any dtype: bytes are moved)."""
     _need_gpu(x)
     assert x.is_contiguous() and sorted(perm) == list(range(x.dim()))
-    si, so, block, count = transpose_info(list(x.shape), list(perm), x.element_size())
-    y = torch.empty([x.shape[p] for p in perm], dtype=x.dtype, device=x.device) if out is None else out
-    si_, so_ = np.asarray(si, np.uint32), np.asarray(so, np.uint32)
-    check(lib().rg_hip_transpose(_ptr(y), _ptr(x), si_.ctypes.data_as(C.c_void_p), so_.ctypes.data_as(C.c_void_p),
-                                 len(si), block, count, _stream()), "rg_hip_transpose")
+    rank, si, so, block, count = _transpose_digest(tuple(x.shape), tuple(perm), x.element_size())
+    y = x.new_empty([x.shape[p] for p in perm]) if out is None else out
+    check(lib().rg_hip_transpose(_ptr(y), _ptr(x), si, so, rank, block, count, _stream()), "rg_hip_transpose")
     return y
+
+
+@functools.lru_cache(maxsize=4096)
+def _transpose_digest(shape, perm, itemsize):
+    si, so, block, count = transpose_info(list(shape), list(perm), itemsize)
+    return len(si), (C.c_uint32 * len(si))(*si), (C.c_uint32 * len(so))(*so), block, count
 
 
 def split_info(part_shapes, axis, itemsize):
@@ -244,14 +264,18 @@ def split(x, sizes, axis, outs=None):
     _need_gpu(x)
     axis %= x.dim()
     assert sum(sizes) == x.shape[axis]
-    shapes = [tuple(x.shape[:axis]) + (n,) + tuple(x.shape[axis + 1:]) for n in sizes]
+    shapes, blocks, total, seg = _split_digest(tuple(x.shape), tuple(sizes), axis, x.element_size())
     if outs is None:
-        outs = [torch.empty(sh, dtype=x.dtype, device=x.device) for sh in shapes]
-    blocks, total, segments = split_info(shapes, axis, x.element_size())
-    seg = np.asarray(segments, np.uint32)
-    check(lib().rg_hip_split(_pointer_array(outs), _ptr(x), seg.ctypes.data_as(C.c_void_p), len(outs), blocks, total,
-                             _stream()), "rg_hip_split")
+        outs = [x.new_empty(sh) for sh in shapes]
+    check(lib().rg_hip_split(_pointer_array(outs), _ptr(x), seg, len(outs), blocks, total, _stream()), "rg_hip_split")
     return outs
+
+
+@functools.lru_cache(maxsize=4096)
+def _split_digest(shape, sizes, axis, itemsize):
+    shapes = [shape[:axis] + (n,) + shape[axis + 1:] for n in sizes]
+    blocks, total, segments = split_info(shapes, axis, itemsize)
+    return shapes, blocks, total, (C.c_uint32 * len(segments))(*segments)
 
 
 def concat(parts, axis, out=None):
@@ -352,17 +376,7 @@ def matmul_integer(a, b, a_zp=None, b_zp=None, out=None, dequant_scale=None):
     m, k = a.shape[-2:]
     k2, n = b.shape[-2:]
     assert k == k2
-    ab, bb = tuple(a.shape[:-2]), tuple(b.shape[:-2])
-    ob = tuple(np.broadcast_shapes(ab, bb))
-    batch = math.prod(ob)
-    a_idx = b_idx = None
-    if ab != bb:
-        na, nb = math.prod(ab), math.prod(bb)
-        ia = np.arange(na, dtype=np.uint32).reshape(ab)
-        ib = np.arange(nb, dtype=np.uint32).reshape(bb)
-        oa, obb = np.broadcast_arrays(ia, ib)
-        a_idx = np.ascontiguousarray(oa.reshape(-1))
-        b_idx = np.ascontiguousarray(obb.reshape(-1))
+    ob, batch, a_idx, b_idx = _batches(a, b)
     flags = 0
     if a_zp is not None and a_zp.numel() == 1:
         flags |= abi.MMI_A_ZP_SCALAR
@@ -370,14 +384,14 @@ def matmul_integer(a, b, a_zp=None, b_zp=None, out=None, dequant_scale=None):
         flags |= abi.MMI_B_ZP_SCALAR
     if dequant_scale is not None:
         assert dequant_scale.dtype == torch.float32 and dequant_scale.numel() in (1, n)
-        y = torch.empty(ob + (m, n), dtype=torch.float32, device=a.device) if out is None else out
+        y = a.new_empty(ob + (m, n), dtype=torch.float32) if out is None else out
         check(lib().rg_hip_matmul_integer_dequantize(
             _ptr(y), _ptr(a), _ptr(b), _ptr(a_zp), _ptr(b_zp), flags, batch, m, k, n,
             None if a_idx is None else a_idx.ctypes.data_as(C.c_void_p),
             None if b_idx is None else b_idx.ctypes.data_as(C.c_void_p),
             _ptr(dequant_scale), int(dequant_scale.numel() != 1), None, _stream()), "rg_hip_matmul_integer_dequantize")
         return y
-    y = torch.empty(ob + (m, n), dtype=torch.int32, device=a.device) if out is None else out
+    y = a.new_empty(ob + (m, n), dtype=torch.int32) if out is None else out
     check(lib().rg_hip_matmul_integer(
         _ptr(y), _ptr(a), _ptr(b), _ptr(a_zp), _ptr(b_zp), flags, batch, m, k, n,
         None if a_idx is None else a_idx.ctypes.data_as(C.c_void_p),
