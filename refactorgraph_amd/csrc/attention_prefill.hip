@@ -130,7 +130,7 @@ struct PrefillPlan {
     uint32_t group;        // query heads per kv head
     uint32_t head_chunks;  // group / HW
     uint32_t q_tiles;      // query tiles (of ROWS rows) per stream
-    uint32_t pairs;        // (q_tiles + 1) / 2: workgroups that share a stream
+    uint32_t pairs;        // (q_tiles + 1) / 2, SPLIT: q_tiles: workgroups that share a stream
     uint32_t xcds;         // 8 when the streams divide evenly over the XCDs, else 1
     uint32_t spx;          // streams per XCD
     uint32_t groups;       // sets of `pairs` workgroups per XCD; set g walks streams g, g + groups, ...
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
 
     // Workgroup w: consecutive ids are dealt round-robin to the XCDs.  Within an XCD, set g of
     // `pairs` workgroups walks the XCD's streams g, g + groups, ...; member j of a set takes query
-    // tiles q_tiles - 1 - j and j of each of them (the heavy one first).
+    // tiles q_tiles - 1 - j and j of each of them (the heavy one first; SPLIT: one of the two).
     const uint32_t xcd = uni(blockIdx.x % plan.xcds), lw = uni(blockIdx.x / plan.xcds);
     const uint32_t pj = uni(lw % plan.pairs), set = uni(lw / plan.pairs);
     uint32_t en_k = set, en_sub = 0;
@@ -216,15 +216,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
         raw_past = 0;
         while (en_k < plan.spx) {
             const uint32_t heavy = plan.q_tiles - 1 - pj;
-            const uint32_t qt = en_sub == 0 ? heavy : pj;
-            const bool ok = en_sub == 0 || pj != heavy;
+            // (SPLIT: one query tile a stream, every other set from the other end, so that the two workgroups of a CU
+            // get a long and a short one under a causal prompt)
+            const uint32_t qt = SPLIT ? ((set & 1) ? heavy : pj) : en_sub == 0 ? heavy : pj;
+            const bool ok = SPLIT || en_sub == 0 || pj != heavy;
             uint32_t stream = en_k * plan.xcds + xcd;
             if constexpr (SPLIT) {
                 const uint32_t whole = div_magic(stream, plan.magic_splits);
                 it.ks = stream - whole * plan.splits;
                 stream = whole;
             }
-            if (en_sub == 0) {
+            if (!SPLIT && en_sub == 0) {
                 en_sub = 1;
             } else {
                 en_sub = 0;
@@ -766,10 +768,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
 }
 
 // Finishes the items of a SPLIT launch: workgroups with the threads of attn_prefill (wavefront = head and query
-// sub-tile, lane = query row and half of the keys), each taking eight of a thread's accumulator registers
-// (blockIdx.y: two groups of four consecutive d), add the ranges' records weighted by 2^(m_range - m_max), normalise
+// sub-tile, lane = query row and half of the keys), each taking four of a thread's accumulator registers
+// (blockIdx.y: four consecutive d), add the ranges' records weighted by 2^(m_range - m_max), normalise
 // and store four consecutive d per instruction.
-constexpr int kMergeRegs = 8;
+// (eight registers, half the workgroups: 10.6 against 7.5 us for 32 items of 16 ranges; sixteen: level at 256 items of two)
+constexpr int kMergeRegs = 4;
 template <class T, int HW, int DH>
 __global__ __launch_bounds__(256) void attn_prefill_merge(const PrefillArgs a, const PrefillPlan plan) {
     constexpr int QS = 4 / HW, ROWS = 32 * QS, DBLK = (DH + 31) / 32;
@@ -782,11 +785,12 @@ __global__ __launch_bounds__(256) void attn_prefill_merge(const PrefillArgs a, c
     const float *rec = plan.part + static_cast<uint64_t>(blockIdx.x) * plan.splits * part_floats(DH);
     const uint32_t e0 = blockIdx.y * kMergeRegs;
     float m_max = kMinusBig;
+#pragma unroll 8
     for (uint32_t r = 0; r < plan.splits; ++r) m_max = fmaxf(m_max, rec[r * part_floats(DH) + (DBLK * 16) * 256 + tid]);
     float o[kMergeRegs], l = 0.f;
 #pragma unroll
     for (int e = 0; e < kMergeRegs; ++e) o[e] = 0.f;
-#pragma unroll 4
+#pragma unroll 8
     for (uint32_t r = 0; r < plan.splits; ++r) {
         const float *p = rec + r * part_floats(DH);
         const float w = __builtin_amdgcn_exp2f(p[(DBLK * 16) * 256 + tid] - m_max);
@@ -845,7 +849,12 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
         if (splits > kSplitMax) splits = kSplitMax;
         const uint64_t room = a.part ? a.part_bytes / (items * part_floats(DH) * sizeof(float)) : 0;
         if (splits > room) splits = room;
-        if (splits >= 2 && streams * splits * plan.pairs <= 0x7fffffffu) plan.splits = static_cast<uint32_t>(splits);
+        if (splits >= 2 && streams * splits * plan.q_tiles <= 0x7fffffffu) {
+            plan.splits = static_cast<uint32_t>(splits);
+            // a query tile per workgroup: with a pair each only half of the resident workgroups were launched, one
+            // wavefront on a SIMD (128 new rows behind 16384, 32 heads: 64.7 -> 50.2 us, 690 TFLOP/s)
+            plan.pairs = plan.q_tiles;
+        }
     }
     plan.magic_splits = plan.splits > 1 ? static_cast<uint32_t>((1ull << 32) / plan.splits + 1) : 0;
     plan.part = a.part;
