@@ -580,29 +580,32 @@ __global__ __launch_bounds__(256, 1) void mmi_mfma_256x256(int32_t *__restrict__
 // have their zero point subtracted one k-step ahead; the barrier behind the second k-step frees the stage of tile t for
 // tile t + NS and makes tile t + 1 visible.  Where k ends with half a tile, the last tile starts 64 earlier and its first
 // two k-steps are not multiplied.
+// WK = 2: half of the wavefronts take the first two k-steps of every tile, half the last two (64 x 64 tiles, whose chain of
+// steps is what a launch waits for: [100, 4096] x [4096, 4096] 16.6 -> 14.9 us); their sums meet in LDS at the end.
 // Eight wavefronts for the larger tiles: two on a SIMD, one of which issues products while the other issues its copies or
 // subtracts zero points (four vector instructions per word of A: with 1 x 2 blocks per wavefront they fit behind the products,
 // with 2 x 1 blocks a launch takes 8 % longer).  Bound by what the CUs together take from L2 and the memory-side cache.
 // uint8 activations with an arbitrary zero point, k = 4096, before (mmi_tiles, 256 x 256 tiles with k shared) and now:
 // [1000, 4096] x [4096, 4096] 43.6 -> 31.6 us (1,060 TOP/s), 2048 rows 61 -> 46, 512 rows 44 -> 20.5, 100 rows 27 -> 17 us.
-template <int WM, int WN, int MI, int NJ, int NS>
+template <int WM, int WN, int MI, int NJ, int NS, int WK>
 struct Ring {
-    static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, WAVES = WM * WN, STAGE = (TM + TN) * 128, LDS = NS * STAGE;
+    static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, WAVES = WM * WN * WK, STAGE = (TM + TN) * 128, LDS = NS * STAGE;
     static constexpr int COPIES_A = TM / 8 / WAVES, COPIES_B = TN / 8 / WAVES, COPIES = COPIES_A + COPIES_B;  // of a wavefront and tile
     static constexpr int PW = TN % 128 == 0 ? 128 : 64;  // columns of a panel of B
-    static_assert(TM % (8 * WAVES) == 0 && TN % (8 * WAVES) == 0 && LDS <= 163840 && (NS - 2) * COPIES + (COPIES + 1) / 2 < 64);
+    static_assert(TM % (8 * WAVES) == 0 && TN % (8 * WAVES) == 0 && LDS <= 163840 && (NS - 1) * COPIES < 64 && (WK == 1 || WK == 2));
 };
 
-template <bool B_ZP, int WM, int WN, int MI, int NJ, int NS>
+template <bool B_ZP, int WM, int WN, int MI, int NJ, int NS, int WK>
 __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, const uint8_t *A, const uint8_t *B, uint32_t row0,
                                           uint32_t col0, uint32_t m, uint32_t k, uint32_t n, const uint32_t (&za)[MI], uint32_t zb) {
-    typedef Ring<WM, WN, MI, NJ, NS> R;
-    constexpr int KS = 4, D = 2, PW = R::PW, C = R::COPIES, CA = R::COPIES_A, CB = R::COPIES_B;
-    constexpr int HALF = (C + 1) / 2;  // copies of a tile that are issued in the second half of a step, right behind the barrier
+    typedef Ring<WM, WN, MI, NJ, NS, WK> R;
+    constexpr int KS = 4 / WK, D = 2, PW = R::PW,  // k-steps of a wavefront, k-steps from a fragment's read to its product
+                  C = R::COPIES, CA = R::COPIES_A, CB = R::COPIES_B;
+    constexpr int HALF = D == KS ? C : (C + 1) / 2;  // copies of a tile that are issued in the second half of a step, right behind the barrier
     constexpr int LINES = 1024 / PW;   // lines of B per copy
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wm = wave / WN, wn = wave % WN, h = lane >> 5;
+    const uint32_t kq = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN, h = lane >> 5;
     auto swizzle_a = [](uint32_t r) -> uint32_t { return (r & 7) ^ ((r >> 3) & 1); };
     auto swizzle_b = [](uint32_t r) -> uint32_t { return (PW == 128 ? 2 * ((r >> 1) & 3) : 2 * ((r >> 2) & 1)) ^ ((r >> 4) & 1); };
     // copy q < CA of this wavefront: rows 8 (CA wave + q) .. + 7 of A's tile; copy CA + q: lines LINES (CB wave + q) .. of B's
@@ -632,7 +635,7 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
                      : "v"(lane_off), "s"(from), "s"(to)
                      : "memory", "m0");
     };
-    const uint32_t a_off = (wm * 32 * MI + (lane & 31)) * 128 + 16 * (h ^ swizzle_a(lane & 31));
+    const uint32_t a_off = (wm * 32 * MI + (lane & 31)) * 128 + (16 * (h ^ swizzle_a(lane & 31)) ^ (32 * KS * (WK > 1 ? kq : 0)));
     auto read_a = [&](uint32_t stage, int ks, int i) -> v4i {
         return *reinterpret_cast<const v4i *>(lds + stage + (a_off ^ (32 * ks)) + i * 4096);
     };
@@ -641,7 +644,7 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
     for (int j = 0; j < NJ; ++j) {
         const uint32_t a16 = lane & 15, r = 16 * h + (a16 >> 1), col = 32 * (wn * NJ + j);
         const uint32_t chunk = (col % PW) / 16 + ((lane >> 4) & 1);
-        b_off[j] = R::TM * 128 + (col / PW) * 128 * PW + r * PW + 16 * (chunk ^ swizzle_b(r)) + 8 * (a16 & 1);
+        b_off[j] = R::TM * 128 + (col / PW) * 128 * PW + (r + 32 * KS * (WK > 1 ? kq : 0)) * PW + 16 * (chunk ^ swizzle_b(r)) + 8 * (a16 & 1);
     }
     typedef int v2i __attribute__((ext_vector_type(2)));
     auto read_b = [&](uint32_t stage, int ks, int j, v4i &f) {
@@ -685,8 +688,12 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
         else if (B_ZP) fb[ks][w / 4 - MI][w % 4] = static_cast<int>(sub_bytes(static_cast<uint32_t>(fb[ks][w / 4 - MI][w % 4]), zb));
     };
     constexpr int WORDS = 4 * (MI + (B_ZP ? NJ : 0));
+    // (a wavefront with two k-steps a tile reads a whole tile ahead and subtracts right before the products)
+    constexpr int AHEAD = D == KS ? 0 : 1;
+    if constexpr (AHEAD != 0) {
 #pragma unroll
-    for (int w = 0; w < WORDS; ++w) fix(0, w);
+        for (int w = 0; w < WORDS; ++w) fix(0, w);
+    }
     // MODE 0: tile t + NS exists; 1: tile t + NS - 1 is the last one; 2: nothing is left to copy.  SKIP: of the tile's four
     // k-steps only the last two are multiplied.
     auto step = [&]<int MODE, bool SKIP>(uint32_t t, uint32_t stage, uint32_t next, uint32_t prev) __attribute__((always_inline)) {
@@ -694,16 +701,20 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
         const uint8_t *a_old = a_tile(t + NS - 1), *b_old = b_tile(t + NS - 1), *a_new = a_tile(t + NS), *b_new = b_tile(t + NS);
         auto slot = [&]<int s>() __attribute__((always_inline)) {
             constexpr int ks = s / P, o = s % P, row = o / NJ, col = (row & 1) ? NJ - 1 - o % NJ : o % NJ;
-            if constexpr (s == D * P) {
+            if constexpr (s == (KS - D) * P) {
                 // tile t + 1 has landed and this wavefront's reads of tile t are done
                 if constexpr (MODE == 2) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
                 else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * C) : "memory");
                 __syncthreads();
             }
-            if constexpr (!SKIP || ks >= 2)
+            if constexpr (AHEAD == 0 && o == 0) {
+#pragma unroll
+                for (int w = 0; w < WORDS; ++w) fix(ks, w);
+            }
+            if (!SKIP || (WK == 1 ? ks >= 2 : kq != 0))
                 acc[row][col] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks][row], fb[ks][col], acc[row][col], 0, 0, 0);
             constexpr int nks = (ks + D) % KS;
-            const uint32_t src = ks < D ? stage : next;
+            const uint32_t src = ks < KS - D ? stage : next;
             [&]<int... F>(std::integer_sequence<int, F...>) __attribute__((always_inline)) {
                 ([&] {
                     if constexpr (F / 2 == o || (o == P - 1 && F / 2 >= P)) {
@@ -712,13 +723,15 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
                     }
                 }(), ...);
             }(std::make_integer_sequence<int, MI + NJ>{});
+            if constexpr (AHEAD != 0) {
 #pragma unroll
-            for (int w = 0; w < WORDS; ++w)
-                if (w * P / WORDS == o) fix((ks + 1) % KS, w);
+                for (int w = 0; w < WORDS; ++w)
+                    if (w * P / WORDS == o) fix((ks + 1) % KS, w);
+            }
             [&]<int... Q>(std::integer_sequence<int, Q...>) __attribute__((always_inline)) {
                 ([&] {
-                    if constexpr (MODE < 2 && s < D * P && Q < C - HALF && Q * D * P / HALF == s) copy.template operator()<HALF + Q>(a_old, b_old, prev);
-                    if constexpr (MODE < 1 && s >= D * P && Q * D * P / HALF == s - D * P) copy.template operator()<Q>(a_new, b_new, stage);
+                    if constexpr (MODE < 2 && s < (KS - D) * P && Q < C - HALF && Q * D * P / HALF == s) copy.template operator()<HALF + Q>(a_old, b_old, prev);
+                    if constexpr (MODE < 1 && s >= (KS - D) * P && Q * D * P / HALF == s - (KS - D) * P) copy.template operator()<Q>(a_new, b_new, stage);
                 }(), ...);
             }(std::make_integer_sequence<int, HALF>{});
             __builtin_amdgcn_sched_barrier(0);
@@ -745,11 +758,11 @@ __device__ __forceinline__ void ring_loop(v16i (&acc)[MI][NJ], uint8_t *lds, con
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land after the workgroup's LDS is released
 }
 
-template <bool DEQ, int WM, int WN, int MI, int NJ, int NS>
-__global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 2 : 1) void mmi_ring(
+template <bool DEQ, int WM, int WN, int MI, int NJ, int NS, int WK>
+__global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK > 4 ? 2 : 1) void mmi_ring(
     int32_t *__restrict__ y, const uint8_t *__restrict__ a, const uint8_t *__restrict__ b, ZeroPoint za, ZeroPoint zb, Dequant dq,
     uint32_t m, uint32_t k, uint32_t n, uint32_t a_matrix0, uint32_t b_matrix0, uint32_t y_matrix0) {
-    typedef Ring<WM, WN, MI, NJ, NS> R;
+    typedef Ring<WM, WN, MI, NJ, NS, WK> R;
     __shared__ __align__(1024) uint8_t lds[R::LDS];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, bz = blockIdx.z;
     const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
@@ -759,7 +772,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 2 : 1) void mmi_ring(
     const uint32_t xcd = blockIdx.x % 8, share = n_tiles / 8, more = n_tiles % 8;
     const uint32_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / 8;
     const uint32_t row0 = (tile % row_tiles) * R::TM, col0 = (tile / row_tiles) * R::TN;
-    const uint32_t wave_row = row0 + (wave / WN) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
+    const uint32_t wave_row = row0 + (wave / WN % WM) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
     uint32_t za_f[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -775,8 +788,20 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN > 4 ? 2 : 1) void mmi_ring(
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
     const uint8_t *A = a + am * m * static_cast<uint64_t>(k), *B = b + bm * static_cast<uint64_t>(k) * n;
-    if (zb_f == 0) ring_loop<false, WM, WN, MI, NJ, NS>(acc, lds, A, B, row0, col0, m, k, n, za_f, 0);
-    else ring_loop<true, WM, WN, MI, NJ, NS>(acc, lds, A, B, row0, col0, m, k, n, za_f, zb_f);
+    if (zb_f == 0) ring_loop<false, WM, WN, MI, NJ, NS, WK>(acc, lds, A, B, row0, col0, m, k, n, za_f, 0);
+    else ring_loop<true, WM, WN, MI, NJ, NS, WK>(acc, lds, A, B, row0, col0, m, k, n, za_f, zb_f);
+    if constexpr (WK > 1) {  // the second half of k joins the first through LDS
+        int32_t *part = reinterpret_cast<int32_t *>(lds) + (wave % (WM * WN)) * (MI * NJ * 16 * 64) + lane;
+        __syncthreads();  // every wavefront has read its last fragments
+        if (wave >= WM * WN) {
+#pragma unroll
+            for (int i = 0; i < MI * NJ * 16; ++i) part[i * 64] = acc[i / 16 / NJ][i / 16 % NJ][i % 16];
+        }
+        __syncthreads();
+        if (wave >= WM * WN) return;
+#pragma unroll
+        for (int i = 0; i < MI * NJ * 16; ++i) acc[i / 16 / NJ][i / 16 % NJ][i % 16] += part[i * 64];
+    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const uint32_t col = wave_col + 32 * j + (lane & 31);
@@ -1287,7 +1312,7 @@ struct RingShape {
     uint32_t rows, cols;
     double fixed, alone, full;
 };
-constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 410, 430}, {64, 128, 3.5, 420, 535}, {128, 128, 6, 530, 800}, {128, 256, 9, 660, 1140}};
+constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 370, 390}, {64, 128, 3.5, 420, 535}, {128, 128, 6, 530, 800}, {128, 256, 9, 660, 1140}};
 constexpr int kRingShapeCount = 4;
 constexpr RingShape kLargeShape = {256, 256, 12, 1250, 1800};  // mmi_mfma_256x256
 
@@ -1372,13 +1397,13 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
         const auto *a8 = static_cast<const uint8_t *>(a);
         const auto *b8 = static_cast<const uint8_t *>(b);
         const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
-#define RG_RING(WM, WN, MI, NJ, NS) \
-    mmi_ring<DEQ, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a8, b8, za, zb, dq, m32, k32, n32, am0, bm0, ym0)
+#define RG_RING(WM, WN, MI, NJ, NS, WK) \
+    mmi_ring<DEQ, WM, WN, MI, NJ, NS, WK><<<grid, 64 * WM * WN * WK, 0, s>>>(y, a8, b8, za, zb, dq, m32, k32, n32, am0, bm0, ym0)
         switch (shape) {
-            case 0: RG_RING(2, 2, 1, 1, 8); break;
-            case 1: RG_RING(2, 4, 1, 1, 6); break;
-            case 2: RG_RING(4, 2, 1, 2, 4); break;
-            default: RG_RING(4, 2, 1, 4, 3);
+            case 0: RG_RING(2, 2, 1, 1, 8, 2); break;
+            case 1: RG_RING(2, 4, 1, 1, 6, 1); break;
+            case 2: RG_RING(4, 2, 1, 2, 4, 1); break;
+            default: RG_RING(4, 2, 1, 4, 3, 1);
         }
 #undef RG_RING
         return launch_status();
@@ -1566,3 +1591,4 @@ extern "C" int rg_hip_matmul_integer_dequantize(float *y, const void *a, const v
     return rg::mmi_launch<true>(reinterpret_cast<int32_t *>(y), a, b, a_zp, b_zp, flags, batch, m, k, n, a_index, b_index,
                                 rg::Dequant{scale, scale_per_column ? 1u : 0u}, stream);
 }
+
