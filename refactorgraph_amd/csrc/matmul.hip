@@ -628,9 +628,17 @@ __device__ __forceinline__ void ring_loop(f16v (&acc)[MI][NJ], uint8_t *lds, con
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land after the workgroup's LDS is released
 }
 
+// STREAM: past L2, for the largest tiles, whose workgroups all store at their common end ([2048, 4096] x [4096, 8192]
+// 116 -> 109 us; the smaller tiles' outputs are left where the next kernel finds them)
+template <bool STREAM, class T>
+__device__ __forceinline__ void store_chunk(T *p, u32x4 v) {
+    if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p));
+    else *reinterpret_cast<u32x4 *>(p) = v;
+}
+
 // The same outputs in 128-bit stores (n a multiple of 8, Y on a 16-byte boundary): a wavefront's blocks pass through
 // 2 KiB MI NJ of LDS of its own, a row of them in 64 NJ bytes.
-template <class T, int MI, int NJ>
+template <class T, int MI, int NJ, bool STREAM>
 __device__ __forceinline__ void store_rows(const f16v (&acc)[MI][NJ], uint8_t *stage, T *__restrict__ y, const Bias &bias, uint64_t ym,
                                            uint32_t row0, uint32_t col0, uint32_t m, uint32_t n, float alpha, float beta) {
     const uint32_t lane = threadIdx.x & 63, l32 = lane & 31, kh = lane >> 5;
@@ -688,7 +696,7 @@ __device__ __forceinline__ void store_rows(const f16v (&acc)[MI][NJ], uint8_t *s
         const uint32_t idx = lane + 64 * it, row = idx / (4 * NJ), chunk = idx % (4 * NJ);
         const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + at(row, 16 * chunk));
         if (row0 + row < m && col0 + 8 * chunk < n)
-            *reinterpret_cast<u32x4 *>(y + (ym * m + row0 + row) * n + col0 + 8 * chunk) = v;
+            store_chunk<STREAM>(y + (ym * m + row0 + row) * n + col0 + 8 * chunk, v);
     }
 }
 
@@ -719,7 +727,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void mm_ring(T *__restri
     const uint32_t wave_row = row0 + (wave / WN) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
     if (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0) {
         __syncthreads();  // every wavefront has read its last fragments
-        store_rows<T, MI, NJ>(acc, lds + wave * (32 * MI * 64 * NJ), y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
+        store_rows<T, MI, NJ, R::TM * R::TN >= 65536>(acc, lds + wave * (32 * MI * 64 * NJ), y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
     } else {
         store_blocks<T, MI, NJ>(acc, y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
     }
@@ -733,7 +741,7 @@ struct RingShape {
     double fixed, alone, full;
 };
 constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 180, 260},  {64, 128, 3, 235, 405},  {128, 128, 4.5, 300, 560},
-                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 11, 1000, 1660}};
+                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 10, 1000, 1560}};
 constexpr int kRingShapeCount = 6;
 constexpr uint32_t kCus = 256;
 
