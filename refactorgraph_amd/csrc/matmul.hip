@@ -1783,16 +1783,16 @@ inline KnSplitPlan kn_split_plan(size_t k, size_t n, uint32_t rows_padded) {
 // the products 1.2, and 3.0 for everything behind them.
 constexpr int KM_COLS = 64;       // columns of a strip (128 bytes of a k-row)
 constexpr int KM_ROWB = 128;      // bytes of a k-row of the strip in LDS
-constexpr int KM_MAX_KR = 1024;   // k-rows of a share: 128 KiB of LDS
+constexpr int KM_MAX_KR = 1024;   // k-rows of a share: 128 KiB of LDS, or half of that with two workgroups on a CU
 constexpr int KM_PART = 2048;     // floats a workgroup leaves: 32 rows of A x 64 columns
-template <class T>
+template <class T, int MAX_KR>
 __global__ __launch_bounds__(256) void mm_kn_mfma_split(T *__restrict__ y, const T *__restrict__ a, const T *__restrict__ b, Bias bias,
                                                        uint32_t m, uint32_t k, uint32_t n, float alpha, float beta, uint32_t kr,
                                                        uint32_t shares, float *__restrict__ part, unsigned long long *__restrict__ sync,
                                                        unsigned long long launch_no) {
-    // kr: k-rows per share, a multiple of 256, at most KM_MAX_KR; k a multiple of 8, n of 64
+    // kr: k-rows per share, a multiple of 256, at most MAX_KR; k a multiple of 8, n of 64
     // sync: one arrival counter per strip, then one flag per strip and share
-    __shared__ __align__(1024) uint8_t lds[KM_MAX_KR * KM_ROWB];
+    __shared__ __align__(1024) uint8_t lds[MAX_KR * KM_ROWB];
     const uint32_t tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t strip = blockIdx.x, share = blockIdx.y;
@@ -1802,7 +1802,7 @@ __global__ __launch_bounds__(256) void mm_kn_mfma_split(T *__restrict__ y, const
 
     // the operand from A first: row l32 (rows beyond m repeat the last one, their results are not stored), k-rows
     // row0 + 16 ks + 8 half .. + 7; beyond the share's last k-row the operand is zero
-    constexpr int MAX_STEPS = KM_MAX_KR / 4 / 16;
+    constexpr int MAX_STEPS = MAX_KR / 4 / 16;
     u32x4 af[MAX_STEPS];
     {
         const T *arow = a + static_cast<uint64_t>(l32 < m ? l32 : m - 1) * k + k0;
@@ -1947,6 +1947,13 @@ inline KnSplitPlan kn_mfma_split_plan(size_t k, size_t n) {
     kr = (kr + 255) / 256 * 256;  // a wavefront's quarter in groups of four k-steps
     if (kr > KM_MAX_KR) kr = KM_MAX_KR;
     p.shares = static_cast<uint32_t>((k + kr - 1) / kr);
+    // More workgroups than CUs: halves of the shares, two of which a CU holds, one multiplying and handing its sums over
+    // while the other's copies arrive ([16, 4096] x [4096, 6144] 21.4 -> 19.2 us, 11008 columns 32.1 -> 29.7; where one round
+    // of whole shares suffices halves only add sums to be exchanged, 4096 columns 13.1 -> 14.2)
+    if (p.strips * p.shares > static_cast<uint32_t>(cus) && kr > KM_MAX_KR / 2 && p.shares <= 127) {
+        kr = KM_MAX_KR / 2;
+        p.shares = static_cast<uint32_t>((k + kr - 1) / kr);
+    }
     p.kr = kr;
     p.ticket_bytes = (static_cast<size_t>(p.strips) * (p.shares + 1) * 8 + 255) / 256 * 256;  // a counter per strip, a flag per share
     p.bytes = p.ticket_bytes + static_cast<size_t>(p.strips) * p.shares * KM_PART * sizeof(float);
@@ -1972,8 +1979,11 @@ int launch_kn_mfma_split(T *y, const T *a, const T *b, Bias bias, uint32_t m, ui
     if constexpr (sizeof(T) == 2) {
         auto *sync = static_cast<unsigned long long *>(workspace);
         float *part = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + plan.ticket_bytes);
-        mm_kn_mfma_split<T><<<dim3(plan.strips, plan.shares, 1), 256, 0, s>>>(y, a, b, bias, m, k, n, alpha, beta, plan.kr, plan.shares,
-                                                                                part, sync, next_launch_number());
+        const dim3 grid(plan.strips, plan.shares, 1);
+        if (plan.kr <= KM_MAX_KR / 2)
+            mm_kn_mfma_split<T, KM_MAX_KR / 2><<<grid, 256, 0, s>>>(y, a, b, bias, m, k, n, alpha, beta, plan.kr, plan.shares, part, sync, next_launch_number());
+        else
+            mm_kn_mfma_split<T, KM_MAX_KR><<<grid, 256, 0, s>>>(y, a, b, bias, m, k, n, alpha, beta, plan.kr, plan.shares, part, sync, next_launch_number());
         return launch_status();
     } else {
         return RG_HIP_E_UNSUPPORTED;
