@@ -24,6 +24,7 @@ namespace {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kMaxDims = 8;
 constexpr int UNROLL = 4;  // words a thread has in flight
+constexpr uint64_t kFewTiles = 1024;
 constexpr uint32_t TILE_H = 8, TILE_S = 8;   // blocks of a tile along the two dimensions that change places
 
 struct Divisor {
@@ -119,7 +120,8 @@ struct TilePlan {
     Divisor tiles_per_outer;
 };
 
-template <class Word>
+// U: words a thread has in flight; the workgroups along y share a tile.
+template <class Word, int U>
 __global__ __launch_bounds__(256) void transpose_tiles(Word *__restrict__ y, const Word *__restrict__ x, const TilePlan t) {
     const Plan &p = t.plan;
     const uint32_t wpb = p.words_per_block.d;
@@ -135,11 +137,11 @@ __global__ __launch_bounds__(256) void transpose_tiles(Word *__restrict__ y, con
         rem -= q * p.stride_o[d].d;
     }
     const uint32_t words = TILE_H * TILE_S * wpb;  // of the tile
-    for (uint32_t w0 = 0; w0 < words; w0 += 256 * UNROLL) {
-        Word v[UNROLL];
-        uint32_t row[UNROLL], col[UNROLL];
+    for (uint32_t w0 = blockIdx.y * (256 * U); w0 < words; w0 += gridDim.y * (256 * U)) {
+        Word v[U];
+        uint32_t row[U], col[U];
 #pragma unroll
-        for (int j = 0; j < UNROLL; ++j) {
+        for (int j = 0; j < U; ++j) {
             const uint32_t w = w0 + j * 256 + threadIdx.x;
             row[j] = p.words_per_block.div(w);  // TILE_H ss + hh: neighbouring rows are neighbouring input blocks
             col[j] = w - row[j] * wpb;
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(256) void transpose_tiles(Word *__restrict__ y, con
             }
         }
 #pragma unroll
-        for (int j = 0; j < UNROLL; ++j) {
+        for (int j = 0; j < U; ++j) {
             const uint32_t w = w0 + j * 256 + threadIdx.x;
             if (w < words) {
                 const uint32_t hh = row[j] % TILE_H, ss = row[j] / TILE_H;
@@ -351,8 +353,12 @@ int launch(void *y, const void *x, const Plan &p, const uint32_t *stride_i, cons
             t.tiles_per_outer = make_divisor((extent_h / TILE_H) * (extent_s / TILE_S));
             const uint64_t tiles = block_count / (TILE_H * TILE_S);
             if (tiles <= 0x7fffffffull) {
-                transpose_tiles<Word><<<static_cast<unsigned>(tiles), 256, 0, s>>>(static_cast<Word *>(y),
-                                                                                  static_cast<const Word *>(x), t);
+// few tiles: four workgroups each, a word per thread (8 kv heads x 1000 tokens of 256 bytes, 125 tiles: 5.0 -> 4.0 us,
+                // 32 heads 6.6 -> 5.4 us)
+                if (tiles < kFewTiles)
+                    transpose_tiles<Word, 1><<<dim3(static_cast<unsigned>(tiles), 4), 256, 0, s>>>(static_cast<Word *>(y), static_cast<const Word *>(x), t);
+                else
+                    transpose_tiles<Word, UNROLL><<<static_cast<unsigned>(tiles), 256, 0, s>>>(static_cast<Word *>(y), static_cast<const Word *>(x), t);
                 return launch_status();
             }
         }
