@@ -1583,6 +1583,15 @@ def test_matmul_ring_tiles_exact_on_small_integers(m, k, n, tb):
             assert torch.equal(y, ref.to(dt)), (n_, dt, None if c is None else tuple(c.shape))
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 64, 17), (3, 128, 9), (5, 320, 1), (12, 832, 2680), (14, 3520, 583), (32, 192, 31), (33, 576, 121)])
+def test_matmul_f32_few_rows_any_column_count(m, k, n):
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a, b, c = (torch.randint(-8, 9, s, generator=g, device="cuda").float() for s in ((m, k), (n, k), (n,)))
+    exact = a.double() @ b.double().t().contiguous()  # sums of small integers: exact in float in any order
+    assert torch.equal(ops.matmul(a, b, trans_b=True).double(), exact)
+    assert torch.equal(ops.matmul(a, b, c, trans_b=True).double(), exact + c.double())
+
+
 def test_matmul_ring_tiles_bias_in_place_and_batch():
     g = torch.Generator(device="cuda").manual_seed(5)
     rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda")
