@@ -1604,6 +1604,42 @@ def test_matmul_ring_tiles_bias_in_place_and_batch():
     assert torch.equal(ops.matmul(a.half(), b.half()), ref)
 
 
+@pytest.mark.parametrize("n", [1033, 1030])
+def test_matmul_ring_tiles_bias_in_place_columns_no_multiple_of_8(n):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda")
+    a, b, y = rand(700, 320), rand(n, 320), rand(700, n).half()
+    ref = (a.double() @ b.double().t().contiguous() + y.double()).half()
+    ops.matmul(a.half(), b.half(), y, trans_b=True, out=y)
+    assert torch.equal(y, ref)
+
+
+def fastest_us(call, reps=10):
+    """Least time of a call among others, for kernels that take longer than a call's host work."""
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    call()
+    best = math.inf
+    for _ in range(6):
+        a.record()
+        for _ in range(reps):
+            call()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) / reps * 1e3)
+    return best
+
+
+def test_matmul_bias_per_output_is_not_a_load_at_a_time():
+    # 64 products [300,128] x [1001,128]^T: the bias values of a block requested together cost 1.2 times the product
+    # without a bias, one dependent load per output 2.6 times
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda").half()
+    a, w, c, y = rand(64, 300, 128), rand(64, 1001, 128), rand(300, 1001), rand(64, 300, 1001)
+    none = fastest_us(lambda: ops.matmul(a, w, None, trans_b=True, out=y))
+    bias = fastest_us(lambda: ops.matmul(a, w, c, trans_b=True, out=y))
+    assert bias < 1.9 * none, (none, bias)
+
+
 def test_matmul_fp16_exact_on_small_integers_full_tile_grid():
     # integer-valued operands with |sum| < 2048: every fp16 result is exact, so the MFMA path must
     # reproduce numpy's integer product bit for bit over a 3 x 2 grid of tiles and 5 k-tiles
