@@ -780,6 +780,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK > 4 ? 2 : 1) void m
         za_f[i] = splat(zp_byte(za, am * m + (row < m ? row : m - 1)));
     }
     const uint32_t zb_f = splat(zp_byte(zb, 0));  // (none or a scalar)
+    // the scales ahead of the copies: a load behind the epilogue's stores waits for those too, column block by column block
+    // (128 products [200, 128] x [128, 1024] 51.2 -> 40.4 us, 32.1 with integer outputs)
+    float scale[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const uint32_t col = wave_col + 32 * j + (lane & 31);
+        scale[j] = DEQ ? dq.scale[dq.per_column ? (col < n ? col : n - 1) : 0] : 0.f;
+    }
     v16i acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -806,13 +814,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK > 4 ? 2 : 1) void m
     for (int j = 0; j < NJ; ++j) {
         const uint32_t col = wave_col + 32 * j + (lane & 31);
         if (col >= n) continue;
-        const float scale = DEQ ? dq.scale[dq.per_column ? col : 0] : 0.f;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const uint32_t row = wave_row + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
-                if (row < m) y[(ym * m + row) * n + col] = finish<DEQ>(acc[i][j][e], scale);
+                if (row < m) y[(ym * m + row) * n + col] = finish<DEQ>(acc[i][j][e], scale[j]);
             }
     }
 }

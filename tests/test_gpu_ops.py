@@ -1640,6 +1640,20 @@ def test_matmul_bias_per_output_is_not_a_load_at_a_time():
     assert bias < 1.9 * none, (none, bias)
 
 
+def test_matmul_integer_scales_are_not_waited_for_behind_stores():
+    # 128 products [200,128] x [128,1024]: the dequantising epilogue costs 1.25 times the integer one with the scales
+    # requested ahead of the tiles, 1.6 times with a load per column block behind the previous block's stores
+    g = torch.Generator(device="cuda").manual_seed(11)
+    a = torch.randint(0, 256, (128, 200, 128), generator=g, device="cuda", dtype=torch.uint8)
+    b = torch.randint(-128, 128, (128, 128, 1024), generator=g, device="cuda", dtype=torch.int8)
+    z, s = torch.full((1,), 100, device="cuda", dtype=torch.uint8), torch.rand(1024, generator=g, device="cuda")
+    yi, yf = (torch.empty(128, 200, 1024, device="cuda", dtype=t) for t in (torch.int32, torch.float32))
+    whole = fastest_us(lambda: ops.matmul_integer(a, b, z, out=yi))
+    scaled = fastest_us(lambda: ops.matmul_integer(a, b, z, out=yf, dequant_scale=s))
+    assert torch.equal(yf, yi.float() * s)
+    assert scaled < 1.42 * whole, (whole, scaled)
+
+
 def test_matmul_fp16_exact_on_small_integers_full_tile_grid():
     # integer-valued operands with |sum| < 2048: every fp16 result is exact, so the MFMA path must
     # reproduce numpy's integer product bit for bit over a 3 x 2 grid of tiles and 5 k-tiles
