@@ -45,6 +45,18 @@ def test_error_strings_and_workspace_queries_need_no_gpu():
     assert L.rg_hip_attention_kvcache_workspace(32, 32, 8, 1, 4096, 128) > 0
 
 
+@pytest.mark.parametrize("m,k,n,shares", [
+    (8, 760, 20480, 1), (16, 1024, 128000, 1), (32, 1024, 32000, 1),      # a share is all of k: nothing to exchange
+    (16, 4096, 4096, 4),                                                  # whole shares fill one round of CUs
+    (16, 4096, 6144, 8), (16, 4096, 11008, 8), (5, 1536, 32000, 3)])      # more workgroups than CUs: half shares
+def test_matmul_workspace_holds_the_shares_of_k_the_launch_takes(m, k, n, shares):
+    """Five to 32 rows of FP16 / BF16 against [k, n] weights: a counter and a flag per share of every strip of 64 columns,
+    then 32 x 64 floats per share and strip (256 CUs, which is also what the query assumes without a device)."""
+    strips = n // 64
+    tickets = (strips * (shares + 1) * 8 + 255) // 256 * 256
+    assert abi.lib().rg_hip_matmul_workspace(abi.FP16, 0, 0, 1, m, k, n) == tickets + strips * shares * 8192
+
+
 def test_product_package_does_not_touch_the_oracle():
     pkg = os.path.join(ROOT, "refactorgraph_amd")
     for dirpath, _, files in os.walk(pkg):
