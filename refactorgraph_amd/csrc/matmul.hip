@@ -24,6 +24,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "product_plan.hpp"
 #include "split_handoff.hpp"
 
 namespace rg {
@@ -2141,26 +2142,17 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
         return rows_kn ? tile_us < rows_kn_us : !gemv_kn || (m > 4 && tile_us < gemv_kn_us);
     };
 
-    // F32 on the matrix cores.  A launch of the 128 x 128 tiles walks all of k in every workgroup and takes about
-    // 300 us at k = 4096 however few tiles there are; up to that cost few rows go through the block products of
-    // mm_rows / mm_rows_kn (one k per block and instruction; no transposition needed for B as [k, n], an operand
-    // being one float), 32 rows a pass: 27 us (B as [n, k]) and 33 us (as [k, n]) per pass and 4096 columns.
+    // F32 on the matrix cores: the block products of mm_rows / mm_rows_kn (one k per block and instruction; no transposition
+    // needed for B as [k, n], an operand being one float), 32 rows a pass, 128 x 128 tiles, or the plain kernel.
     constexpr bool is_f32 = std::is_same<T, float>::value;
     const bool f32_tiles_ok = is_f32 && !trans_a && k % FK == 0 && k > 0 && aligned16(a) && aligned16(b) &&
                               (trans_b || (n % 4 == 0 && n >= 4));
     // (any n: [12, 8320] x [2680, 8320]^T, n no multiple of 16, took 613 us on the tiles and 32 us here)
-    const bool rows_f32_ok = is_f32 && !trans_a && trans_b && k % 64 == 0 && k > 0 && k < (1u << 25) &&
-                             aligned16(a) && aligned16(b);
-    const bool rows_kn_f32_ok = is_f32 && !trans_a && !trans_b && n % 16 == 0 && k % 128 == 0 && k > 0 &&
-                                static_cast<uint64_t>(k) * n < (1ull << 30) && k < (1u << 25) && aligned16(a) && aligned16(b);
-    // (microseconds, from those figures, with 3 us for a launch; 768 tiles run side by side)
-    const double kn4096 = static_cast<double>(n) / 4096 * static_cast<double>(k) / 4096;
-    const double f32_tile_rounds = static_cast<double>((((m + FT - 1) / FT) * ((n + FT - 1) / FT) + 767) / 768);
-    const double f32_cost_tiles = f32_tiles_ok ? 3.0 + 300.0 * static_cast<double>(k) / 4096 * f32_tile_rounds : 1e30;
-    const double f32_passes = static_cast<double>((m + 31) / 32);
-    const bool rows_f32 = rows_f32_ok && f32_passes * (3.0 + 27.0 * kn4096) <= f32_cost_tiles;
-    const bool rows_kn_f32 = rows_kn_f32_ok && f32_passes * (3.0 + 33.0 * kn4096) <= f32_cost_tiles;
-    const bool f32_tiles = f32_tiles_ok && m > 8;
+    const bool rows_f32_ok = is_f32 && !trans_a && k > 0 && k < (1u << 25) && aligned16(a) && aligned16(b) &&
+                             (trans_b ? k % 64 == 0 : n % 16 == 0 && k % 128 == 0 && static_cast<uint64_t>(k) * n < (1ull << 30));
+    const F32Route f32 = is_f32 ? f32_route(m, k, n, side_by_side, trans_b, rows_f32_ok, f32_tiles_ok) : F32Route::plain;
+    const bool rows_f32 = f32 == F32Route::rows && trans_b, rows_kn_f32 = f32 == F32Route::rows && !trans_b;
+    const bool f32_tiles = f32 == F32Route::tiles;
 
     auto launch_tiles16 = [&](uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
         if constexpr (narrow) {

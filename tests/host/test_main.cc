@@ -38,6 +38,7 @@
 #include "rg_mirror/executor.h"
 #include "rg_mirror/hip_kernels.h"
 #include "oracle.h"
+#include "../../refactorgraph_amd/csrc/product_plan.hpp"
 
 #include <chrono>
 #include <cmath>
@@ -107,6 +108,36 @@ static void broadcasterKnownAnswer() {
     same.locate(4, ans.data());
     EXPECT(ans[0] == 4 && ans[1] == 4);
     EXPECT(throws<std::runtime_error>([] { Broadcaster bad({{2, 3}, {4, 3}}); }));
+}
+
+static void productPlanF32() {
+    // which kernel a float product takes; the times beside the sizes are the measured ones, in that order
+    using R = rg::F32Route;
+    auto nk = [](size_t m, size_t k, size_t n) { return rg::f32_route(m, k, n, 1, true, true, true); };
+    auto kn = [](size_t m, size_t k, size_t n) { return rg::f32_route(m, k, n, 1, false, true, true); };
+    // up to eight rows against a vocabulary: never the plain kernel because of tiles that are not launched
+    EXPECT(nk(8, 4096, 50257) == R::rows);  // rows 151, tiles 536, plain 545
+    EXPECT(nk(1, 2048, 50257) == R::rows);  // 63, 285, 280
+    EXPECT(nk(4, 1024, 151936) == R::rows);
+    EXPECT(nk(8, 512, 65536) == R::rows);
+    EXPECT(kn(8, 2048, 32000) == R::rows);  // 75
+    // more rows: tiles in rounds of 256
+    EXPECT(nk(9, 2048, 50257) == R::rows);  // 91, 284
+    EXPECT(nk(12, 4096, 50257) == R::rows); // 183, 533
+    EXPECT(nk(12, 8320, 2680) == R::rows);  // 32, 613
+    EXPECT(nk(64, 128, 4096) == R::rows);   // 8.8, 14.7
+    EXPECT(nk(256, 4096, 4096) == R::rows); // 232, 307
+    EXPECT(kn(128, 512, 4096) == R::rows);  // 28, 43
+    EXPECT(nk(64, 64, 5833) == R::tiles);   // 14.4, 9.9
+    EXPECT(nk(128, 512, 5833) == R::tiles); // 49.2, 43.5
+    EXPECT(nk(128, 1024, 50257) == R::tiles);// 477, 146
+    EXPECT(kn(17, 128, 32000) == R::tiles); // 34.8, 14.4
+    // a k so short that a pass is all overhead; operands that a kernel does not take
+    EXPECT(nk(8, 64, 32000) == R::plain);   // 10.9, (8.5), 7.0
+    EXPECT(rg::f32_route(8, 4096, 4096, 1, false, false, true) == R::plain);
+    EXPECT(rg::f32_route(9, 4096, 4096, 1, false, false, true) == R::tiles);
+    EXPECT(rg::f32_route(9, 4096, 4096, 1, true, true, false) == R::rows);
+    EXPECT(rg::f32_route(300, 100, 100, 1, true, false, false) == R::plain);
 }
 
 static void shapeDigests() {
@@ -2087,6 +2118,7 @@ int main(int argc, char **argv) {
     std::string only = argc > 2 ? argv[2] : "";
     RUN(broadcasterKnownAnswer);
     RUN(shapeDigests);
+    RUN(productPlanF32);
     RUN(memPoolBestFit);
     RUN(resourcesAndErrors);
     RUN(collectorsSelectOrDecline);

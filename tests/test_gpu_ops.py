@@ -1592,6 +1592,18 @@ def test_matmul_f32_few_rows_any_column_count(m, k, n):
     assert torch.equal(ops.matmul(a, b, c, trans_b=True).double(), exact + c.double())
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 128, 50257), (8, 192, 50257), (4, 256, 40001), (8, 64, 32000), (9, 64, 50257), (33, 128, 16385), (64, 64, 5833)])
+def test_matmul_f32_few_rows_against_a_vocabulary(m, k, n):
+    """Wide weights on either side of the choice between the passes, the tiles and the plain kernel."""
+    g = torch.Generator(device="cuda").manual_seed(m * k + n)
+    a, b, c = (torch.randint(-8, 9, s, generator=g, device="cuda").float() for s in ((m, k), (n, k), (n,)))
+    exact = a.double() @ b.double().t().contiguous()  # sums of small integers: exact in float in any order
+    assert torch.equal(ops.matmul(a, b, trans_b=True).double(), exact)
+    assert torch.equal(ops.matmul(a, b, c, trans_b=True).double(), exact + c.double())
+    if n % 16 == 0:
+        assert torch.equal(ops.matmul(a, b.t().contiguous()).double(), exact)
+
+
 def test_matmul_ring_tiles_bias_in_place_and_batch():
     g = torch.Generator(device="cuda").manual_seed(5)
     rand = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda")
