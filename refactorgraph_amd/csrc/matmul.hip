@@ -12,9 +12,9 @@
 // straight into a ring of LDS stages; a cost model picks the shape, or two of them for one product.
 // Few rows of A with the weights as [n, k] (a decode step) are bound by reading the weights once: one row goes
 // through a matrix-vector kernel on the vector ALUs, 2 to 16 rows through 4x4x4 block products whose operands
-// come straight from global memory, up to 255 rows through 32x32x16 products with the tiles passed through LDS.
-// With the weights as [k, n] the block products sit behind a transposition in registers (32 rows a pass).  Where
-// those passes would take longer than the tiles, fewer than 256 rows go to the tiles too.
+// come straight from global memory, up to 32 rows through 32x32x16 products with the tiles passed through LDS.
+// With the weights as [k, n] the block products sit behind a transposition in registers.  Where the tiles are
+// expected to end earlier, these rows go there too (product_plan.hpp holds the costs and the choice).
 // F32 (A not transposed) has 128 x 128 tiles of 32x32x2 products and the block-product kernels for few rows.
 // Everything else (F64, transposed A, other shapes) goes through a plain tiled kernel.
 #include <hip/hip_bf16.h>
@@ -235,8 +235,6 @@ template <> struct Mfma<__hip_bfloat16> {
 // elements come from five aligned words.
 constexpr int HT = 128, HK = 64, HP = 72, HF = 3;
 constexpr size_t kHalfTiles = 128;   // tiles of 128 rows up to which tiles of 64 rows are launched instead
-constexpr size_t kSmallGrid = 384;  // workgroups up to which these tiles are weighed against the few-rows kernels
-constexpr size_t kFewRows = 256;     // rows of A below which those kernels are considered
 
 // Stores the MI x NJ blocks of 32 x 32 accumulators of a wavefront, whose first output is (row0, col0) of matrix ym.
 template <class T, int MI, int NJ>
@@ -746,71 +744,16 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void mm_ring(T *__restri
     }
 }
 
-// The tile shapes and what a launch of them takes: `fixed` us a round of 256 workgroups (a CU holds one), and per 64 of
-// k `alone` ns while few CUs have a tile, `full` ns while all have one (they then share what L2 and the memory-side cache
-// deliver, 30 to 40 % of the time of every shape).  Measured at k = 512 to 4096, FP16 and BF16, both layouts of B.
-struct RingShape {
-    uint32_t rows, cols;
-    double fixed, alone, full;
-};
-constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 180, 260},  {64, 128, 3, 235, 405},  {128, 128, 4.5, 300, 560},
-                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 10, 1000, 1560}};
-constexpr int kRingShapeCount = 6;
-constexpr uint32_t kCus = 256;
-
-struct RingPlan {
-    int first, rest;   // shape of the first `columns` columns and of those behind them
-    uint32_t columns;  // 0: all on `rest`
-    double us;
-};
-
-inline double ring_us(const RingShape &t, double tiles, double steps) {
-    const double rounds = static_cast<double>(static_cast<uint64_t>(tiles / kCus)), left = tiles / kCus - rounds;
-    return rounds * (t.fixed + 1e-3 * steps * t.full) + (left > 0 ? t.fixed + 1e-3 * steps * (t.alone + (t.full - t.alone) * left) : 0);
-}
-
-// One shape for the whole product, or whole rounds of one shape and another one for the columns that are left: 344 tiles of
-// 256 x 256 ([2048, 4096] x [4096, 11008]) would be a full round and one with two thirds of the CUs idle (208 us); a full
-// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.
-inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t batch) {
-    RingPlan best{0, 0, 0, 1e30};
-    const double steps = static_cast<double>(k / 64);
-    auto single = [&](size_t columns) {
-        std::pair<int, double> one{0, 1e30};
-        for (int i = 0; i < kRingShapeCount; ++i) {
-            const RingShape &t = kRingShapes[i];
-            const double us = ring_us(t, static_cast<double>((m + t.rows - 1) / t.rows) * static_cast<double>((columns + t.cols - 1) / t.cols) *
-                                             static_cast<double>(batch), steps);
-            if (us < one.second) one = {i, us};
-        }
-        return one;
-    };
-    const auto whole = single(n);
-    best.rest = whole.first;
-    best.us = whole.second;
-    if (batch != 1) return best;
-    for (int i = 0; i < kRingShapeCount; ++i) {
-        const RingShape &t = kRingShapes[i];
-        const size_t row_tiles = (m + t.rows - 1) / t.rows, tiles = row_tiles * (n / t.cols);
-        const size_t wide = tiles / kCus * kCus / row_tiles;  // columns of tiles in whole rounds
-        if (wide == 0 || wide * t.cols >= n) continue;
-        const auto rest = single(n - wide * t.cols);
-        const double us = ring_us(t, static_cast<double>(row_tiles * wide), steps) + rest.second;
-        if (us < 0.97 * best.us) best = {i, rest.first, static_cast<uint32_t>(wide * t.cols), us};
-    }
-    return best;
-}
-
 // ---------------------------------------------------------------- few rows of A (decode): weight streaming
 //
-// Y[m, n] = alpha * A[m, k] @ W[n, k]^T (+ bias) for m <= 32 SLABS, FP16 / BF16: bound by reading W once
+// Y[m, n] = alpha * A[m, k] @ W[n, k]^T (+ bias) for m <= 32, FP16 / BF16: bound by reading W once
 // from HBM.  A workgroup owns 32 rows of W (32 columns of Y); its four wavefronts each take a
-// quarter of k.  A wavefront loads a 32 x 128 tile of W and the matching tile of A (one per slab of
-// 32 rows) with coalesced 128-bit loads (4 rows of 256 bytes per instruction: longer runs per row
+// quarter of k.  A wavefront loads a 32 x 128 tile of W and the matching tile of A
+// with coalesced 128-bit loads (4 rows of 256 bytes per instruction: longer runs per row
 // serve the DRAM pages better than 128 bytes did) two tiles ahead into registers, passes a tile
-// through its own 8 KiB of LDS (chunk-swizzled rows) to bring it into MFMA operand layout, and
+// through its own 16 KiB of LDS (chunk-swizzled rows) to bring it into MFMA operand layout, and
 // multiplies with v_mfma_f32_32x32x16 (W rows as the first operand, so a lane holds one row of A in
-// the result; with two slabs the W fragments are read once for both).  No barrier in the loop: a wavefront only reads what it wrote itself.  The four
+// the result).  No barrier in the loop: a wavefront only reads what it wrote itself.  The four
 // partial sums meet once at the end.  (Copying the tiles straight into LDS, as the big kernels
 // do, is slower here: that path moves about 24 bytes per clock and CU, a third of what plain
 // loads reach, and this kernel has nothing else to hide behind.)
@@ -818,13 +761,12 @@ constexpr int SK_DEPTH = 2;   // tiles in flight per wavefront
 constexpr int SK_TK = 128;    // k elements per tile (256 bytes per row)
 constexpr int SK_LOADS = 8;   // 128-bit loads per lane and operand tile
 
-template <class T, int SLABS>  // slabs of 32 rows of A that share one pass over W
+template <class T>
 __global__ __launch_bounds__(256) void mm_skinny(T *__restrict__ y, const T *__restrict__ a, const T *__restrict__ w,
-                                                 Bias bias, uint32_t m, uint32_t m_total, uint32_t row_first,
-                                                 uint32_t k, uint32_t n, float alpha, float beta, uint32_t a_matrix0,
-                                                 uint32_t b_matrix0, uint32_t y_matrix0) {
-    constexpr int WAVE_LDS = 8192 * (1 + SLABS);  // the tile of W and one tile of A per slab
-    __shared__ __align__(16) uint8_t lds[4 * WAVE_LDS + 4 * 32 * SLABS * 33 * 4];
+                                                 Bias bias, uint32_t m, uint32_t k, uint32_t n, float alpha, float beta,
+                                                 uint32_t a_matrix0, uint32_t b_matrix0, uint32_t y_matrix0) {
+    constexpr int WAVE_LDS = 16384;  // the tile of W and the tile of A
+    __shared__ __align__(16) uint8_t lds[4 * WAVE_LDS + 4 * 32 * 33 * 4];
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t bz = blockIdx.z;
@@ -832,7 +774,7 @@ __global__ __launch_bounds__(256) void mm_skinny(T *__restrict__ y, const T *__r
     const uint32_t n0 = blockIdx.x * 32;
     const uint64_t pitch = 2ull * k;  // bytes of a row of A or W
     const uint8_t *W = reinterpret_cast<const uint8_t *>(w + (bm * n + n0) * static_cast<uint64_t>(k));
-    const uint8_t *A = reinterpret_cast<const uint8_t *>(a + (am * m_total + row_first) * static_cast<uint64_t>(k));
+    const uint8_t *A = reinterpret_cast<const uint8_t *>(a + am * m * static_cast<uint64_t>(k));
 
     // this wavefront's k-tiles (128 elements = 256 bytes each)
     const uint32_t k_tiles = k / SK_TK;
@@ -843,53 +785,42 @@ __global__ __launch_bounds__(256) void mm_skinny(T *__restrict__ y, const T *__r
     // (their results are not stored)
     const uint32_t ld_row = lane >> 4, ld_chunk = lane & 15;
     const uint8_t *w_src = W + ld_row * pitch + 16 * ld_chunk;
-    uint32_t a_row[SLABS][SK_LOADS];
+    uint32_t a_row[SK_LOADS];
 #pragma unroll
-    for (int sl = 0; sl < SLABS; ++sl)
-#pragma unroll
-        for (int i = 0; i < SK_LOADS; ++i) a_row[sl][i] = 32 * sl + 4 * i + ld_row < m ? 32 * sl + 4 * i + ld_row : m - 1;
+    for (int i = 0; i < SK_LOADS; ++i) a_row[i] = 4 * i + ld_row < m ? 4 * i + ld_row : m - 1;
     struct Tile {
-        u32x4 w[SK_LOADS], a[SLABS][SK_LOADS];
+        u32x4 w[SK_LOADS], a[SK_LOADS];
     };
     auto load = [&](Tile &t, uint32_t kt) {
 #pragma unroll
         for (int i = 0; i < SK_LOADS; ++i)
             t.w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w_src + 4 * i * pitch + kt * 256));
 #pragma unroll
-        for (int sl = 0; sl < SLABS; ++sl)
-#pragma unroll
-            for (int i = 0; i < SK_LOADS; ++i)
-                t.a[sl][i] = *reinterpret_cast<const u32x4 *>(A + a_row[sl][i] * pitch + 16 * ld_chunk + kt * 256);
+        for (int i = 0; i < SK_LOADS; ++i) t.a[i] = *reinterpret_cast<const u32x4 *>(A + a_row[i] * pitch + 16 * ld_chunk + kt * 256);
     };
     // fragment of k-step ks: row lane % 32, chunk 2 ks + lane / 32
     const uint32_t r = lane & 31, h = lane >> 5;
     const uint32_t f_off = r * 256 + 16 * (h ^ (r & 15));
     uint8_t *mine = lds + wave * WAVE_LDS;
 
-    f16v acc0[SLABS], acc1[SLABS];
+    f16v acc0, acc1;
 #pragma unroll
-    for (int sl = 0; sl < SLABS; ++sl)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc0[sl][e] = acc1[sl][e] = 0.f;
+    for (int e = 0; e < 16; ++e) acc0[e] = acc1[e] = 0.f;
     auto multiply = [&](const Tile &t) {
 #pragma unroll
         for (int i = 0; i < SK_LOADS; ++i) {
             const uint32_t row = 4 * i + ld_row, off = row * 256 + 16 * (ld_chunk ^ (row & 15));
             *reinterpret_cast<u32x4 *>(mine + off) = t.w[i];
-#pragma unroll
-            for (int sl = 0; sl < SLABS; ++sl) *reinterpret_cast<u32x4 *>(mine + 8192 * (1 + sl) + off) = t.a[sl][i];
+            *reinterpret_cast<u32x4 *>(mine + 8192 + off) = t.a[i];
         }
 #pragma unroll
         for (int ks = 0; ks < SK_TK / 16; ks += 2) {
             const u32x4 w0 = *reinterpret_cast<const u32x4 *>(mine + (f_off ^ (32 * ks)));
             const u32x4 w1 = *reinterpret_cast<const u32x4 *>(mine + (f_off ^ (32 * (ks + 1))));
-#pragma unroll
-            for (int sl = 0; sl < SLABS; ++sl) {
-                const u32x4 a0 = *reinterpret_cast<const u32x4 *>(mine + 8192 * (1 + sl) + (f_off ^ (32 * ks)));
-                const u32x4 a1 = *reinterpret_cast<const u32x4 *>(mine + 8192 * (1 + sl) + (f_off ^ (32 * (ks + 1))));
-                acc0[sl] = Mfma<T>::run(w0, a0, acc0[sl]);
-                acc1[sl] = Mfma<T>::run(w1, a1, acc1[sl]);
-            }
+            const u32x4 a0 = *reinterpret_cast<const u32x4 *>(mine + 8192 + (f_off ^ (32 * ks)));
+            const u32x4 a1 = *reinterpret_cast<const u32x4 *>(mine + 8192 + (f_off ^ (32 * (ks + 1))));
+            acc0 = Mfma<T>::run(w0, a0, acc0);
+            acc1 = Mfma<T>::run(w1, a1, acc1);
         }
     };
 
@@ -922,25 +853,19 @@ __global__ __launch_bounds__(256) void mm_skinny(T *__restrict__ y, const T *__r
     // partial sums: lane holds row (lane % 32) of A, register e column 8 (e/4) + 4 (lane/32) + e%4 of the block
     float *part = reinterpret_cast<float *>(lds + 4 * WAVE_LDS);  // [wave][row of A][column], pitch 33
 #pragma unroll
-    for (int sl = 0; sl < SLABS; ++sl)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const uint32_t col = 8 * (e / 4) + 4 * h + (e % 4);
-            part[(wave * 32 * SLABS + 32 * sl + r) * 33 + col] = acc0[sl][e] + acc1[sl][e];
-        }
+    for (int e = 0; e < 16; ++e) part[(wave * 32 + r) * 33 + 8 * (e / 4) + 4 * h + (e % 4)] = acc0[e] + acc1[e];
     __syncthreads();
     const T *C = static_cast<const T *>(bias.ptr);
 #pragma unroll
-    for (int q = 0; q < 4 * SLABS; ++q) {
+    for (int q = 0; q < 4; ++q) {
         const uint32_t idx = tid + 256 * q, row = idx / 32, col = idx % 32;
         if (row < m) {
             float v = 0.f;
 #pragma unroll
-            for (int wv = 0; wv < 4; ++wv) v += part[(wv * 32 * SLABS + row) * 33 + col];
+            for (int wv = 0; wv < 4; ++wv) v += part[(wv * 32 + row) * 33 + col];
             v *= alpha;
-            const uint64_t yrow = row_first + row;
-            if (C) v += beta * up(C[ym * bias.sb + yrow * bias.sm + (n0 + col) * bias.sn]);
-            y[(ym * m_total + yrow) * n + n0 + col] = down<T>(v);
+            if (C) v += beta * up(C[ym * bias.sb + row * bias.sm + (n0 + col) * bias.sn]);
+            y[(ym * m + row) * n + n0 + col] = down<T>(v);
         }
     }
 }
@@ -2074,9 +1999,8 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     typedef typename Acc<T>::type A_t;
     const A_t al = through<T>(alpha), be = bias.ptr ? through<T>(beta) : A_t(0);
     constexpr bool narrow = sizeof(T) == 2;
-    // fewer than 256 rows, weights as [n, k]: stream W once per slab of 32 rows of A
-    const bool skinny = narrow && !trans_a && trans_b && m < kFewRows && n % 32 == 0 && k % SK_TK == 0 &&
-                        aligned16(a) && aligned16(b);
+    // up to 32 rows, weights as [n, k]: stream W once
+    const bool skinny = narrow && !trans_a && trans_b && m <= 32 && n % 32 == 0 && k % SK_TK == 0 && aligned16(a) && aligned16(b);
 
     // one row (and up to four where the block-product kernel below does not apply): matrix-vector products on the
     // vector ALUs, A (padded to 1, 2 or 4 rows) in LDS
@@ -2097,50 +2021,19 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
     const bool rows = narrow && !trans_a && trans_b && (m >= 2 || k > 8192 || k <= 2048) && m <= 16 && n % 16 == 0 && k % 128 == 0 &&
                       k > 0 && k < (1u << 26) && aligned16(a) && aligned16(b);
 
-    // fewer than 256 rows, weights as [k, n]: the same block products behind a transposition in registers, 32 rows a
-    // pass (one to four rows against a wide B stay with the matrix-vector kernel, which is a little faster there)
-    const bool rows_kn = narrow && !trans_a && !trans_b && m < kFewRows && !(m <= 4 && n >= 8192) && n % 16 == 0 && k % 128 == 0 &&
+    // up to 32 rows, weights as [k, n]: the same block products behind a transposition in registers (one to four rows
+    // against a wide B stay with the matrix-vector kernel, which is a little faster there)
+    const bool rows_kn = narrow && !trans_a && !trans_b && m <= 32 && !(m <= 4 && n >= 8192) && n % 16 == 0 && k % 128 == 0 &&
                          k > 0 && static_cast<uint64_t>(k) * n < (1ull << 31) && k < (1u << 26) && aligned16(a) && aligned16(b);
 
     // FP16 / BF16 on the tiles, any m: the ring kernel where k is in whole tiles and rows of B as [k, n] start on 16-byte
     // boundaries (its lane offsets, up to 256 rows of A or B or 64 k-rows of B, stay below 2^32), mm_tiles16 for the rest.
-    // Up to 8 rows only where the plain kernel is expected to take longer (it needs 2.9 ns per thousand elements of B,
-    // 596 us for [8, 4096] x [4096, 50257]; a tile launch about 4 us and 0.83 us per 64 of k).
     const size_t side_by_side = a_index || b_index ? 1 : batch;  // matrices that are tiles of one launch
-    const bool tile_operands = narrow && !trans_a && k % 8 == 0 && k > 0 && aligned16(a) && (!trans_b || aligned16(b));
-    const size_t tiles128 = ((m + HT - 1) / HT) * ((n + HT - 1) / HT) * side_by_side;
-    const bool ring_ok = tile_operands && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
-    RingPlan plan{0, 0, 0, 0};
-    auto tiles_plan = [&]() -> const RingPlan & {  // (worked out for the launches that look at it)
-        if (plan.us == 0) plan = ring_plan(m, k, n, side_by_side);
-        return plan;
-    };
-    // (the plain kernel's own chain of steps is 0.54 us per 16 of k: [8, 3648] x [2376, 3648]^T 123 us, 14 on the ring)
-    const bool tiles16_rows = m > 8 || static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k) ||
-                              (ring_ok && !gemv && !rows && !gemv_kn && tiles_plan().us < 0.034 * static_cast<double>(k));
-    const bool tiles16 = tile_operands && tiles16_rows, ring = ring_ok && tiles16_rows;
-    // A short k leaves a tile little to do between fetching its operands and storing its results, and two small tiles
-    // per CU overlap the one's stores with the other's loads: with k <= 128 (k <= 512 below 256 rows) more tiles than CUs
-    // are mm_tiles16's ([8192, 128] x [128, 8192] 76 us, 32 products [128, 128] x [4096, 128]^T 25 us).
-    const bool short_k = tiles16 && m > 16 && n >= 256 && n % 8 == 0 && k % 64 == 0 && aligned16(b) && aligned16(y_) &&
-                         k <= (m < kFewRows ? 512u : 128u) && tiles128 > kCus;
-    // Fewer than 256 rows: the tiles, or the passes of the few-rows kernels where those end earlier (us, from
-    // measurements at k = 4096: mm_skinny 13.5 for 32 and 19 for 64 rows of 4096 columns, 38 for 11008 columns;
-    // mm_rows_kn 22 for 32 rows of 4096 columns; a pass of four rows of mm_gemv_kn 4.3, or B at 5 TB/s).  One to 16 rows
-    // that mm_gemv and mm_rows take read W as [n, k] once at the speed of the memory whatever n is: never a tile.
-    auto tiles_first = [&]() -> bool {
-        if (!tiles16 || m >= kFewRows) return tiles16;
-        if (!ring && tiles128 > kSmallGrid) return false;
-        if (trans_b && (rows || gemv)) return false;
-        const double tile_us = ring ? tiles_plan().us : 4.0 + 0.83 * static_cast<double>((k + HK - 1) / HK);
-        const double columns = static_cast<double>(n * side_by_side), k4096 = static_cast<double>(k) / 4096;
-        const double skinny_us = static_cast<double>((m + 63) / 64) * (3.0 + columns * (m <= 32 ? 2.6e-3 : 3.4e-3) * k4096);
-        const double rows_kn_us = static_cast<double>((m + 31) / 32) * (2.0 + columns * (m <= 16 ? 3.5e-3 : 5.0e-3) * k4096);
-        const double b_us = 2.0 * static_cast<double>(k) * columns / 5.0e6;
-        const double gemv_kn_us = static_cast<double>((m + 3) / 4) * (b_us > 4.3 ? b_us : 4.3);
-        if (trans_b) return !skinny || tile_us < skinny_us;
-        return rows_kn ? tile_us < rows_kn_us : !gemv_kn || (m > 4 && tile_us < gemv_kn_us);
-    };
+    const bool tiles16 = narrow && !trans_a && k % 8 == 0 && k > 0 && aligned16(a) && (!trans_b || aligned16(b));
+    const bool ring = tiles16 && k % 64 == 0 && k < (1u << 22) && aligned16(b) && (trans_b || (n % 8 == 0 && n < (1u << 24)));
+    const bool rough_stores = n % 8 != 0 || !aligned16(y_);
+    const HalfRoute route = narrow ? half_route(m, k, n, side_by_side, trans_b, {ring, tiles16, gemv, rows, skinny, gemv_kn, rows_kn}, rough_stores)
+                                   : HalfRoute::plain;
 
     // F32 on the matrix cores: the block products of mm_rows / mm_rows_kn (one k per block and instruction; no transposition
     // needed for B as [k, n], an operand being one float), 32 rows a pass, 128 x 128 tiles, or the plain kernel.
@@ -2181,8 +2074,7 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
         if constexpr (narrow) {
             const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
             auto part = [&](int shape, uint32_t first, uint32_t columns) -> int {
-                const RingShape &t = kRingShapes[shape];
-                const uint64_t tiles = ((m + t.rows - 1) / t.rows) * static_cast<uint64_t>((columns + t.cols - 1) / t.cols);
+                const uint64_t tiles = tile_count(kRingShapes[shape], m, columns, 1);
                 if (tiles > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
                 const dim3 grid(static_cast<unsigned>(tiles), 1, count);
 #define RG_RING(WM, WN, MI, NJ, NS)                                                                                          \
@@ -2202,7 +2094,7 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
 #undef RG_RING
                 return launch_status();
             };
-            const RingPlan &p = tiles_plan();
+            const RingPlan p = ring_plan(m, k, n, side_by_side, rough_stores);
             if (p.columns) {
                 const int rc = part(p.first, 0, p.columns);
                 if (rc) return rc;
@@ -2236,25 +2128,18 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                                               b + static_cast<uint64_t>(bm0) * k * n, bias, static_cast<uint32_t>(m),
                                               static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, workspace, plan, s);
             }
-            if (short_k) return launch_tiles16(am0, bm0, ym0, count);
-            if (tiles_first()) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
-            if (rows_kn) {
+            if (route == HalfRoute::tiles) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
+            if (route == HalfRoute::rows_kn) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 const bool wide = n % 32 == 0 && n >= 8192;
-                for (uint32_t r0 = 0; r0 < m32; r0 += 32) {
-                    const uint32_t rows = m32 - r0 < 32 ? m32 - r0 : 32;
-                    int e;
-#define RG_ROWS_KN(G, CW) launch_rows_kn<T, G, 8, CW>(y, a, b, bias, rows, m32, r0, k32, n32, al, be, am0, bm0, ym0, count, s)
-                    if (rows <= 4) e = wide ? RG_ROWS_KN(1, 8) : RG_ROWS_KN(1, 4);
-                    else if (rows <= 8) e = wide ? RG_ROWS_KN(2, 8) : RG_ROWS_KN(2, 4);
-                    else if (rows <= 16) e = wide ? RG_ROWS_KN(4, 8) : RG_ROWS_KN(4, 4);
-                    else e = RG_ROWS_KN(8, 4);
+#define RG_ROWS_KN(G, CW) launch_rows_kn<T, G, 8, CW>(y, a, b, bias, m32, m32, 0, k32, n32, al, be, am0, bm0, ym0, count, s)
+                if (m <= 4) return wide ? RG_ROWS_KN(1, 8) : RG_ROWS_KN(1, 4);
+                if (m <= 8) return wide ? RG_ROWS_KN(2, 8) : RG_ROWS_KN(2, 4);
+                if (m <= 16) return wide ? RG_ROWS_KN(4, 8) : RG_ROWS_KN(4, 4);
+                return RG_ROWS_KN(8, 4);
 #undef RG_ROWS_KN
-                    if (e) return e;
-                }
-                return 0;
             }
-            if (rows) {
+            if (route == HalfRoute::rows) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 if (m <= 4 && k > 8192) return launch_rows<T, 1, 16, 2>(y, a, b, bias, m32, m32, 0, k32, n32, al, be, am0, bm0, ym0, count, s);
                 if (m <= 4) return launch_rows<T, 1, 16, 1>(y, a, b, bias, m32, m32, 0, k32, n32, al, be, am0, bm0, ym0, count, s);
@@ -2263,7 +2148,7 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                 if (n / 16 > 384) return launch_rows<T, 4, 4, 3>(y, a, b, bias, m32, m32, 0, k32, n32, al, be, am0, bm0, ym0, count, s);
                 return launch_rows<T, 4, 16, 1>(y, a, b, bias, m32, m32, 0, k32, n32, al, be, am0, bm0, ym0, count, s);
             }
-            if (gemv_kn) {
+            if (route == HalfRoute::gemv_kn) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 for (uint32_t r0 = 0; r0 < m32; r0 += 4) {
                     const uint32_t rows = m32 - r0 < 4 ? m32 - r0 : 4;
@@ -2277,7 +2162,7 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                 }
                 return 0;
             }
-            if (gemv) {
+            if (route == HalfRoute::gemv) {
                 const uint32_t m32 = static_cast<uint32_t>(m), k32 = static_cast<uint32_t>(k), n32 = static_cast<uint32_t>(n);
                 switch (gv_m) {
                     case 1: return launch_gemv<T, 1>(y, a, b, bias, m32, k32, n32, al, be, am0, bm0, ym0, count, s);
@@ -2285,25 +2170,11 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                     default: return launch_gemv<T, 4>(y, a, b, bias, m32, k32, n32, al, be, am0, bm0, ym0, count, s);
                 }
             }
-            if (skinny) {
-                // two slabs of 32 rows share one pass over W
-                for (size_t r0 = 0; r0 < m; r0 += 64) {
-                    const uint32_t rows = static_cast<uint32_t>(m - r0 < 64 ? m - r0 : 64);
-                    const dim3 grid(static_cast<unsigned>(n / 32), 1, count);
-                    if (rows <= 32)
-                        mm_skinny<T, 1><<<grid, 256, 0, s>>>(y, a, b, bias, rows, static_cast<uint32_t>(m), static_cast<uint32_t>(r0),
-                                                             static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                    else
-                        mm_skinny<T, 2><<<grid, 256, 0, s>>>(y, a, b, bias, rows, static_cast<uint32_t>(m), static_cast<uint32_t>(r0),
-                                                             static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
-                    const int rc = launch_status();
-                    if (rc) return rc;
-                }
-                return 0;
+            if (route == HalfRoute::skinny) {
+                mm_skinny<T><<<dim3(static_cast<unsigned>(n / 32), 1, count), 256, 0, s>>>(
+                    y, a, b, bias, static_cast<uint32_t>(m), static_cast<uint32_t>(k), static_cast<uint32_t>(n), al, be, am0, bm0, ym0);
+                return launch_status();
             }
-        }
-        if constexpr (narrow) {
-            if (tiles16) return ring ? launch_ring(am0, bm0, ym0, count) : launch_tiles16(am0, bm0, ym0, count);
         }
         if constexpr (std::is_same<T, float>::value) {
             if (rows_f32) {

@@ -5,8 +5,144 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <utility>
 
 namespace rg {
+
+// ---------------------------------------------------------------- tiles, one workgroup on a CU
+//
+// `fixed` us a round of 256 workgroups, and per step of k `alone` ns while few CUs have a tile, `full` ns while all have one
+// (they then share what the memory side of the CUs delivers); a launch takes kLaunchUs besides.
+struct TileShape {
+    uint32_t rows, cols;
+    double fixed, alone, full;
+};
+constexpr uint32_t kPlanCus = 256;
+
+inline uint64_t tile_count(const TileShape &t, size_t m, size_t n, size_t count) {
+    return static_cast<uint64_t>((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols) * count;
+}
+inline double tiles_us(const TileShape &t, uint64_t tiles, double steps, double extra_fixed = 0) {
+    const double rounds = static_cast<double>(tiles / kPlanCus), left = static_cast<double>(tiles % kPlanCus) / kPlanCus;
+    const double fixed = t.fixed + extra_fixed;
+    return rounds * (fixed + 1e-3 * steps * t.full) + (left > 0 ? fixed + 1e-3 * steps * (t.alone + (t.full - t.alone) * left) : 0);
+}
+
+// ---------------------------------------------------------------- FP16 / BF16
+//
+// Fitted over 5,900 products of 1 to 2048 rows, k 64 to 11008, 64 to 32000 columns, 1 to 256 of them side by side, both
+// layouts of B, with and without a bias.
+
+// mm_ring, steps of 64 k.
+constexpr TileShape kRingShapes[] = {{64, 64, 2.7, 145, 265},  {64, 128, 3, 200, 415},   {128, 128, 4.5, 300, 560},
+                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 10, 1000, 1560}};
+constexpr int kRingShapeCount = 6;
+constexpr double kRingLaunchUs = 1.0;
+// the 256 x 256 tiles store element by element where rows of the output are no whole 16-byte words (16 products
+// [512, 64] x [4099, 64]^T with a bias per output 129 us, 128 x 128 tiles 82); the smaller tiles hide that
+constexpr double kRoughStoresUs = 4.7;
+
+struct RingPlan {
+    int first, rest;   // shape of the first `columns` columns and of those behind them
+    uint32_t columns;  // 0: all on `rest`
+    double us;
+};
+
+// One shape for the whole product, or whole rounds of one shape and another one for the columns that are left: 344 tiles of
+// 256 x 256 ([2048, 4096] x [4096, 11008]) would be a full round and one with two thirds of the CUs idle (208 us); a full
+// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.  Over the sizes above the plan takes 1 % longer
+// than the fastest shape of each product.
+inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t count, bool rough_stores) {
+    RingPlan best{0, 0, 0, 1e30};
+    const double steps = static_cast<double>(k / 64);
+    auto rough = [&](const TileShape &t) { return rough_stores && t.rows == 256 ? kRoughStoresUs : 0.0; };
+    auto single = [&](size_t columns) {
+        std::pair<int, double> one{0, 1e30};
+        for (int i = 0; i < kRingShapeCount; ++i) {
+            const TileShape &t = kRingShapes[i];
+            const double us = tiles_us(t, tile_count(t, m, columns, count), steps, rough(t));
+            if (us < one.second) one = {i, us};
+        }
+        return one;
+    };
+    const auto whole = single(n);
+    best.rest = whole.first;
+    best.us = kRingLaunchUs + whole.second;
+    if (count != 1) return best;
+    for (int i = 0; i < kRingShapeCount; ++i) {
+        const TileShape &t = kRingShapes[i];
+        const size_t row_tiles = (m + t.rows - 1) / t.rows, tiles = row_tiles * (n / t.cols);
+        const size_t wide = tiles / kPlanCus * kPlanCus / row_tiles;  // columns of tiles in whole rounds
+        if (wide == 0 || wide * t.cols >= n) continue;
+        const auto rest = single(n - wide * t.cols);
+        const double us = kRingLaunchUs + tiles_us(t, row_tiles * wide, steps, rough(t)) + rest.second;
+        if (us < 0.97 * best.us) best = {i, rest.first, static_cast<uint32_t>(wide * t.cols), us};
+    }
+    return best;
+}
+
+// Up to 32 rows on the kernels that read the weights once, columns of all products side by side: mm_skinny (B as [n, k]) and
+// a pass of mm_rows_kn (B as [k, n]).  Beyond 32 rows neither ended before the tiles at any size.  Where the choice is
+// between these and the tiles it takes 0.3 % longer than the faster one on average.
+inline double skinny_us(size_t k, size_t columns) {
+    const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
+    return 1.5 + 0.74 * kilo + 0.3 * kilo * wide + 0.21 * wide;
+}
+inline double rows_kn_us(size_t m, size_t k, size_t columns) {
+    const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
+    if (m <= 8) return 0.9 + 1.64 * kilo + 0.32 * kilo * wide + 0.28 * wide;
+    if (m <= 16) return 2.9 + 1.64 * kilo + 0.334 * kilo * wide + 0.15 * wide;
+    return 5.35 + 1.9 * kilo + 0.57 * kilo * wide + 0.135 * wide;
+}
+// A pass of four rows of mm_gemv_kn: a workgroup's chain through k, or B at what 16-byte pieces of its rows come in at.
+inline double gemv_kn_us(size_t m, size_t k, size_t columns) {
+    const double chain = 2.5 + 3.1e-3 * static_cast<double>(k), bytes = 2.0 * static_cast<double>(k) * static_cast<double>(columns) / 1.25e6;
+    return static_cast<double>((m + 3) / 4) * (chain > bytes ? chain : bytes);
+}
+// mm_generic, up to 16 rows.
+inline double plain_us(size_t k, size_t columns) {
+    const double chain = 31e-3 * static_cast<double>(k), work = 2.6e-6 * static_cast<double>(k) * static_cast<double>(columns);
+    return 1.5 + (chain > work ? chain : work);
+}
+// mm_tiles16, steps of 64 k.
+inline double tiles16_us(size_t k) { return 4.0 + 0.83 * static_cast<double>((k + 63) / 64); }
+
+enum class HalfRoute { tiles, rows, rows_kn, gemv, gemv_kn, skinny, plain };
+
+// Which kernels take the operands (alignment, layouts, divisibility), with the row counts each is made for.
+struct HalfKernels {
+    bool ring, tiles16;        // mm_ring; mm_tiles16, which takes what mm_ring takes and more
+    bool gemv, rows, skinny;   // B as [n, k]: up to 4, 2 to 16, up to 32 rows
+    bool gemv_kn, rows_kn;     // B as [k, n]: up to 32 rows each
+};
+
+// `count` products side by side.  One to 16 rows that mm_gemv and mm_rows take read W as [n, k] once: never a tile.
+inline HalfRoute half_route(size_t m, size_t k, size_t n, size_t count, bool b_is_nk, const HalfKernels &can, bool rough_stores) {
+    const bool tiles = can.ring || can.tiles16;
+    if (tiles && m > 32) return HalfRoute::tiles;
+    const size_t columns = n * count;
+    auto ring_us = [&] { return ring_plan(m, k, n, count, rough_stores).us; };
+    if (b_is_nk) {
+        if (can.rows) return HalfRoute::rows;
+        if (can.gemv) return HalfRoute::gemv;
+        if (can.skinny) return can.ring && ring_us() < skinny_us(k, columns) ? HalfRoute::tiles : HalfRoute::skinny;
+    } else {
+        if (can.rows_kn) return can.ring && ring_us() < rows_kn_us(m, k, columns) ? HalfRoute::tiles : HalfRoute::rows_kn;
+        if (can.gemv_kn) {
+            // (a second pass of four rows never ended before the tiles: [5, 4096] x [4096, 1000] 34 us, 14 on mm_ring)
+            if (m <= 4) return HalfRoute::gemv_kn;
+            if (can.ring) return HalfRoute::tiles;
+            const uint64_t tiles128 = static_cast<uint64_t>((n + 127) / 128) * count;  // (mm_tiles16, one launch of few tiles)
+            return can.tiles16 && tiles128 <= 384 && tiles16_us(k) < gemv_kn_us(m, k, columns) ? HalfRoute::tiles : HalfRoute::gemv_kn;
+        }
+    }
+    if (!tiles) return HalfRoute::plain;
+    if (m > 8) return HalfRoute::tiles;
+    // up to eight rows that no few-rows kernel takes ([8, 3648] x [2376, 3648]^T 123 us on the plain kernel, 14 on mm_ring;
+    // 256 products [8, 512] x [1000, 512]^T 303 and 55)
+    if (can.ring) return ring_us() < plain_us(k, columns) ? HalfRoute::tiles : HalfRoute::plain;
+    return static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k) ? HalfRoute::tiles : HalfRoute::plain;
+}
 
 // ---------------------------------------------------------------- F32
 //

@@ -140,6 +140,65 @@ static void productPlanF32() {
     EXPECT(rg::f32_route(300, 100, 100, 1, true, false, false) == R::plain);
 }
 
+static void productPlanHalf() {
+    // which kernel an FP16 / BF16 product takes, operands as mat mul's launcher classifies aligned ones
+    using R = rg::HalfRoute;
+    auto can = [](size_t m, size_t k, size_t n, bool nk) {
+        rg::HalfKernels c{};
+        c.tiles16 = k % 8 == 0;
+        c.ring = k % 64 == 0 && (nk || n % 8 == 0);
+        c.gemv = nk && m <= 4 && k % 8 == 0;
+        c.rows = nk && (m >= 2 || k > 8192 || k <= 2048) && m <= 16 && n % 16 == 0 && k % 128 == 0;
+        c.skinny = nk && m <= 32 && n % 32 == 0 && k % 128 == 0;
+        c.gemv_kn = !nk && m <= 32 && k % 8 == 0 && n % 8 == 0;
+        c.rows_kn = !nk && m <= 32 && !(m <= 4 && n >= 8192) && n % 16 == 0 && k % 128 == 0;
+        return c;
+    };
+    auto nk = [&](size_t count, size_t m, size_t k, size_t n) { return rg::half_route(m, k, n, count, true, can(m, k, n, true), n % 8 != 0); };
+    auto kn = [&](size_t count, size_t m, size_t k, size_t n) { return rg::half_route(m, k, n, count, false, can(m, k, n, false), n % 8 != 0); };
+    // a second pass of four rows over B as [k, n] (measured: the passes, the tiles, us)
+    EXPECT(kn(1, 24, 8192, 520) == R::tiles);   // 176, 24
+    EXPECT(kn(1, 17, 11008, 1000) == R::tiles); // 200, 34
+    EXPECT(kn(1, 5, 4096, 264) == R::tiles);    // 30, 13
+    EXPECT(kn(1, 4, 4096, 264) == R::gemv_kn);
+    EXPECT(kn(1, 5, 1032, 520) == R::gemv_kn);  // 10, 14 (mm_tiles16)
+    EXPECT(kn(1, 24, 2056, 1000) == R::tiles);  // 63, 24 (mm_tiles16)
+    // up to eight rows that no few-rows kernel takes: the plain kernel's work counts, not only its chain
+    EXPECT(nk(256, 5, 512, 1000) == R::tiles);  // 303, 55
+    EXPECT(nk(256, 8, 512, 264) == R::tiles);   // 90, 23
+    EXPECT(nk(64, 5, 256, 1000) == R::tiles);   // 42, 15
+    EXPECT(nk(1, 8, 64, 264) == R::plain);      // 3.7, 3.9
+    EXPECT(nk(1, 8, 3648, 2376) == R::tiles);   // 123, 14
+    // up to 32 rows: the weights once, or the tiles
+    EXPECT(nk(1, 17, 128, 128) == R::skinny);   // 3.0, 3.9
+    EXPECT(nk(32, 24, 512, 128) == R::skinny);  // 4.0, 4.8
+    EXPECT(nk(1, 24, 8192, 64) == R::skinny);   // 14, 23
+    EXPECT(nk(1, 32, 4096, 20000) == R::tiles);
+    EXPECT(kn(1, 8, 4096, 128) == R::rows_kn);  // 5.9, 13
+    EXPECT(kn(1, 16, 8192, 1024) == R::rows_kn);// 14, 23
+    EXPECT(kn(1, 32, 4096, 4096) == R::tiles);  // 18, 14
+    EXPECT(kn(256, 8, 512, 1024) == R::tiles);  // 120, 53
+    EXPECT(nk(1, 16, 4096, 11008) == R::rows && nk(1, 1, 4096, 11008) == R::gemv);
+    // beyond 32 rows always the tiles, with a short k as well
+    EXPECT(nk(1, 33, 4096, 256) == R::tiles);   // mm_skinny 10, 13 at 64 rows 20, 13
+    EXPECT(kn(1, 255, 11008, 128) == R::tiles); // 384, 31
+    EXPECT(nk(32, 128, 128, 4096) == R::tiles && kn(1, 8192, 128, 8192) == R::tiles);
+    // what no matrix kernel takes
+    EXPECT(nk(1, 300, 100, 100) == R::plain && kn(1, 300, 100, 100) == R::plain);
+}
+
+static void productPlanRing() {
+    // shapes of the tiles: {first, rest, columns of first}
+    auto is = [](rg::RingPlan p, int first, int rest, uint32_t columns) {
+        return p.rest == rest && p.columns == columns && (columns == 0 || p.first == first);
+    };
+    EXPECT(is(rg::ring_plan(2048, 4096, 11008, 1, false), 5, 3, 8192)); // 256 x 256, then 128 x 192
+    EXPECT(is(rg::ring_plan(64, 4096, 4096, 1, false), 0, 0, 0));
+    EXPECT(is(rg::ring_plan(4096, 4096, 4096, 1, false), 5, 5, 0));
+    // element-wise stores: the largest tiles give way (16 products [512, 64] x [4099, 64]^T)
+    EXPECT(rg::ring_plan(512, 64, 4096, 16, false).rest == 5 && rg::ring_plan(512, 64, 4099, 16, true).rest < 5);
+}
+
 static void shapeDigests() {
     auto x = Tensor::share(DataType::F32, Shape{2, 3, 4, 5});
     SoftmaxInfo s(*x, 1);
@@ -2119,6 +2178,8 @@ int main(int argc, char **argv) {
     RUN(broadcasterKnownAnswer);
     RUN(shapeDigests);
     RUN(productPlanF32);
+    RUN(productPlanHalf);
+    RUN(productPlanRing);
     RUN(memPoolBestFit);
     RUN(resourcesAndErrors);
     RUN(collectorsSelectOrDecline);
