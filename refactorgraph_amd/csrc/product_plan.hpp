@@ -34,8 +34,8 @@ inline double tiles_us(const TileShape &t, uint64_t tiles, double steps, double 
 // layouts of B, with and without a bias.
 
 // mm_ring, steps of 64 k.
-constexpr TileShape kRingShapes[] = {{64, 64, 2.7, 145, 265},  {64, 128, 3, 200, 415},   {128, 128, 4.5, 300, 560},
-                                     {128, 192, 6, 400, 720}, {128, 256, 8, 490, 875}, {256, 256, 10, 1000, 1560}};
+constexpr TileShape kRingShapes[] = {{64, 64, 2.7, 145, 300},   {64, 128, 3.4, 210, 440},  {128, 128, 4.2, 360, 580},
+                                     {128, 192, 6, 370, 800}, {128, 256, 7.2, 580, 888}, {256, 256, 12.2, 920, 1525}};
 constexpr int kRingShapeCount = 6;
 constexpr double kRingLaunchUs = 1.0;
 // the 256 x 256 tiles store element by element where rows of the output are no whole 16-byte words (16 products
@@ -50,8 +50,8 @@ struct RingPlan {
 
 // One shape for the whole product, or whole rounds of one shape and another one for the columns that are left: 344 tiles of
 // 256 x 256 ([2048, 4096] x [4096, 11008]) would be a full round and one with two thirds of the CUs idle (208 us); a full
-// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.  Over the sizes above the plan takes 1 % longer
-// than the fastest shape of each product.
+// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.  Over the sizes above the plan takes 0.9 %
+// longer than the fastest shape of each product.
 inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t count, bool rough_stores) {
     RingPlan best{0, 0, 0, 1e30};
     const double steps = static_cast<double>(k / 64);
