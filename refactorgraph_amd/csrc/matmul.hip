@@ -640,7 +640,8 @@ __device__ __forceinline__ void ring_loop(f16v (&acc)[MI][NJ], uint8_t *lds, con
 }
 
 // STREAM: past L2, for the largest tiles, whose workgroups all store at their common end ([2048, 4096] x [4096, 8192]
-// 116 -> 109 us; the smaller tiles' outputs are left where the next kernel finds them)
+// 116 -> 109 us; the smaller tiles' outputs are left where the next kernel finds them), where rows are whole 128-byte lines:
+// lines that two workgroups share are written in pieces this way (64 products [512, 64] x [1000, 64]^T 44 us, 35 through L2)
 template <bool STREAM, class T>
 __device__ __forceinline__ void store_chunk(T *p, u32x4 v) {
     if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p));
@@ -649,7 +650,7 @@ __device__ __forceinline__ void store_chunk(T *p, u32x4 v) {
 
 // The same outputs in 128-bit stores (n a multiple of 8, Y on a 16-byte boundary): a wavefront's blocks pass through
 // 2 KiB MI NJ of LDS of its own, a row of them in 64 NJ bytes.
-template <class T, int MI, int NJ, bool STREAM>
+template <bool STREAM, class T, int MI, int NJ>
 __device__ __forceinline__ void store_rows(const f16v (&acc)[MI][NJ], uint8_t *stage, T *__restrict__ y, const Bias &bias, uint64_t ym,
                                            uint32_t row0, uint32_t col0, uint32_t m, uint32_t n, float alpha, float beta) {
     const uint32_t lane = threadIdx.x & 63, l32 = lane & 31, kh = lane >> 5;
@@ -738,7 +739,10 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void mm_ring(T *__restri
     const uint32_t wave_row = row0 + (wave / WN) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
     if (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0) {
         __syncthreads();  // every wavefront has read its last fragments
-        store_rows<T, MI, NJ, R::TM * R::TN >= 65536>(acc, lds + wave * (32 * MI * 64 * NJ), y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
+        uint8_t *stage = lds + wave * (32 * MI * 64 * NJ);
+        // (two calls, not a flag: stores that differ in the hint alone are merged into one without it)
+        if (R::TM * R::TN >= 65536 && n % 64 == 0) store_rows<true, T, MI, NJ>(acc, stage, y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
+        else store_rows<false, T, MI, NJ>(acc, stage, y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
     } else {
         store_blocks<T, MI, NJ>(acc, y, bias, ym, wave_row, wave_col, m, n, alpha, beta);
     }
