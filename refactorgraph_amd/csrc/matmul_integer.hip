@@ -15,6 +15,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "product_plan.hpp"
 
 namespace rg {
 namespace {
@@ -851,7 +852,6 @@ constexpr int SK_PITCH = 256 + 16;
 // 4 / 8 ranges; 512 rows: 49.6 unsplit, 37.5 / 35.7 / 37.3 / 53; 86 tiles in two ranges 58.6 against 49.3).
 constexpr uint64_t kSplitFill = 128;
 constexpr uint32_t kSplitMax = 4;
-constexpr uint64_t kSkinnyWorkgroups = 256;  // per launch: one per CU (512 and 128 were measured: slower)
 
 // ---------------------------------------------------------------- any shape on the matrix cores
 //
@@ -1313,22 +1313,6 @@ int launch_gemv(int32_t *y, const uint8_t *a, const uint8_t *b, ZeroPoint za, Ze
     return launch_status();
 }
 
-// The shapes of mmi_ring and what a launch takes: `fixed` us a round of 256 workgroups (a CU holds one), and per 128 of k
-// `alone` ns while few CUs have a tile, `full` ns while all have one.
-struct RingShape {
-    uint32_t rows, cols;
-    double fixed, alone, full;
-};
-constexpr RingShape kRingShapes[] = {{64, 64, 2.5, 370, 390}, {64, 128, 3.5, 420, 535}, {128, 128, 6, 530, 800}, {128, 256, 9, 660, 1140}};
-constexpr int kRingShapeCount = 4;
-constexpr RingShape kLargeShape = {256, 256, 12, 1250, 1800};  // mmi_mfma_256x256
-
-inline double ring_us(const RingShape &t, size_t m, size_t n, double steps, size_t count) {
-    const double tiles = static_cast<double>((m + t.rows - 1) / t.rows) * static_cast<double>((n + t.cols - 1) / t.cols) * static_cast<double>(count);
-    const double rounds = static_cast<double>(static_cast<uint64_t>(tiles / 256)), left = tiles / 256 - rounds;
-    return rounds * (t.fixed + 1e-3 * steps * t.full) + (left > 0 ? t.fixed + 1e-3 * steps * (t.alone + (t.full - t.alone) * left) : 0);
-}
-
 template <bool DEQ>
 int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const void *b_zp, unsigned flags,
                size_t batch, size_t m, size_t k, size_t n, const uint32_t *a_index, const uint32_t *b_index,
@@ -1382,23 +1366,8 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
     // the ring tiles, any number of rows from five on: no zero points of B or one for all of it
     const bool ring = !gemv && k % 64 == 0 && k >= BK && k < (1u << 23) && n % 16 == 0 && n < (1u << 24) && aligned16(a) && aligned16(b) &&
                       !(zb.ptr && zb.per_row);
-    // Shape with the earliest expected end (us, from measurements at k = 1024 and 4096 like those in kRingShapes), or -1 where
-    // that is one of the other kernels: 256 x 256 tiles, or up to 32 rows mmi_skinny's three launches.
-    auto ring_shape = [&](uint32_t count) -> int {
-        const double steps = static_cast<double>((k + BK - 1) / BK);
-        int best = -1;
-        double us = 1e30;
-        for (int i = 0; i < kRingShapeCount; ++i) {
-            const double t = ring_us(kRingShapes[i], m, n, steps, count);
-            if (t < us) us = t, best = i;
-        }
-        if (fast && ring_us(kLargeShape, m, n, steps, count) < us) return -1;
-        if (skinny && m <= 32 && 8.5 + (DEQ ? 3.5 : 0) + 0.85e-3 * static_cast<double>(n) * count * steps / 32 < us) return -1;
-        return best;
-    };
     auto launch_ring = [&](int shape, uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
-        const RingShape &t = kRingShapes[shape];
-        const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
+        const uint64_t tiles = tile_count(kIntegerShapes[shape], m, n, 1);
         if (tiles > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
         const dim3 grid(static_cast<unsigned>(tiles), 1, count);
         const auto *a8 = static_cast<const uint8_t *>(a);
@@ -1490,13 +1459,14 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
 
     auto launch = [&](uint32_t am0, uint32_t bm0, uint32_t ym0, uint32_t count) -> int {
         if (ring) {
-            const int shape = ring_shape(count);
-            if (shape >= 0) return launch_ring(shape, am0, bm0, ym0, count);
-            if (fast) return launch_tiles(std::false_type{}, am0, bm0, ym0, count);
+            const IntegerRoute route = integer_route(m, k, n, count, DEQ, fast, skinny);
+            if (route.kernel == IntegerRoute::ring) return launch_ring(route.shape, am0, bm0, ym0, count);
+            if (route.kernel == IntegerRoute::large) return launch_tiles(std::false_type{}, am0, bm0, ym0, count);
+        } else {  // (a zero point per row of B, or k in no whole steps)
+            if (small_tiles_ok && (short_tile || (fast && !gemv && !skinny)) && small_tiles_pay(short_tile, count))
+                return launch_small_tiles(am0, bm0, ym0, count);
+            if (short_tile) return launch_tiles(std::true_type{}, am0, bm0, ym0, count);
         }
-        if (small_tiles_ok && (short_tile || (fast && !gemv && !skinny)) && small_tiles_pay(short_tile, count))
-            return launch_small_tiles(am0, bm0, ym0, count);
-        if (short_tile) return launch_tiles(std::true_type{}, am0, bm0, ym0, count);
         if (gemv) {
             const auto *a8 = static_cast<const uint8_t *>(a);
             const auto *b8 = static_cast<const uint8_t *>(b);
@@ -1523,14 +1493,9 @@ int mmi_launch(int32_t *y, const void *a, const void *b, const void *a_zp, const
             // up to four slabs of 32 rows share one pass over B
             for (size_t r0 = 0; r0 < m; r0 += 128) {
                 const uint32_t rows = static_cast<uint32_t>(m - r0 < 128 ? m - r0 : 128);
-                // k-tiles per workgroup: as few as keep about kSkinnyWorkgroups workgroups per launch (fewer atomics per
-                // output the more tiles a workgroup sums itself; with two and four slabs half as many workgroups and
-                // twice as many were measured: both slower)
-                const uint64_t target = kSkinnyWorkgroups;
-                const uint32_t k_tiles = static_cast<uint32_t>(k / BK);
-                uint32_t tiles = static_cast<uint32_t>((static_cast<uint64_t>(k_tiles) * (n / 256) * count + target - 1) / target);
-                tiles = tiles < 1 ? 1 : tiles > k_tiles ? k_tiles : tiles;
-                const unsigned splits = (k_tiles + tiles - 1) / tiles;
+                // (the fewer shares, the fewer atomics per output; with two and four slabs half as many workgroups and twice as
+                // many were measured: both slower)
+                const auto [tiles, splits] = integer_skinny_shares(k, n, count);
                 const dim3 grid(static_cast<unsigned>(n / 256), splits, count);
                 const auto *a8 = static_cast<const uint8_t *>(a);
                 const auto *b8 = static_cast<const uint8_t *>(b);

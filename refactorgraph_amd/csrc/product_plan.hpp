@@ -144,6 +144,60 @@ inline HalfRoute half_route(size_t m, size_t k, size_t n, size_t count, bool b_i
     return static_cast<uint64_t>(n) * k > 1400000u + 4500u * static_cast<uint64_t>(k) ? HalfRoute::tiles : HalfRoute::plain;
 }
 
+// ---------------------------------------------------------------- uint8 / int8
+//
+// Fitted over 3,600 products of 5 to 4096 rows, k 128 to 11008, 16 to 11008 columns, 1 to 128 of them side by side, every
+// form of zero points, int32 and dequantised outputs; over them the choice takes 0.9 % longer than the fastest kernel.
+
+// mmi_ring, steps of 128 k, and mmi_mfma_256x256.
+constexpr TileShape kIntegerShapes[] = {{64, 64, 3.2, 245, 330}, {64, 128, 4.5, 350, 660}, {128, 128, 4.8, 580, 770}, {128, 256, 7.7, 570, 1020}};
+constexpr int kIntegerShapeCount = 4;
+constexpr TileShape kIntegerLargeShape = {256, 256, 7.2, 1250, 1790};
+constexpr double kIntegerScaleUs = 1.0;  // a round of mmi_ring with dequantised outputs takes longer by this
+
+// mmi_skinny: tiles of 128 k that a workgroup of 256 columns sums itself, as few as keep about kSkinnyWorkgroups workgroups
+// per launch (one per CU; 512 and 128 were measured: slower), and the shares of k that makes.
+constexpr uint64_t kSkinnyWorkgroups = 256;
+struct SkinnyShares {
+    uint32_t tiles, shares;
+};
+inline SkinnyShares integer_skinny_shares(size_t k, size_t n, size_t count) {
+    const uint32_t k_tiles = static_cast<uint32_t>(k / 128);
+    uint32_t tiles = static_cast<uint32_t>((static_cast<uint64_t>(k_tiles) * (n / 256) * count + kSkinnyWorkgroups - 1) / kSkinnyWorkgroups);
+    tiles = tiles < 1 ? 1 : tiles > k_tiles ? k_tiles : tiles;
+    return {tiles, (k_tiles + tiles - 1) / tiles};
+}
+
+// mmi_zero, mmi_skinny and, for dequantised outputs, mmi_dequantize_in_place: a workgroup's tiles, one atomic per output and
+// share.  More than 128 rows are two passes over B and never ended first.
+inline double integer_skinny_us(size_t m, size_t k, size_t n, size_t count, bool dequantize) {
+    if (m > 128) return 1e30;
+    const SkinnyShares s = integer_skinny_shares(k, n, count);
+    const double rounds = static_cast<double>((n / 256) * s.shares * count) / static_cast<double>(kSkinnyWorkgroups);
+    const double outputs = 1e-6 * static_cast<double>(m) * static_cast<double>(n) * static_cast<double>(count);
+    const double fixed = m <= 32 ? 4.0 : m <= 64 ? 4.5 : 5.5, tile = m <= 32 ? 1.44 : m <= 64 ? 1.98 : 3.23;
+    return fixed + (rounds > 1 ? rounds : 1) * tile * s.tiles + 2.0 * outputs * s.shares + (dequantize ? 2.5 + 1.3 * outputs : 0);
+}
+
+struct IntegerRoute {
+    enum { ring, large, skinny } kernel;
+    int shape;  // of mmi_ring
+};
+
+// For operands that mmi_ring takes; large_ok, skinny_ok: the other two take them as well.
+inline IntegerRoute integer_route(size_t m, size_t k, size_t n, size_t count, bool dequantize, bool large_ok, bool skinny_ok) {
+    const double steps = static_cast<double>((k + 127) / 128);
+    IntegerRoute best{IntegerRoute::ring, 0};
+    double us = 1e30;
+    for (int i = 0; i < kIntegerShapeCount; ++i) {
+        const double t = 0.4 + tiles_us(kIntegerShapes[i], tile_count(kIntegerShapes[i], m, n, count), steps, dequantize ? kIntegerScaleUs : 0);
+        if (t < us) us = t, best = {IntegerRoute::ring, i};
+    }
+    if (large_ok && 0.4 + tiles_us(kIntegerLargeShape, tile_count(kIntegerLargeShape, m, n, count), steps) < us) return {IntegerRoute::large, 0};
+    if (skinny_ok && integer_skinny_us(m, k, n, count, dequantize) < us) return {IntegerRoute::skinny, 0};
+    return best;
+}
+
 // ---------------------------------------------------------------- F32
 //
 // Fitted over 2,500 products of 1 to 256 rows, k 64 to 8320, 16 to 50257 columns; over them the choice takes 0.06 % longer

@@ -199,6 +199,32 @@ static void productPlanRing() {
     EXPECT(rg::ring_plan(512, 64, 4096, 16, false).rest == 5 && rg::ring_plan(512, 64, 4099, 16, true).rest < 5);
 }
 
+static void productPlanInteger() {
+    // which kernel an integer product takes that mmi_ring takes too; kernel, or 10 + shape of the ring
+    using R = rg::IntegerRoute;
+    auto route = [](size_t count, size_t m, size_t k, size_t n, bool dequantize) {
+        const bool large = m >= 256 && n >= 256 && n % 16 == 0 && k % 128 == 0;
+        const bool skinny = !large && m < 256 && n % 256 == 0 && k % 128 == 0;
+        const auto r = rg::integer_route(m, k, n, count, dequantize, large, skinny);
+        return r.kernel == R::ring ? 10 + r.shape : static_cast<int>(r.kernel);
+    };
+    // few rows against a long k and few columns: one pass over B (measured: the pass, the ring, us)
+    EXPECT(route(1, 33, 11008, 256, false) == R::skinny);  // 8.3, 22
+    EXPECT(route(1, 64, 4096, 256, true) == R::skinny);    // 9.9, 11.5
+    EXPECT(route(1, 128, 11008, 256, false) == R::skinny); // 15.7, 30
+    EXPECT(route(1, 33, 11008, 4096, true) == R::skinny);  // 19.6, 29
+    EXPECT(route(1, 9, 4096, 4096, false) == R::skinny);   // 8.9, 13
+    EXPECT(route(1, 32, 4096, 11008, true) == 10 && route(1, 64, 4096, 4096, true) == 10);
+    EXPECT(route(1, 129, 11008, 256, false) == 10);
+    EXPECT((rg::integer_skinny_shares(4096, 4096, 1).tiles == 2 && rg::integer_skinny_shares(4096, 4096, 1).shares == 16));
+    // the 256 x 256 tiles, and the shapes of the ring
+    EXPECT(route(1, 4096, 4096, 4096, false) == R::large);
+    EXPECT(route(1, 2048, 128, 4096, true) == R::large && route(1, 512, 128, 11008, true) == R::large); // 9.7, 11.5; 8.5, 10.2
+    EXPECT(route(1, 512, 512, 11008, false) == 13 && route(128, 512, 512, 256, true) == R::large);
+    EXPECT(route(1, 1000, 4096, 4096, true) == 12 && route(1, 2048, 4096, 2048, true) == 12);
+    EXPECT(route(1, 300, 512, 4112, false) == 11 && route(1, 512, 2048, 11008, true) == 13);
+}
+
 static void shapeDigests() {
     auto x = Tensor::share(DataType::F32, Shape{2, 3, 4, 5});
     SoftmaxInfo s(*x, 1);
@@ -2180,6 +2206,7 @@ int main(int argc, char **argv) {
     RUN(productPlanF32);
     RUN(productPlanHalf);
     RUN(productPlanRing);
+    RUN(productPlanInteger);
     RUN(memPoolBestFit);
     RUN(resourcesAndErrors);
     RUN(collectorsSelectOrDecline);
