@@ -1,0 +1,46 @@
+// Which attention kernel a call with several new rows takes: a plain function of sizes (no device, no HIP), so that the
+// choice is tested on the CPU.
+#pragma once
+
+#include <cstddef>
+
+namespace rg {
+
+// Several query rows per batch row: the tiled kernel stages K/V once per 32 query rows x 4 heads, but an item walks
+// all of its keys by itself, while the split kernel reads K/V once per query row and spreads the keys over every
+// CU.  With the history length h: tiled about rounds * h * 0.020 us (rounds = items over the 512 workgroups that
+// are resident), split about N * Hkv * seq * h * 512 B at 7 TB/s; h cancels.  Measured at N = 32, 8 kv heads,
+// h = 4000: 4 rows 109 us tiled against 318 us split, 2 rows 108 against 159; at N = 1: 4 rows 84 against 20.
+constexpr size_t kPrefillAlways = 32;  // query rows from which the tiled kernel is used whatever the batch
+
+// ranges_fit: the workspace holds the records of shared keys.
+inline bool prefill_pays(size_t N, size_t n_head, size_t n_kv_head, size_t seq, size_t cap, size_t D, bool ranges_fit) {
+    if (seq >= kPrefillAlways) return true;
+    const size_t group = n_head / n_kv_head, heads_per_item = group == 1 ? 1 : group == 2 ? 2 : 4;
+    // the split kernel takes eight, four, two or one heads of a group per launch and reads K/V again in every launch
+    // (a group of 7: three times), while the chunks of a group on the tiled kernel find them in L2
+    size_t split_launches = 0;
+    for (size_t left = group; left > 0; left -= left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1) ++split_launches;
+    if (seq < 2 && split_launches < 2) return false;
+    const size_t rows_per_item = 32 * (4 / heads_per_item);
+    const size_t items = N * n_kv_head * ((group + heads_per_item - 1) / heads_per_item) * ((seq + rows_per_item - 1) / rows_per_item);
+    if (ranges_fit && seq == 1 && split_launches >= 2 && (D == 64 || D == 128)) return true;  // (16 x 28/4 heads, history 4000: 80 -> 52 us)
+    // Few items: the tiled kernel shares an item's keys between workgroups (head dims 64 and 128, records in the
+    // workspace).  Fitted over 2,300 calls (1 to 8 sequences, groups of 1 to 8, 2 to 31 rows, capacities 1024 to 32768, four
+    // histories each): tiled about 14 us + 9.2e-5 us per kv head and key, split 9.6 us a launch + 6.7e-5 us per kv head, key
+    // and query row at D = 128 (half the bytes at 64).  So a second launch alone is worth the tiled kernel (28 / 4 heads,
+    // 3 rows behind 8189: 50 us split, 23 tiled).  The history is device data and the host may not read it, so half of the
+    // capacity stands for it.  Both costs are linear in the history with the tiled kernel's slope the smaller one, so the
+    // wrong choice costs most at the ends: with a history near nothing where the rule chose tiled (10 us lost at 8 kv heads,
+    // 19 at 16: the records of ranges without a key), with a full cache where it chose split.  3 us between the constants
+    // gave the least time lost over those calls, 1.1 us a call (1.7 with 9.5 us and slopes of 9.4e-5 and 7.3e-5).
+    if (ranges_fit && seq >= 2 && items * 2 <= 512 && cap >= 1024 && (D == 64 || D == 128)) {
+        if (split_launches >= 2) return true;
+        const double keys = static_cast<double>(N * n_kv_head) * static_cast<double>(cap) / 2;
+        return 3.0 < keys * (6.7e-5 * static_cast<double>(D) / 128 * static_cast<double>(seq) - 9.2e-5);
+    }
+    const size_t rounds = (items + 511) / 512;
+    return N * n_kv_head * seq * split_launches >= 280 * rounds;
+}
+
+}  // namespace rg

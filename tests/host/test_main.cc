@@ -38,6 +38,7 @@
 #include "rg_mirror/executor.h"
 #include "rg_mirror/hip_kernels.h"
 #include "oracle.h"
+#include "../../refactorgraph_amd/csrc/attention_plan.hpp"
 #include "../../refactorgraph_amd/csrc/product_plan.hpp"
 
 #include <chrono>
@@ -223,6 +224,21 @@ static void productPlanInteger() {
     EXPECT(route(1, 512, 512, 11008, false) == 13 && route(128, 512, 512, 256, true) == R::large);
     EXPECT(route(1, 1000, 4096, 4096, true) == 12 && route(1, 2048, 4096, 2048, true) == 12);
     EXPECT(route(1, 300, 512, 4112, false) == 11 && route(1, 512, 2048, 11008, true) == 13);
+}
+
+static void attentionPlan() {
+    // tiled kernel or not: N, query heads, kv heads, new rows, capacity, head dim (measured at half the capacity: split, tiled, us)
+    auto tiled = [](size_t n, size_t h, size_t hk, size_t seq, size_t cap, size_t d) { return rg::prefill_pays(n, h, hk, seq, cap, d, true); };
+    EXPECT(!tiled(1, 32, 8, 1, 32768, 128) && tiled(1, 32, 8, 32, 64, 128));
+    EXPECT(!tiled(1, 32, 8, 2, 1024, 128) && !tiled(1, 32, 8, 2, 4096, 64));
+    EXPECT(tiled(1, 32, 8, 31, 1024, 128));   // a second reading of the keys per row soon costs more than the records
+    EXPECT(tiled(1, 32, 8, 8, 4096, 128));
+    EXPECT(tiled(1, 32, 8, 4, 8192, 128) && tiled(1, 32, 8, 2, 32768, 128));
+    EXPECT(tiled(1, 28, 4, 2, 4096, 128));    // 36.6, 15.6: three launches on the split kernel
+    EXPECT(tiled(1, 28, 4, 3, 8192, 128));    // 40.5, 18.6
+    EXPECT(tiled(16, 28, 4, 1, 4096, 128));
+    // without room for records, other head dims: the rule for items that walk all of their keys
+    EXPECT(!rg::prefill_pays(1, 32, 8, 4, 4096, 128, false) && !tiled(1, 32, 8, 4, 4096, 96) && tiled(32, 32, 8, 2, 4096, 96));
 }
 
 static void shapeDigests() {
@@ -2207,6 +2223,7 @@ int main(int argc, char **argv) {
     RUN(productPlanHalf);
     RUN(productPlanRing);
     RUN(productPlanInteger);
+    RUN(attentionPlan);
     RUN(memPoolBestFit);
     RUN(resourcesAndErrors);
     RUN(collectorsSelectOrDecline);
