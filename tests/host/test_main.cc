@@ -196,6 +196,17 @@ static void productPlanRing() {
     EXPECT(is(rg::ring_plan(2048, 4096, 11008, 1, false), 5, 3, 8192)); // 256 x 256, then 128 x 192
     EXPECT(is(rg::ring_plan(64, 4096, 4096, 1, false), 0, 0, 0));
     EXPECT(is(rg::ring_plan(4096, 4096, 4096, 1, false), 5, 5, 0));
+    // the sizes of the GPU tests of the ring tiles (0: 64 x 64, 1: 64 x 128, 2: 128 x 128, 3: 128 x 192, 4: 128 x 256, 5: 256 x 256)
+    struct { size_t m, k, n; int rest; uint32_t columns; } const sizes[] = {
+        {9, 64, 4096, 0, 0}, {17, 128, 264, 0, 0}, {64, 192, 520, 0, 0}, {65, 320, 1000, 0, 0}, {130, 448, 2056, 0, 0}, {255, 512, 1032, 0, 0},
+        {300, 576, 4000, 1, 0}, {513, 640, 4104, 2, 0}, {1025, 256, 6152, 4, 0}, {1000, 320, 6144, 3, 0}, {2048, 1024, 4096, 4, 0},
+        {4000, 512, 4104, 0, 4096}, {2049, 1024, 11016, 4, 0}, {256, 64, 256, 0, 0},
+        {100, 1024, 520, 0, 0}, {70, 704, 200, 0, 0}, {130, 832, 1040, 0, 0},
+        {2048, 512, 11016, 3, 8192}, {4100, 512, 8200, 2, 7680}, {1800, 512, 12040, 4, 8192}, {2000, 704, 9000, 1, 8192}};
+    for (auto const &z : sizes) {
+        const auto p = rg::ring_plan(z.m, z.k, z.n, 1, false);
+        EXPECT(p.rest == z.rest && p.columns == z.columns && (p.columns == 0 || p.first == 5));
+    }
     // element-wise stores: the largest tiles give way (16 products [512, 64] x [4099, 64]^T)
     EXPECT(rg::ring_plan(512, 64, 4096, 16, false).rest == 5 && rg::ring_plan(512, 64, 4099, 16, true).rest < 5);
 }
@@ -223,6 +234,13 @@ static void productPlanInteger() {
     EXPECT(route(1, 2048, 128, 4096, true) == R::large && route(1, 512, 128, 11008, true) == R::large); // 9.7, 11.5; 8.5, 10.2
     EXPECT(route(1, 512, 512, 11008, false) == 13 && route(128, 512, 512, 256, true) == R::large);
     EXPECT(route(1, 1000, 4096, 4096, true) == 12 && route(1, 2048, 4096, 2048, true) == 12);
+    // the sizes of the GPU test of the ring tiles
+    EXPECT(route(1, 5, 128, 16, false) == 10 && route(1, 33, 192, 80, false) == 10 && route(1, 64, 704, 1040, false) == 10);
+    EXPECT(route(1, 100, 1088, 4096, false) == 10 && route(1, 130, 960, 272, false) == 10);
+    for (size_t k : {640, 896, 1088}) EXPECT(route(1, 300, k, 4112, false) == 11 && route(1, 300, k, 4112, true) == 11);
+    EXPECT(route(1, 200, 1024, 6160, false) == 11 && route(1, 250, 960, 5008, false) == 11);
+    EXPECT(route(1, 513, 576, 4096, false) == 12 && route(1, 1000, 1088, 4096, false) == 12);
+    EXPECT(route(1, 2048, 448, 4096, false) == 13 && route(1, 1025, 320, 6160, false) == 13);
     EXPECT(route(1, 300, 512, 4112, false) == 11 && route(1, 512, 2048, 11008, true) == 13);
 }
 

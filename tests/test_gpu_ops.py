@@ -403,6 +403,12 @@ def test_dynamic_quantize_bit_exact(n, lo, hi):
     _dql_check(x)
 
 
+@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1, (1 << 19) - 3, 1 << 19, (1 << 19) + 1, 1 << 22, (1 << 22) + 5, 9_000_003, (1 << 26) + 8197])
+def test_dynamic_quantize_vectors_per_thread(n):
+    """Both sides of every change of the vectors a thread takes (1, 2, 4, 8), more than one step in either launch."""
+    _dql_check(np.random.default_rng(n).uniform(-3.0, 5.0, n).astype(np.float32))
+
+
 def test_dynamic_quantize_ties_zeros_and_unaligned():
     y, scale, zp = _dql_check(np.array([0.0, 255.0, 2.5, 0.5, 1.5, 254.5], np.float32))
     assert y.tolist() == [0, 255, 3, 1, 2, 255]           # ties away from zero
@@ -664,9 +670,11 @@ def test_matmul_integer_one_to_four_rows_matrix_vector(m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(5, 128, 16), (33, 192, 80), (64, 704, 1040), (100, 1088, 4096), (130, 960, 272), (300, 640, 4112),
-                                   (513, 576, 4096), (1000, 1088, 4096), (2048, 448, 4096), (1025, 320, 6160)])
+                                   (513, 576, 4096), (1000, 1088, 4096), (2048, 448, 4096), (1025, 320, 6160),
+                                   # 64 x 128 tiles (the CPU test productPlanInteger has the shapes): more k-tiles than stages, half tiles
+                                   (300, 896, 4112), (300, 1088, 4112), (200, 1024, 6160), (250, 960, 5008)])
 def test_matmul_integer_ring_tiles(m, k, n):
-    """Edges of the tiles, k that ends with half a tile, fewer k-tiles than the ring has stages, every zero point form."""
+    """Edges of the tiles, k that ends with half a tile, fewer and more k-tiles than the ring has stages, every zero point form."""
     rng = np.random.default_rng(m + k + n)
     a, b = rng.integers(0, 256, (m, k), dtype=np.uint8), rng.integers(-128, 128, (k, n), dtype=np.int8)
     s = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
@@ -1566,9 +1574,9 @@ def test_matmul_groups_of_matrices_that_share_one_b(S, T, D):
 
 @pytest.mark.parametrize("tb", [True, False])
 @pytest.mark.parametrize("m,k,n", [
-    (9, 64, 4096), (17, 128, 264), (64, 192, 520), (65, 320, 1000), (130, 448, 2056), (255, 512, 1032),   # 64-row tiles
-    (300, 576, 4000), (513, 640, 4104), (1025, 256, 6152), (1000, 320, 6144),                             # wider ones
-    (2048, 1024, 4096), (4000, 512, 4104), (2049, 1024, 11016), (256, 64, 256)])                          # 256 rows, two shapes
+    (9, 64, 4096), (17, 128, 264), (64, 192, 520), (65, 320, 1000), (130, 448, 2056), (255, 512, 1032),   # 64 x 64
+    (300, 576, 4000), (513, 640, 4104), (1025, 256, 6152), (1000, 320, 6144),           # 64 x 128, 128 x 128, 128 x 256, 128 x 192
+    (2048, 1024, 4096), (4000, 512, 4104), (2049, 1024, 11016), (256, 64, 256)])        # 128 x 256, two shapes, 128 x 256, 64 x 64
 def test_matmul_ring_tiles_exact_on_small_integers(m, k, n, tb):
     """Edges of the tiles and fewer k-tiles than the ring has stages: sums of small integers are exact in float, so the
     result is the exact product rounded once, whatever the order of the sum."""
@@ -1581,6 +1589,20 @@ def test_matmul_ring_tiles_exact_on_small_integers(m, k, n, tb):
             y = ops.matmul(a.to(dt), b.to(dt), None if c is None else c.to(dt), trans_b=tb)
             ref = exact if c is None else exact + c.double()
             assert torch.equal(y, ref.to(dt)), (n_, dt, None if c is None else tuple(c.shape))
+
+
+# (the CPU test productPlanRing holds the shapes that these sizes take)
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("m,k,n", [
+    (100, 1024, 520), (70, 704, 200), (130, 832, 1040),                   # 64 x 64, more k-tiles than the ring has stages
+    (2048, 512, 11016), (4100, 512, 8200), (1800, 512, 12040), (2000, 704, 9000)])  # 256 x 256, then 128 x 192, 128 x 128, 128 x 256, 64 x 128
+def test_matmul_ring_tiles_two_shapes_and_steady_state(m, k, n, tb):
+    """Several ragged tiles of a second shape behind whole rounds of the first, exact on small integers."""
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a, b, c = (torch.randint(-2, 3, s, generator=g, device="cuda").bfloat16() for s in ((m, k), (n, k) if tb else (k, n), (n,)))
+    exact = a.double() @ (b.double().t().contiguous() if tb else b.double())
+    assert torch.equal(ops.matmul(a, b, trans_b=tb), exact.bfloat16())
+    assert torch.equal(ops.matmul(a, b, c, trans_b=tb), (exact + c.double()).bfloat16())
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 64, 17), (3, 128, 9), (5, 320, 1), (12, 832, 2680), (14, 3520, 583), (32, 192, 31), (33, 576, 121)])
