@@ -771,7 +771,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
 // sub-tile, lane = query row and half of the keys), each taking four of a thread's accumulator registers
 // (blockIdx.y: four consecutive d), add the ranges' records weighted by 2^(m_range - m_max), normalise
 // and store four consecutive d per instruction.
-// (eight registers, half the workgroups: 10.6 against 7.5 us for 32 items of 16 ranges; sixteen: level at 256 items of two)
+// (eight registers, half the workgroups: 10.6 against 7.5 us for 32 items of 16 ranges; many items of few ranges would rather
+// have more: 256 items of two 10.9 us with four, 10.3 with eight, 10.0 with sixteen)
 constexpr int kMergeRegs = 4;
 template <class T, int HW, int DH>
 __global__ __launch_bounds__(256) void attn_prefill_merge(const PrefillArgs a, const PrefillPlan plan) {

@@ -21,6 +21,23 @@ inline int launch_status() { return static_cast<int>(hipGetLastError()); }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// ---------------------------------------------------------------- tile kernels
+
+// A wave-uniform pointer, moved to scalar registers (so that what is added to it later is scalar arithmetic).
+// (The builtin returns int: without the casts the low word would be sign-extended over the high one.)
+__device__ __forceinline__ const uint8_t *scalar_pointer(const uint8_t *p) {
+    const uint64_t bits = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits)));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32)));
+    return reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// The tile of a workgroup: consecutive workgroup ids go round-robin to the 8 XCDs, each XCD gets a contiguous run of tiles.
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t workgroup, uint32_t tiles) {
+    const uint32_t xcd = workgroup % 8, share = tiles / 8, more = tiles % 8;
+    return xcd * share + (xcd < more ? xcd : more) + workgroup / 8;
+}
+
 // ---------------------------------------------------------------- DPP lane exchange
 // dpp_ctrl encodings (GCN3+ ISA): quad_perm = perm bits, row_half_mirror = 0x141,
 // row_mirror = 0x140.  Four DPP steps leave every lane of a 16-lane row holding the row's

@@ -452,19 +452,11 @@ __global__ __launch_bounds__(256, 2) void mm_tiles16(T *__restrict__ y, const T 
     store_blocks<T, MI, 2>(acc, y, bias, ym, row0 + wm * (TM / 2), col0 + wn * 64, m, n, alpha, beta);
 }
 
-// A wave-uniform pointer, moved to scalar registers (so that what is added to it later is scalar arithmetic).
-__device__ __forceinline__ const uint8_t *uniform_pointer(const uint8_t *p) {
-    const uint64_t bits = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits)));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32)));
-    return reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-
 // ---------------------------------------------------------------- FP16 / BF16: middle-sized products
 //
-// 64 MI x 64 NJ outputs per workgroup of four wavefronts (32 MI x 32 NJ each, blocks of v_mfma_f32_32x32x16), k in tiles
-// of 64 copied straight into a ring of NS stages of LDS, up to NS - 1 tiles ahead of the one being multiplied.
-// A stage is a row of 8 KiB panels, 64 lines of 128 bytes each, A's MI panels first:
+// 32 MI WM x 32 NJ WN outputs per workgroup of WM x WN wavefronts (32 MI x 32 NJ each, blocks of v_mfma_f32_32x32x16), k in
+// tiles of 64 copied straight into a ring of NS stages of LDS, up to NS - 1 tiles ahead of the one being multiplied.
+// A stage is a row of 8 KiB panels, 64 lines of 128 bytes each, A's TM / 64 panels first, then B's TN / 64:
 //   A, and B as [n, k]: a line is a row of the tile (64 k); chunk c (16 bytes) of row r at position c ^ (r & 7) ^ ((r >> 3) & 1)
 //   B as [k, n]: a line is a k-row of 64 columns; chunk c of k-row r at position c ^ 4 ((r >> 1) & 1) ^ 2 ((r >> 3) & 1), read
 //   by ds_read_b64_tr_b16 (four k-rows of 16 columns per 16 lanes); both patterns meet every LDS bank once.
@@ -474,15 +466,20 @@ __device__ __forceinline__ const uint8_t *uniform_pointer(const uint8_t *p) {
 // Eight wavefronts (but for the smallest tile): two on a SIMD, so that the products of one fill the clocks in which the
 // other issues its copies (with four of twice the size 128 x 128 takes 44.5 us at [1000, 4096] x [4096, 4096]^T instead of
 // 40.8, 128 x 256 71 instead of 64 at 2048 rows).  k-tiles of 32 in twice the stages are slower (51 us: lines are fetched in
-// halves), a fifth stage changes nothing.  Bound by what the CUs together take from L2 and the memory-side cache: a
-// workgroup with the chip to itself needs 24 us for 128 x 128 x 4096, 256 of them 41 us (13 TB/s of operands; the products
-// alone would be 14 us).  FP16 / BF16, k = 4096, device time before (registers filled three tiles ahead for 128 x 128, two
+// halves), a fifth stage changes nothing.
+// What bounds it, at that size (256 tiles of 128 x 128, 38 us on the day): without the copies 26.6 us, without the products
+// 26.3 us (536 MB from L2 at 20 TB/s), so neither alone; the two overlap by half.  Counters of a launch: the matrix pipe
+// busy 61 % of the resident clocks, fragment reads on the LDS data path 48 %, L2 hits 80 %.
+// FP16 / BF16, k = 4096, device time before (registers filled three tiles ahead for 128 x 128, two
 // LDS buffers for 256 x 256) and now: [1000, 4096] x [4096, 4096]^T 62 -> 41 us (825 TFLOP/s), 6144 columns 78 -> 53,
 // [2048, 4096] x [4096, 4096]^T 110 -> 64 us (1,070 TFLOP/s), 11008 columns 210 -> 169, 64 rows as [k, n] 47 -> 17 us.
 template <class T, bool TRANS_B, int WM, int WN, int MI, int NJ, int NS>
 struct Ring {
     static constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, WAVES = WM * WN, LINE = 128, STAGE = (TM + TN) * LINE, LDS = NS * STAGE;
     static constexpr int COPIES_A = TM * LINE / 1024 / WAVES, COPIES_B = TN * LINE / 1024 / WAVES, COPIES = COPIES_A + COPIES_B;  // of a wavefront and tile
+    // whole panels, whole copies per wavefront, copies in flight within the wait counter, room for the epilogue's rows
+    static_assert(TM % 64 == 0 && TN % 64 == 0 && TM % (8 * WAVES) == 0 && TN % (8 * WAVES) == 0 && (NS - 1) * COPIES < 64);
+    static_assert(LDS <= 163840 && WAVES * 2048 * MI * NJ <= LDS);
 };
 
 template <class T, bool TRANS_B, int WM, int WN, int MI, int NJ, int NS>
@@ -517,8 +514,8 @@ __device__ __forceinline__ void ring_loop(f16v (&acc)[MI][NJ], uint8_t *lds, con
             voff[CA + q] = 2 * (kr * n + (col + 8 <= n ? col : n - 8));
         }
     }
-    const uint8_t *a_base = uniform_pointer(A + static_cast<uint64_t>(row0) * (2 * k));
-    const uint8_t *b_base = uniform_pointer(TRANS_B ? B + static_cast<uint64_t>(col0) * (2 * k) : B);
+    const uint8_t *a_base = scalar_pointer(A + static_cast<uint64_t>(row0) * (2 * k));
+    const uint8_t *b_base = scalar_pointer(TRANS_B ? B + static_cast<uint64_t>(col0) * (2 * k) : B);
     const uint64_t b_step = TRANS_B ? LINE : static_cast<uint64_t>(LINE) * n;  // bytes from one tile of B to the next
     const uint32_t lds0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
         static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds))));
@@ -564,8 +561,8 @@ __device__ __forceinline__ void ring_loop(f16v (&acc)[MI][NJ], uint8_t *lds, con
     };
 
     const uint32_t k_tiles = k / 64;
-    auto a_tile = [&](uint32_t t) { return uniform_pointer(a_base + (t < k_tiles ? t : 0) * static_cast<uint64_t>(LINE)); };
-    auto b_tile = [&](uint32_t t) { return uniform_pointer(b_base + (t < k_tiles ? t : 0) * b_step); };
+    auto a_tile = [&](uint32_t t) { return scalar_pointer(a_base + (t < k_tiles ? t : 0) * static_cast<uint64_t>(LINE)); };
+    auto b_tile = [&](uint32_t t) { return scalar_pointer(b_base + (t < k_tiles ? t : 0) * b_step); };
     // tiles 0 .. NS - 2 and the first half of tile NS - 1's copies (behind the end: tile 0 again, never multiplied)
     auto fill = [&]<int COUNT>(uint32_t tile, uint32_t stage) __attribute__((always_inline)) {
         const uint8_t *a_from = a_tile(tile), *b_from = b_tile(tile);
@@ -720,11 +717,9 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void mm_ring(T *__restri
     __shared__ __align__(1024) uint8_t lds[R::LDS];
     const uint32_t bz = blockIdx.z;
     const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
-    // consecutive workgroup ids go round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, walked down the
-    // rows of one column panel after the other
-    const uint32_t row_tiles = (m + R::TM - 1) / R::TM, n_tiles = row_tiles * ((columns + R::TN - 1) / R::TN);
-    const uint32_t xcd = blockIdx.x % 8, share = n_tiles / 8, more = n_tiles % 8;
-    const uint32_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / 8;
+    // an XCD's run of tiles is walked down the rows of one column panel after the other
+    const uint32_t row_tiles = (m + R::TM - 1) / R::TM;
+    const uint32_t tile = xcd_tile(blockIdx.x, row_tiles * ((columns + R::TN - 1) / R::TN));
     const uint32_t row0 = (tile % row_tiles) * R::TM, col0 = col_first + (tile / row_tiles) * R::TN;
     f16v acc[MI][NJ];
 #pragma unroll
@@ -2084,7 +2079,6 @@ int launch_typed(void *y_, const void *a_, const void *b_, Bias bias, int trans_
                 const dim3 grid(static_cast<unsigned>(tiles), 1, count);
 #define RG_RING(WM, WN, MI, NJ, NS)                                                                                          \
     do {                                                                                                                     \
-        static_assert(Ring<T, true, WM, WN, MI, NJ, NS>::LDS <= 163840);                                                     \
         if (trans_b) mm_ring<T, true, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a, b, bias, m32, k32, n32, first, columns, al, be, am0, bm0, ym0); \
         else mm_ring<T, false, WM, WN, MI, NJ, NS><<<grid, 64 * WM * WN, 0, s>>>(y, a, b, bias, m32, k32, n32, first, columns, al, be, am0, bm0, ym0);        \
     } while (0)

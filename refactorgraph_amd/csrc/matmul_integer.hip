@@ -124,15 +124,6 @@ constexpr int D_STAGE = 2 * D_TILE;      // one LDS buffer
 
 __device__ __forceinline__ uint32_t b_swizzle(uint32_t x) { return ((x & 3) << 1) | ((x >> 2) * 9); }  // x < 8
 
-// A wave-uniform pointer, moved to scalar registers (so that what is added to it later is scalar arithmetic).
-// (The builtin returns int: without the casts the low word would be sign-extended over the high one.)
-__device__ __forceinline__ const uint8_t *scalar_pointer(const uint8_t *p) {
-    const uint64_t bits = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits)));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bits >> 32)));
-    return reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-
 // SHORT_M: A has only a_rows < 256 rows; the tile's rows beyond them are copied from the last one (their results
 // are not stored).
 template <int A_MODE, bool B_ZP, bool SHORT_M>
@@ -585,7 +576,10 @@ __global__ __launch_bounds__(256, 1) void mmi_mfma_256x256(int32_t *__restrict__
 // steps is what a launch waits for: [100, 4096] x [4096, 4096] 16.6 -> 14.9 us); their sums meet in LDS at the end.
 // Eight wavefronts for the larger tiles: two on a SIMD, one of which issues products while the other issues its copies or
 // subtracts zero points (four vector instructions per word of A: with 1 x 2 blocks per wavefront they fit behind the products,
-// with 2 x 1 blocks a launch takes 8 % longer).  Bound by what the CUs together take from L2 and the memory-side cache.
+// with 2 x 1 blocks a launch takes 8 % longer).
+// What bounds it, [1000, 4096] x [4096, 4096] dequantised on 128 x 128 tiles (31.0 us): without the copies 24.7 us, without the
+// products 21.2, without the subtraction 25.5 (100 rows on 64 x 64 tiles: 12.3, 10.1, 11.4 and 9.7).  Counters of a launch:
+// vector issue busy 49 % of the resident clocks, the matrix pipe 32 %, the LDS data path 25 %, L2 hits 78 %.
 // uint8 activations with an arbitrary zero point, k = 4096, before (mmi_tiles, 256 x 256 tiles with k shared) and now:
 // [1000, 4096] x [4096, 4096] 43.6 -> 31.6 us (1,060 TOP/s), 2048 rows 61 -> 46, 512 rows 44 -> 20.5, 100 rows 27 -> 17 us.
 template <int WM, int WN, int MI, int NJ, int NS, int WK>
@@ -767,11 +761,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK > 4 ? 2 : 1) void m
     __shared__ __align__(1024) uint8_t lds[R::LDS];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, bz = blockIdx.z;
     const uint64_t am = a_matrix0 + bz, bm = b_matrix0 + bz, ym = y_matrix0 + bz;
-    // consecutive workgroup ids go round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, walked down the
-    // rows of one column panel after the other
-    const uint32_t row_tiles = (m + R::TM - 1) / R::TM, n_tiles = row_tiles * ((n + R::TN - 1) / R::TN);
-    const uint32_t xcd = blockIdx.x % 8, share = n_tiles / 8, more = n_tiles % 8;
-    const uint32_t tile = xcd * share + (xcd < more ? xcd : more) + blockIdx.x / 8;
+    // an XCD's run of tiles is walked down the rows of one column panel after the other
+    const uint32_t row_tiles = (m + R::TM - 1) / R::TM;
+    const uint32_t tile = xcd_tile(blockIdx.x, row_tiles * ((n + R::TN - 1) / R::TN));
     const uint32_t row0 = (tile % row_tiles) * R::TM, col0 = (tile / row_tiles) * R::TN;
     const uint32_t wave_row = row0 + (wave / WN % WM) * 32 * MI, wave_col = col0 + (wave % WN) * 32 * NJ;
     uint32_t za_f[MI];

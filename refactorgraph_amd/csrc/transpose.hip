@@ -24,7 +24,7 @@ namespace {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kMaxDims = 8;
 constexpr int UNROLL = 4;  // words a thread has in flight
-constexpr uint64_t kFewTiles = 1024;
+constexpr uint64_t kFewTiles = 1024;  // tiles that four workgroups each share, below four per CU
 constexpr uint32_t TILE_H = 8, TILE_S = 8;   // blocks of a tile along the two dimensions that change places
 
 struct Divisor {
@@ -353,7 +353,7 @@ int launch(void *y, const void *x, const Plan &p, const uint32_t *stride_i, cons
             t.tiles_per_outer = make_divisor((extent_h / TILE_H) * (extent_s / TILE_S));
             const uint64_t tiles = block_count / (TILE_H * TILE_S);
             if (tiles <= 0x7fffffffull) {
-// few tiles: four workgroups each, a word per thread (8 kv heads x 1000 tokens of 256 bytes, 125 tiles: 5.0 -> 4.0 us,
+                // few tiles: four workgroups each, a word per thread (8 kv heads x 1000 tokens of 256 bytes, 125 tiles: 5.0 -> 4.0 us,
                 // 32 heads 6.6 -> 5.4 us)
                 if (tiles < kFewTiles)
                     transpose_tiles<Word, 1><<<dim3(static_cast<unsigned>(tiles), 4), 256, 0, s>>>(static_cast<Word *>(y), static_cast<const Word *>(x), t);
