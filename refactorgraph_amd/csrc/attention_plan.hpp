@@ -26,18 +26,16 @@ inline bool prefill_pays(size_t N, size_t n_head, size_t n_kv_head, size_t seq, 
     const size_t items = N * n_kv_head * ((group + heads_per_item - 1) / heads_per_item) * ((seq + rows_per_item - 1) / rows_per_item);
     if (ranges_fit && seq == 1 && split_launches >= 2 && (D == 64 || D == 128)) return true;  // (16 x 28/4 heads, history 4000: 80 -> 52 us)
     // Few items: the tiled kernel shares an item's keys between workgroups (head dims 64 and 128, records in the
-    // workspace).  Fitted over 2,300 calls (1 to 8 sequences, groups of 1 to 8, 2 to 31 rows, capacities 1024 to 32768, four
-    // histories each): tiled about 14 us + 9.2e-5 us per kv head and key, split 9.6 us a launch + 6.7e-5 us per kv head, key
-    // and query row at D = 128 (half the bytes at 64).  So a second launch alone is worth the tiled kernel (28 / 4 heads,
-    // 3 rows behind 8189: 50 us split, 23 tiled).  The history is device data and the host may not read it, so half of the
-    // capacity stands for it.  Both costs are linear in the history with the tiled kernel's slope the smaller one, so the
-    // wrong choice costs most at the ends: with a history near nothing where the rule chose tiled (10 us lost at 8 kv heads,
-    // 19 at 16: the records of ranges without a key), with a full cache where it chose split.  3 us between the constants
-    // gave the least time lost over those calls, 1.1 us a call (1.7 with 9.5 us and slopes of 9.4e-5 and 7.3e-5).
+    // workspace).  The history is device data and the host may not read it, so half of the capacity stands for it.  The costs
+    // below are those of the tiled kernel with a pair of query tiles per workgroup; with one it takes about 14 us + 9.2e-5 us
+    // per kv head and key, the split kernel 9.6 us a launch + 6.7e-5 us per kv head, key and query row (2,300 calls).  The line
+    // stays where it was all the same: the split kernel keeps probabilities in float, the tiled one in 16 bits for the matrix
+    // cores (2.1e-4 and 2.9e-4 from 64 bits in fp16), and a call does not lose that for 2 to 10 us (8 rows behind 2048 of 4096
+    // positions, 8 kv heads: split 20.7 us, tiled 15.9).  Both costs are linear in the history with the tiled kernel's slope
+    // the smaller one, so the wrong choice costs most at the ends.
     if (ranges_fit && seq >= 2 && items * 2 <= 512 && cap >= 1024 && (D == 64 || D == 128)) {
-        if (split_launches >= 2) return true;
         const double keys = static_cast<double>(N * n_kv_head) * static_cast<double>(cap) / 2;
-        return 3.0 < keys * (6.7e-5 * static_cast<double>(D) / 128 * static_cast<double>(seq) - 9.2e-5);
+        return 9.5 < keys * (7.3e-5 * static_cast<double>(seq * split_launches) - 9.4e-5);
     }
     const size_t rounds = (items + 511) / 512;
     return N * n_kv_head * seq * split_launches >= 280 * rounds;

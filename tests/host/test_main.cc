@@ -245,18 +245,15 @@ static void productPlanInteger() {
 }
 
 static void attentionPlan() {
-    // tiled kernel or not: N, query heads, kv heads, new rows, capacity, head dim (measured at half the capacity: split, tiled, us)
+    // tiled kernel or not: N, query heads, kv heads, new rows, capacity, head dim
     auto tiled = [](size_t n, size_t h, size_t hk, size_t seq, size_t cap, size_t d) { return rg::prefill_pays(n, h, hk, seq, cap, d, true); };
     EXPECT(!tiled(1, 32, 8, 1, 32768, 128) && tiled(1, 32, 8, 32, 64, 128));
     EXPECT(!tiled(1, 32, 8, 2, 1024, 128) && !tiled(1, 32, 8, 2, 4096, 64));
-    EXPECT(tiled(1, 32, 8, 31, 1024, 128));   // a second reading of the keys per row soon costs more than the records
-    EXPECT(tiled(1, 32, 8, 8, 4096, 128));
-    EXPECT(tiled(1, 32, 8, 4, 8192, 128) && tiled(1, 32, 8, 2, 32768, 128));
-    EXPECT(tiled(1, 28, 4, 2, 4096, 128));    // 36.6, 15.6: three launches on the split kernel
-    EXPECT(tiled(1, 28, 4, 3, 8192, 128));    // 40.5, 18.6
-    EXPECT(tiled(16, 28, 4, 1, 4096, 128));
+    EXPECT(!tiled(1, 32, 8, 8, 4096, 128)); // (5 us slower on the split kernel, whose probabilities are floats)
+    EXPECT(tiled(1, 32, 8, 16, 4096, 128) && tiled(1, 32, 8, 8, 8192, 128));
+    EXPECT(tiled(16, 28, 4, 1, 4096, 128)); // three launches on the split kernel
     // without room for records, other head dims: the rule for items that walk all of their keys
-    EXPECT(!rg::prefill_pays(1, 32, 8, 4, 4096, 128, false) && !tiled(1, 32, 8, 4, 4096, 96) && tiled(32, 32, 8, 2, 4096, 96));
+    EXPECT(!rg::prefill_pays(1, 32, 8, 4, 4096, 128, false) && !tiled(1, 32, 8, 4, 4096, 96) && tiled(32, 32, 8, 16, 4096, 96));
 }
 
 static void shapeDigests() {
