@@ -200,8 +200,8 @@ inline IntegerRoute integer_route(size_t m, size_t k, size_t n, size_t count, bo
 
 // ---------------------------------------------------------------- F32
 //
-// Fitted over 2,500 products of 1 to 256 rows, k 64 to 8320, 16 to 50257 columns; over them the choice takes 0.06 % longer
-// than the faster kernel of each call.
+// Fitted over 2,500 products of 1 to 256 rows, k 64 to 8320, 16 to 50257 columns: the cheaper one by these costs takes 0.06 %
+// longer than the faster kernel of each call.
 
 // mm_rows (B as [n, k]) and mm_rows_kn (B as [k, n]): passes of up to 32 rows, a workgroup per 16 columns.  A round is 256
 // workgroups; passes of more than 16 rows go in whole rounds (one wavefront per SIMD).
@@ -228,23 +228,21 @@ inline double f32_tiles_us(size_t m, size_t k, size_t n, size_t count) {
     return 3.7 + 1e-3 * static_cast<double>(k) * (12.6 + 62.0 * static_cast<double>((tiles + 255) / 256)) + 2.46 * static_cast<double>(tiles) / 256;
 }
 
-// mm_generic, up to 16 rows: its own chain of steps through k, or the elements of B.
-inline double f32_plain_us(size_t k, size_t n, size_t count) {
-    const double chain = 28e-3 * static_cast<double>(k), work = 2.84e-6 * static_cast<double>(k) * static_cast<double>(n) * static_cast<double>(count);
-    return 1.6 + (chain > work ? chain : work);
-}
-
 enum class F32Route { rows, tiles, plain };
 
 // rows_ok, tiles_ok: the kernels take these operands.  Up to eight rows the tiles, which do the work of 128, are not
-// considered: the passes end first from k = 128 on ([8, 4096] x [50257, 4096]^T 151 us in a pass, 536 on the tiles, 545 on
-// the plain kernel), the plain kernel below that.
+// launched and so not weighed either ([8, 4096] x [50257, 4096]^T 151 us in a pass, 545 on the plain kernel).  Beyond, the passes
+// where they are expected to end first, and where they lose little: their sums are 16 partial sums of k each, a tile's are one
+// chain (0.9e-7 and 4e-7 from 64 bits at k = 512), so the tiles have to win on costs that flatter the passes too (27 us for 32 rows
+// against 4096 x 4096, 300 us for up to 768 tiles at k = 4096).
 inline F32Route f32_route(size_t m, size_t k, size_t n, size_t count, bool b_is_nk, bool rows_ok, bool tiles_ok) {
-    const double rows = rows_ok ? f32_rows_us(m, k, n, count, b_is_nk) : 1e30;
-    if (m <= 8) return rows <= f32_plain_us(k, n, count) ? F32Route::rows : F32Route::plain;
-    const double tiles = tiles_ok ? f32_tiles_us(m, k, n, count) : 1e30;
-    if (!rows_ok && !tiles_ok) return F32Route::plain;
-    return rows <= tiles ? F32Route::rows : F32Route::tiles;
+    if (m <= 8) return rows_ok ? F32Route::rows : F32Route::plain;
+    if (!rows_ok) return tiles_ok ? F32Route::tiles : F32Route::plain;
+    if (!tiles_ok || f32_rows_us(m, k, n, count, b_is_nk) <= f32_tiles_us(m, k, n, count)) return F32Route::rows;
+    const double weights = static_cast<double>(n) / 4096 * static_cast<double>(k) / 4096;
+    const double tiles = static_cast<double>(((m + 127) / 128) * ((n + 127) / 128));
+    const double passes = static_cast<double>((m + 31) / 32) * (3.0 + (b_is_nk ? 27.0 : 33.0) * weights);
+    return passes <= 3.0 + 300.0 * static_cast<double>(k) / 4096 * static_cast<double>((static_cast<uint64_t>(tiles) + 767) / 768) ? F32Route::rows : F32Route::tiles;
 }
 
 }  // namespace rg

@@ -129,12 +129,13 @@ static void productPlanF32() {
     EXPECT(nk(64, 128, 4096) == R::rows);   // 8.8, 14.7
     EXPECT(nk(256, 4096, 4096) == R::rows); // 232, 307
     EXPECT(kn(128, 512, 4096) == R::rows);  // 28, 43
-    EXPECT(nk(64, 64, 5833) == R::tiles);   // 14.4, 9.9
-    EXPECT(nk(128, 512, 5833) == R::tiles); // 49.2, 43.5
     EXPECT(nk(128, 1024, 50257) == R::tiles);// 477, 146
-    EXPECT(kn(17, 128, 32000) == R::tiles); // 34.8, 14.4
-    // a k so short that a pass is all overhead; operands that a kernel does not take
-    EXPECT(nk(8, 64, 32000) == R::plain);   // 10.9, (8.5), 7.0
+    EXPECT(nk(128, 768, 11008) == R::tiles);
+    // close calls stay with the passes, which round less
+    EXPECT(nk(64, 64, 5833) == R::rows);    // 14.4, 9.9
+    EXPECT(kn(17, 128, 32000) == R::rows);  // 34.8, 14.4
+    EXPECT(nk(8, 64, 32000) == R::rows);    // 10.9, (8.5), 7.0
+    // operands that a kernel does not take
     EXPECT(rg::f32_route(8, 4096, 4096, 1, false, false, true) == R::plain);
     EXPECT(rg::f32_route(9, 4096, 4096, 1, false, false, true) == R::tiles);
     EXPECT(rg::f32_route(9, 4096, 4096, 1, true, true, false) == R::rows);
