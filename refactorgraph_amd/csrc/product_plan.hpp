@@ -82,8 +82,14 @@ inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t count, bool rough
 }
 
 // Up to 32 rows on the kernels that read the weights once, columns of all products side by side: mm_skinny (B as [n, k]) and
-// a pass of mm_rows_kn (B as [k, n]).  Beyond 32 rows neither ended before the tiles at any size.  Where the choice is
-// between these and the tiles it takes 0.3 % longer than the faster one on average.
+// a pass of mm_rows_kn (B as [k, n]).  With the weights in the caches, as the fit has them, the choice between these and the
+// tiles takes 0.3 % longer than the faster one on average, and beyond 32 rows neither ended before the tiles at any size.
+// With weights from memory the tiles, which wait for each step's copies, take up to 1.6 times as long and the few-rows kernels
+// about what they took: there the rule takes 0.2 % (mm_skinny), 1 % (up to 8 rows of mm_rows_kn) and 3.6 % (9 to 16 rows, whose
+// cost is 0.3 us per 1000 of k below the fit for this) longer.  33 to 64 rows stay on the tiles: two slabs of mm_skinny took
+// 40 us against 53 from memory and 39 against 32 from the caches ([64, 11008] x [1024, 11008]^T), 20 and 22, 19 and 14.5 at
+// [64, 4096] x [4096, 4096]^T; over k from 3072 and 512 to 6144 columns they take 7 % longer than the faster kernel from
+// memory and 31 % from the caches, the tiles 10 % and nothing.
 inline double skinny_us(size_t k, size_t columns) {
     const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
     return 1.5 + 0.74 * kilo + 0.3 * kilo * wide + 0.21 * wide;
@@ -91,8 +97,7 @@ inline double skinny_us(size_t k, size_t columns) {
 inline double rows_kn_us(size_t m, size_t k, size_t columns) {
     const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
     if (m <= 8) return 0.9 + 1.64 * kilo + 0.32 * kilo * wide + 0.28 * wide;
-    if (m <= 16) return 2.9 + 1.64 * kilo + 0.334 * kilo * wide + 0.15 * wide;
-    return 5.35 + 1.9 * kilo + 0.57 * kilo * wide + 0.135 * wide;
+    return 2.9 + 1.33 * kilo + 0.334 * kilo * wide + 0.15 * wide;  // (9 to 16 rows)
 }
 // A pass of four rows of mm_gemv_kn: a workgroup's chain through k, or B at what 16-byte pieces of its rows come in at.
 inline double gemv_kn_us(size_t m, size_t k, size_t columns) {
@@ -127,6 +132,9 @@ inline HalfRoute half_route(size_t m, size_t k, size_t n, size_t count, bool b_i
         if (can.gemv) return HalfRoute::gemv;
         if (can.skinny) return can.ring && ring_us() < skinny_us(k, columns) ? HalfRoute::tiles : HalfRoute::skinny;
     } else {
+        // (17 rows and more: the tiles take 1.7 % longer than the faster kernel on average, from the caches as from memory;
+        // a choice by a cost fitted like those above took 3.5 %)
+        if (can.rows_kn && can.ring && m > 16) return HalfRoute::tiles;
         if (can.rows_kn) return can.ring && ring_us() < rows_kn_us(m, k, columns) ? HalfRoute::tiles : HalfRoute::rows_kn;
         if (can.gemv_kn) {
             // (a second pass of four rows never ended before the tiles: [5, 4096] x [4096, 1000] 34 us, 14 on mm_ring)
