@@ -51,7 +51,7 @@ MEASURED_TRAFFIC = {
     "matmul_integer": (2 * 50313 + 65560) * 1024,
     "attention_prefill": (2 * 110058 + 196608) * 1024,
     "cast": (2 * 32784 + 32768) * 1024,
-    "matmul": (2 * 98778 + 33024) * 1024,
+    "matmul": (2 * 147666 + 32790) * 1024,
     "matmul_few_rows": (2 * 17456 + 256) * 1024,
     "matmul_eight_rows": (2 * 16661 + 64) * 1024,
     "dequantize_linear_i32": (2 * 32869 + 65611) * 1024,

@@ -27,8 +27,9 @@ for _name, _code in (("uint16", abi.U16), ("uint32", abi.U32), ("uint64", abi.U6
 
 
 # A call's host work is what a decode step of one sequence waits for (seven calls of 13 us each against 40 us of kernels
-# before): addresses go to ctypes as integers, what depends on shapes alone is worked out once per shape (bounded caches of
-# pure functions), two-dimensional products skip the broadcasting of batches.
+# before): addresses go to ctypes as integers, what depends on shapes alone (MatMul's workspace: and on the device's CUs, the
+# same for all devices of a box; too small a workspace is not used) is worked out once per shape, in bounded caches,
+# two-dimensional products skip the broadcasting of batches.
 
 def _stream():
     """Address of torch's current stream of the current device."""
