@@ -50,7 +50,7 @@ struct RingPlan {
 
 // One shape for the whole product, or whole rounds of one shape and another one for the columns that are left: 344 tiles of
 // 256 x 256 ([2048, 4096] x [4096, 11008]) would be a full round and one with two thirds of the CUs idle (208 us); a full
-// round over 8192 columns and 240 tiles of 128 x 192 behind it take 167 us.  Over the sizes above the plan takes 0.9 %
+// round over 8192 columns and 240 tiles of 128 x 192 behind it take 171 us.  Over the sizes above the plan takes 0.9 %
 // longer than the fastest shape of each product.
 inline RingPlan ring_plan(size_t m, size_t k, size_t n, size_t count, bool rough_stores) {
     RingPlan best{0, 0, 0, 1e30};
@@ -132,9 +132,14 @@ inline HalfRoute half_route(size_t m, size_t k, size_t n, size_t count, bool b_i
         if (can.gemv) return HalfRoute::gemv;
         if (can.skinny) return can.ring && ring_us() < skinny_us(k, columns) ? HalfRoute::tiles : HalfRoute::skinny;
     } else {
-        // (17 rows and more: the tiles take 1.7 % longer than the faster kernel on average, from the caches as from memory;
-        // a choice by a cost fitted like those above took 3.5 %)
-        if (can.rows_kn && can.ring && m > 16) return HalfRoute::tiles;
+        // 17 rows and more: the tiles, unless the columns are whole groups of 32 workgroups (an XCD then has whole 128-byte
+        // pieces of B's k-rows) and few, and B fits the L2s: over 75 such calls the tiles take 1.14 times as long from memory
+        // and 1.10 times from the caches ([17, 11008] x [11008, 1024] 52 and 42 us, 31 and 24).  Elsewhere the passes win up to
+        // 20 % from memory and lose more from the caches ([24, 4096] x [4096, 768] level, 1.45 times the tiles' time).
+        if (can.rows_kn && m > 16) {
+            const bool few = count == 1 && n % 512 == 0 && n <= 2048 && static_cast<uint64_t>(k) * n <= 12u << 20;
+            return can.ring && !few ? HalfRoute::tiles : HalfRoute::rows_kn;
+        }
         if (can.rows_kn) return can.ring && ring_us() < rows_kn_us(m, k, columns) ? HalfRoute::tiles : HalfRoute::rows_kn;
         if (can.gemv_kn) {
             // (a second pass of four rows never ended before the tiles: [5, 4096] x [4096, 1000] 34 us, 14 on mm_ring)
