@@ -94,10 +94,13 @@ inline double skinny_us(size_t k, size_t columns) {
     const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
     return 1.5 + 0.74 * kilo + 0.3 * kilo * wide + 0.21 * wide;
 }
-inline double rows_kn_us(size_t m, size_t k, size_t columns) {
-    const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(columns);
-    if (m <= 8) return 0.9 + 1.64 * kilo + 0.32 * kilo * wide + 0.28 * wide;
-    return 2.9 + 1.33 * kilo + 0.334 * kilo * wide + 0.15 * wide;  // (9 to 16 rows)
+inline double rows_kn_us(size_t m, size_t k, size_t n, size_t count) {
+    const double kilo = 1e-3 * static_cast<double>(k), wide = 1e-3 * static_cast<double>(n * count);
+    // (one product: beyond a workgroup per CU a second round walks k again, [8, 2048] x [2048, 6144] 16.6 us, 13.5 on mm_ring)
+    const size_t strips = n % 32 == 0 && n >= 8192 ? n / 32 : (n + 15) / 16;
+    const double again = count == 1 ? 0.6 * kilo * static_cast<double>((strips - 1) / kPlanCus) : 0;
+    if (m <= 8) return 0.9 + 1.64 * kilo + 0.32 * kilo * wide + 0.28 * wide + again;
+    return 2.9 + 1.33 * kilo + 0.334 * kilo * wide + 0.15 * wide + again;  // (9 to 16 rows)
 }
 // A pass of four rows of mm_gemv_kn: a workgroup's chain through k, or B at what 16-byte pieces of its rows come in at.
 inline double gemv_kn_us(size_t m, size_t k, size_t columns) {
@@ -140,7 +143,7 @@ inline HalfRoute half_route(size_t m, size_t k, size_t n, size_t count, bool b_i
             const bool few = count == 1 && n % 512 == 0 && n <= 2048 && static_cast<uint64_t>(k) * n <= 12u << 20;
             return can.ring && !few ? HalfRoute::tiles : HalfRoute::rows_kn;
         }
-        if (can.rows_kn) return can.ring && ring_us() < rows_kn_us(m, k, columns) ? HalfRoute::tiles : HalfRoute::rows_kn;
+        if (can.rows_kn) return can.ring && ring_us() < rows_kn_us(m, k, n, count) ? HalfRoute::tiles : HalfRoute::rows_kn;
         if (can.gemv_kn) {
             // (a second pass of four rows never ended before the tiles: [5, 4096] x [4096, 1000] 34 us, 14 on mm_ring)
             if (m <= 4) return HalfRoute::gemv_kn;

@@ -182,6 +182,7 @@ static void productPlanHalf() {
     EXPECT(kn(1, 17, 8192, 1024) == R::rows_kn && kn(1, 32, 4096, 2048) == R::rows_kn); // whole 128-byte pieces an XCD, B in the L2s
     EXPECT(kn(1, 17, 4096, 768) == R::tiles && kn(1, 17, 11008, 2048) == R::tiles && kn(1, 17, 4096, 4096) == R::tiles);
     EXPECT(kn(2, 17, 8192, 1024) == R::tiles);
+    EXPECT(kn(1, 8, 2048, 6144) == R::tiles && kn(1, 8, 2048, 4096) == R::rows_kn); // a second round of workgroups: 16.6, 13.5
     EXPECT(kn(1, 32, 4096, 4096) == R::tiles);  // 18, 14
     EXPECT(kn(256, 8, 512, 1024) == R::tiles);  // 120, 53
     EXPECT(nk(1, 16, 4096, 11008) == R::rows && nk(1, 1, 4096, 11008) == R::gemv);
