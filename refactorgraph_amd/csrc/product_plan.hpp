@@ -38,9 +38,10 @@ constexpr TileShape kRingShapes[] = {{64, 64, 2.7, 145, 300},   {64, 128, 3.4, 2
                                      {128, 192, 6, 370, 800}, {128, 256, 7.2, 580, 888}, {256, 256, 12.2, 920, 1525}};
 constexpr int kRingShapeCount = 6;
 constexpr double kRingLaunchUs = 1.0;
-// the 256 x 256 tiles store element by element where rows of the output are no whole 16-byte words (16 products
-// [512, 64] x [4099, 64]^T with a bias per output 129 us, 128 x 128 tiles 82); the smaller tiles hide that
-constexpr double kRoughStoresUs = 4.7;
+// the 256 x 256 tiles store element by element where rows of the output are no whole 16-byte words; the smaller tiles hide that.
+// Over 451 products with such rows the plan takes 0.3 % longer than the fastest shape (0.9 with nothing here, 1.8 with 4.7 us:
+// 256 products [256, 512] x [1001, 512]^T 149 us on these tiles, 175 on 128 x 256; 16 of [512, 64] x [4099, 64]^T 45 and 42)
+constexpr double kRoughStoresUs = 1.5;
 
 struct RingPlan {
     int first, rest;   // shape of the first `columns` columns and of those behind them

@@ -215,6 +215,7 @@ static void productPlanRing() {
     }
     // element-wise stores: the largest tiles give way (16 products [512, 64] x [4099, 64]^T)
     EXPECT(rg::ring_plan(512, 64, 4096, 16, false).rest == 5 && rg::ring_plan(512, 64, 4099, 16, true).rest < 5);
+    EXPECT(rg::ring_plan(256, 512, 1001, 256, true).rest == 5 && rg::ring_plan(512, 256, 1001, 32, true).rest == 5); // 149, 175; 27, 33
 }
 
 static void productPlanInteger() {
