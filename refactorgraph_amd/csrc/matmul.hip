@@ -1891,8 +1891,10 @@ inline KnSplitPlan kn_mfma_split_plan(size_t k, size_t n) {
     // while the other's copies arrive ([16, 4096] x [4096, 6144] 21.4 -> 19.2 us, 11008 columns 32.1 -> 29.7; where one round
     // of whole shares suffices halves only add sums to be exchanged, 4096 columns 13.1 -> 14.2; so they do where a share is
     // all of k: [8, 760] x [760, 20480] 9.0 us whole, 12.1 in halves, [24, 1024] x [1024, 128000] 67 and 82; and, without a
-    // reason found, where k-rows lie a multiple of 128 KiB apart: [16, 4096] x [4096, 65536] 169 and 182, 131072 columns 344 and 372)
-    if (p.shares > 1 && n % 65536 != 0 && p.strips * p.shares > static_cast<uint32_t>(cus) && kr > KM_MAX_KR / 2 && p.shares <= 127) {
+    // reason found, where k-rows lie a multiple of 128 KiB apart and k is three whole shares or more: [16, 4096] x [4096, 65536]
+    // 164 and 177, 131072 columns 339 and 361; a short last share weighs more than that, [16, 1280] x [1280, 65536] 69 and 59)
+    const bool whole = n % 65536 == 0 && k % KM_MAX_KR == 0 && p.shares >= 3;
+    if (p.shares > 1 && !whole && p.strips * p.shares > static_cast<uint32_t>(cus) && kr > KM_MAX_KR / 2 && p.shares <= 127) {
         kr = KM_MAX_KR / 2;
         p.shares = static_cast<uint32_t>((k + kr - 1) / kr);
     }

@@ -48,6 +48,7 @@ def test_error_strings_and_workspace_queries_need_no_gpu():
 @pytest.mark.parametrize("m,k,n,shares", [
     (8, 760, 20480, 1), (16, 1024, 128000, 1), (32, 1024, 32000, 1),      # a share is all of k: nothing to exchange
     (16, 4096, 65536, 4), (5, 3072, 131072, 3),                           # k-rows a multiple of 128 KiB apart
+    (16, 1280, 65536, 3), (32, 2048, 65536, 4), (5, 1536, 131072, 3),     # the same, a short last share or two whole ones: half shares
     (16, 4096, 4096, 4),                                                  # whole shares fill one round of CUs
     (16, 4096, 6144, 8), (16, 4096, 11008, 8), (5, 1536, 32000, 3)])      # more workgroups than CUs: half shares
 def test_matmul_workspace_holds_the_shares_of_k_the_launch_takes(m, k, n, shares):
