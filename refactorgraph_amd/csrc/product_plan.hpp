@@ -197,10 +197,14 @@ inline double integer_skinny_us(size_t m, size_t k, size_t n, size_t count, bool
 }
 
 // What a step of mmi_ring takes longer with weights from memory instead of the caches is 0.1 to 0.24 us; mmi_skinny takes the
-// same.  The fits have the caches, so one product's tiles are charged a part of that which serves both: 1 % longer than the faster
-// kernel from the caches as from memory (nothing charged: 0.8 and 2.6 %, twice the time at worst; [33, 11008] x [11008, 6144]
+// same.  The fits have the caches, so one product's tiles are charged a part of that which serves both kinds of call, where B
+// is large (a small one stays in the caches) and mmi_skinny's workgroups have few columns (11008: level from memory, 1.3 times
+// the tiles' time from the caches).  Over 1,820 products of 5 to 128 rows the choice takes 1.5 % longer than the faster kernel
+// from memory and 1.1 % from the caches (nothing charged: 2.3 and 0.9 %, twice the time at worst; [33, 11008] x [11008, 6144]
 // 51 us on the tiles, 26 on mmi_skinny).
-inline double integer_from_memory_us(size_t m, double steps) { return steps * (m <= 32 ? 0.02 : 0.07); }
+inline double integer_from_memory_us(size_t m, size_t k, size_t n, double steps) {
+    return static_cast<uint64_t>(k) * n >= 8u << 20 && n <= 6144 ? steps * (m <= 32 ? 0.02 : 0.07) : 0;
+}
 
 struct IntegerRoute {
     enum { ring, large, skinny } kernel;
@@ -217,7 +221,7 @@ inline IntegerRoute integer_route(size_t m, size_t k, size_t n, size_t count, bo
         if (t < us) us = t, best = {IntegerRoute::ring, i};
     }
     if (large_ok && 0.4 + tiles_us(kIntegerLargeShape, tile_count(kIntegerLargeShape, m, n, count), steps) < us) return {IntegerRoute::large, 0};
-    if (count == 1) us += integer_from_memory_us(m, steps);
+    if (count == 1) us += integer_from_memory_us(m, k, n, steps);
     if (skinny_ok && integer_skinny_us(m, k, n, count, dequantize) < us) return {IntegerRoute::skinny, 0};
     return best;
 }

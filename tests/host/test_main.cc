@@ -236,6 +236,7 @@ static void productPlanInteger() {
     // the ring a little ahead with B in the caches, far behind with B from memory (13.8, 13.4; 14.4, 21)
     EXPECT(route(1, 32, 4096, 6144, false) == R::skinny);
     EXPECT(route(1, 33, 11008, 6144, true) == R::skinny && route(1, 64, 8192, 4096, true) == R::skinny); // 26, 51; 24, 39
+    EXPECT(route(1, 64, 2048, 256, true) == 10);           // 10.2, 8.9
     EXPECT(route(1, 32, 4096, 11008, true) == 10 && route(1, 64, 4096, 4096, true) == 10);
     EXPECT(route(1, 129, 11008, 256, false) == 10);
     EXPECT((rg::integer_skinny_shares(4096, 4096, 1).tiles == 2 && rg::integer_skinny_shares(4096, 4096, 1).shares == 16));
