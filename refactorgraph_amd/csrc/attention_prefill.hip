@@ -96,9 +96,11 @@ template <> struct Ops<__hip_bfloat16> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
     }
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-        const uint32_t l = __builtin_bit_cast(uint16_t, __float2bfloat16(lo));
-        const uint32_t h = __builtin_bit_cast(uint16_t, __float2bfloat16(hi));
-        return l | (h << 16);
+        // one conversion of the pair, nearest, ties to even (two conversions, a shift and an or before: [2, 799 rows, 32/8 heads]
+        // 29.9 -> 28.4 us, 5 x 521 rows 31.2 -> 28.8)
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, b2));
     }
     static __device__ __forceinline__ float add_pair(float sum, uint32_t, float p0, float p1) { return sum + (p0 + p1); }
 };
