@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 
 namespace rg {
 
@@ -39,6 +40,39 @@ inline bool prefill_pays(size_t N, size_t n_head, size_t n_kv_head, size_t seq, 
     }
     const size_t rounds = (items + 511) / 512;
     return N * n_kv_head * seq * split_launches >= 280 * rounds;
+}
+
+// ---------------------------------------------------------------- the tiled kernels: keys shared between workgroups
+constexpr uint64_t kSplitMinTiles = 8;  // key tiles (of 64) of the capacity per range of shared keys, at least
+constexpr uint64_t kSplitMax = 32;      // ranges per item, at most
+
+// Ranges per item of a launch of attn_prefill_wide: as many as bring it to a workgroup per CU, while the records (`room` of
+// them, of an item and range) fit the workspace.
+inline uint64_t wide_splits(uint64_t items, uint64_t cap, uint64_t cus, uint64_t room) {
+    uint64_t splits = items ? cus / items : 1;
+    const uint64_t by_tiles = (cap + 63) / 64 / kSplitMinTiles, by_room = items ? room / items : 0;
+    if (splits > by_tiles) splits = by_tiles;
+    if (splits > kSplitMax) splits = kSplitMax;
+    if (splits > by_room) splits = by_room;
+    return splits < 2 ? 1 : splits;
+}
+
+// attn_prefill_wide (64 query rows a wavefront, one wavefront on a SIMD) instead of attn_prefill (32 rows, two), head dim 128:
+// its steady state is the faster one, but nobody works on a SIMD while its wavefront changes items.  Measured over 60 calls,
+// time of attn_prefill over its time:
+//   whole items, 1024 and more of 1536 and more rows: 1.06 to 1.21 ([4, 32/8 heads, 2048 rows] 162 and 153 us, 56/8 heads 291 and
+//   240); of 1024 rows 0.95 to 1.1, fewer or shorter ones down to 0.77 (512 items of 256 rows 24 and 30 us);
+//   shared keys, 20 and more tiles to a range: 1.01 to 1.19 (128 rows behind 16384 positions 52 and 48 us, 512 behind 8000 93 and
+//   78); at 4 to 16 tiles 0.75 to 1.08.  The capacity stands for the history, which is device data.
+//   Where more than a quarter of the rows of the items is padding (77 rows: 0.87), and for groups of one and two heads, whose
+//   items are 256 and 128 rows (0.61 to 0.95), never.
+inline bool wide_pays(uint64_t N, uint64_t n_head, uint64_t n_kv_head, uint64_t seq, uint64_t cap, uint64_t cus, uint64_t room) {
+    const uint64_t group = n_head / n_kv_head, q_tiles = (seq + 63) / 64;
+    if (group < 3 || 4 * seq < 3 * 64 * q_tiles) return false;
+    const uint64_t items = N * n_kv_head * ((group + 3) / 4) * q_tiles;
+    const uint64_t splits = wide_splits(items, cap, cus, room);
+    if (splits == 1) return seq >= 1536 && items >= 4 * cus;
+    return (cap + 63) / 64 >= 20 * splits;
 }
 
 }  // namespace rg

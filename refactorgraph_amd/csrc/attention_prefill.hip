@@ -33,6 +33,10 @@
 // the query tiles of a stream share in that XCD's L2.
 #include "attention_prefill.hpp"
 
+#include "attention_plan.hpp"
+
+#include <utility>
+
 namespace rg {
 namespace {
 
@@ -50,8 +54,6 @@ constexpr int TILE = BN * ROWB;        // 16384: one K or V tile
 constexpr int BUF_BYTES = 2 * TILE;    // K tile + V tile; two such buffers, reused for the output transposition
 constexpr float kSlack = 6.0f;
 constexpr float kMinusBig = -1e30f;
-constexpr uint64_t kSplitMinTiles = 8;  // key tiles of the capacity per range of a SPLIT launch, at least
-constexpr uint64_t kSplitMax = 32;      // ranges per item, at most
 
 // LDS layout of a tile: the 16-byte chunk c of K row r sits at chunk position c ^ (r & 15), which
 // puts the 128-bit fragment reads of 8 or 16 consecutive rows on distinct banks; chunk c of V row r
@@ -104,6 +106,28 @@ template <> struct Ops<__hip_bfloat16> {
     }
     static __device__ __forceinline__ float add_pair(float sum, uint32_t, float p0, float p1) { return sum + (p0 + p1); }
 };
+
+// The same products with everything about registers said: results, V and P in vector registers, K and Q in accumulation
+// registers (left to itself the compiler keeps S^T and O^T of attn_prefill_wide in accumulation registers, copies them for every
+// use by the vector ALU and spills).  The compiler does not know that these are products and adds no wait states around them: see
+// the phases of attn_prefill_wide.
+typedef uint32_t Frag __attribute__((ext_vector_type(4)));
+template <class T> struct OpsAsm;
+#define RG_PRODUCTS(TYPE, NAME)                                                                                            \
+    template <> struct OpsAsm<TYPE> {                                                                                      \
+        static __device__ __forceinline__ void scores_first(f16v &c, const Frag &k, const Frag &q) {                       \
+            asm volatile(NAME " %0, %1, %2, 0" : "=&v"(c) : "a"(k), "a"(q));                                               \
+        }                                                                                                                  \
+        static __device__ __forceinline__ void scores(f16v &c, const Frag &k, const Frag &q) {                             \
+            asm volatile(NAME " %0, %1, %2, %0" : "+v"(c) : "a"(k), "a"(q));                                               \
+        }                                                                                                                  \
+        static __device__ __forceinline__ void output(f16v &c, const Frag &v, const Frag &p) {                             \
+            asm volatile(NAME " %0, %1, %2, %0" : "+v"(c) : "v"(v), "v"(p));                                               \
+        }                                                                                                                  \
+    };
+RG_PRODUCTS(__half, "v_mfma_f32_32x32x16_f16")
+RG_PRODUCTS(__hip_bfloat16, "v_mfma_f32_32x32x16_bf16")
+#undef RG_PRODUCTS
 
 // Sum and maximum over the two half-wavefronts (lanes i and i + 32), on the vector ALU.
 struct HalfPair {
@@ -776,14 +800,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
 // (eight registers, half the workgroups: 10.6 against 7.5 us for 32 items of 16 ranges; many items of few ranges would rather
 // have more: 256 items of two 10.9 us with four, 10.3 with eight, 10.0 with sixteen)
 constexpr int kMergeRegs = 4;
-template <class T, int HW, int DH>
+template <class T, int HW, int DH, int SUB>  // SUB: sub-tiles of 32 rows per wavefront of an item
 __global__ __launch_bounds__(256) void attn_prefill_merge(const PrefillArgs a, const PrefillPlan plan) {
-    constexpr int QS = 4 / HW, ROWS = 32 * QS, DBLK = (DH + 31) / 32;
+    constexpr int QS = 4 / HW, ROWS = 32 * QS * SUB, DBLK = (DH + 31) / 32;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
-    const uint32_t qt = blockIdx.x % plan.q_tiles, stream = blockIdx.x / plan.q_tiles;
+    const uint32_t item = blockIdx.x / SUB, qt = item % plan.q_tiles, stream = item / plan.q_tiles;
     const uint32_t kvhead = stream / plan.head_chunks, hc = stream % plan.head_chunks;
     const uint32_t h = hc * HW + wave % HW;
-    const uint32_t fr0 = qt * ROWS + 32 * (wave / HW);
+    const uint32_t fr0 = qt * ROWS + 32 * SUB * (wave / HW) + 32 * (blockIdx.x % SUB);
     if (h >= plan.group || fr0 >= a.seq) return;  // (whole wavefronts)
     const float *rec = plan.part + static_cast<uint64_t>(blockIdx.x) * plan.splits * part_floats(DH);
     const uint32_t e0 = blockIdx.y * kMergeRegs;
@@ -812,6 +836,466 @@ __global__ __launch_bounds__(256) void attn_prefill_merge(const PrefillArgs a, c
         if (d >= DH) continue;  // (head dim 80: the second half of the last block)
         const uint2 w = make_uint2(Ops<T>::pack2(o[4 * gg] * inv, o[4 * gg + 1] * inv), Ops<T>::pack2(o[4 * gg + 2] * inv, o[4 * gg + 3] * inv));
         *reinterpret_cast<uint2 *>(out + d) = w;
+    }
+}
+
+// ---------------------------------------------------------------- 64 query rows per wavefront, head dim 128
+//
+// The same items, layouts and arithmetic, with twice the query rows: a wavefront owns two sub-tiles of 32 consecutive rows, so
+// that every K and V fragment read from LDS feeds two products, and one wavefront runs on a SIMD (O^T of 64 rows alone takes
+// 128 registers).  With nobody else on the SIMD the wavefront overlaps its own products with its own softmax: the sub-tiles
+// run half a period apart, in phases of sixteen products (S^T of the next block and O^T of the present one) of one sub-tile,
+// each product followed by a sixteenth of the other sub-tile's softmax:
+//     phase 0 of block j: S0(j + 1), O0 += V(j) P0(j)  beside the softmax of S1(j)
+//     phase 1 of block j: S1(j + 1), O1 += V(j) P1(j)  beside the softmax of S0(j + 1); K(j + 2) and V(j + 1) are read
+// Key tiles of 64 go through a ring of WNS stages of LDS that runs across the items: at the barrier ahead of tile c, tile
+// c + 1 has landed and nobody reads tile c - 1 any more (what is read of a tile is consumed by products ahead of the next
+// barrier), whose stage takes tile c + WNS - 1.  The query rows are loaded into registers under the last block of the item
+// before and pass through LDS of the wavefront's own into operand layout, as the output does on its way out, so that both cross
+// memory in whole rows.
+// What bounds it (128 bf16 rows, 32/8 heads, behind 16384 positions: 37 us beside 8 of the merge, 45 with 32 rows a wavefront;
+// 77 k clocks of a wavefront): its products occupy the matrix pipe for 33 k, its vector instructions the issue for 30 k, and as
+// the two overlap by half only, the rest are waits of the one wavefront.  A product takes 32 clocks of the matrix pipe and 8 of
+// the issue, an exponential 8, other vector instructions 4; a branch that is taken costs about as much as a product, so the
+// loop has none but the rare ones (mask, raised reference) and copies are made with no lane active instead of being skipped.
+constexpr int WNS = 4;                 // stages of the ring
+constexpr int WROWB = 256;             // bytes of a row: head dim 128
+constexpr int WSTAGE = 2 * BN * WROWB; // K tile, V tile
+template <class T, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void attn_prefill_wide(const PrefillArgs a, const PrefillPlan plan) {
+    constexpr int ROWS = 64, HW = 4, DBLK = 4, KSTEPS = 8, TILE_B = BN * WROWB;
+    __shared__ __align__(1024) uint8_t lds[WNS * WSTAGE + 4 * 32 * WROWB];
+    const uint32_t lds_addr0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
+    const uint32_t tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31, wave = uni(tid >> 6);
+    const uint32_t xcd = uni(blockIdx.x % plan.xcds), lw = uni(blockIdx.x / plan.xcds);
+    const uint32_t pj = uni(lw % plan.pairs), set = uni(lw / plan.pairs);
+
+    // Item i of this workgroup (the dealing of attn_prefill in closed form).
+    auto item_at = [&](uint32_t i) __attribute__((always_inline)) -> Item {
+        Item it{0, 0, kNoItem, 0, 0};
+        const uint32_t heavy = plan.q_tiles - 1 - pj;
+        const bool one = SPLIT || pj == heavy;  // one query tile of a stream, not two
+        const uint32_t en = set + plan.groups * (one ? i : i >> 1);
+        if (en >= plan.spx) return it;
+        uint32_t stream = en * plan.xcds + xcd;
+        if constexpr (SPLIT) {
+            const uint32_t whole = div_magic(stream, plan.magic_splits);
+            it.ks = stream - whole * plan.splits;
+            stream = whole;
+        }
+        it.qt = SPLIT ? ((set & 1) ? heavy : pj) : (i & 1) && !one ? pj : heavy;
+        it.kvhead = div_magic(stream, plan.magic_chunks);
+        it.hc = stream - it.kvhead * plan.head_chunks;
+        if (a.kc && a.past) {
+            // (a scalar load: a vector one would be waited for together with every copy in flight)
+            typedef const __attribute__((address_space(4))) uint32_t ScalarWord;
+            ScalarWord *p = reinterpret_cast<ScalarWord *>(reinterpret_cast<uintptr_t>(a.past + (a.past_per_row ? div_magic(it.kvhead, plan.magic_hkv) : 0)));
+            const uint32_t lo = uni(p[0]), hi = uni(p[1]);
+            const uint32_t room = a.cap > a.seq ? a.cap - a.seq : 0;
+            const uint32_t len = hi == 0 ? lo : (hi >> 31 ? 0u : room);
+            it.base = len < room ? len : room;
+        }
+        return it;
+    };
+    // key tiles [first, end) of an item that this workgroup walks; dummy: its range is empty, tile 0 is walked with every key masked
+    auto key_range = [&](const Item &it, uint32_t &first, uint32_t &end, bool &dummy, bool &last) __attribute__((always_inline)) {
+        const uint32_t rows_end = (it.qt + 1) * ROWS < a.seq ? (it.qt + 1) * ROWS : a.seq;
+        const uint32_t tiles = uni((it.base + rows_end - 1) / BN + 1);
+        first = 0;
+        end = tiles;
+        dummy = false;
+        if constexpr (SPLIT) {
+            const uint32_t share = div_magic(tiles + plan.splits - 1, plan.magic_splits);
+            first = it.ks * share;
+            if (first >= tiles) {
+                first = 0;
+                end = 1;
+                dummy = true;
+            } else {
+                end = first + share < tiles ? first + share : tiles;
+            }
+        }
+        last = !dummy && end == tiles;
+    };
+
+    const uint8_t *Q = static_cast<const uint8_t *>(a.q);
+    const uint8_t *Kn = static_cast<const uint8_t *>(a.k);
+    const uint8_t *Vn = static_cast<const uint8_t *>(a.v);
+    uint8_t *Kc = static_cast<uint8_t *>(a.kc);
+    uint8_t *Vc = static_cast<uint8_t *>(a.vc);
+    const float c_log2e = a.scale * 1.4426950408889634f;
+
+    // ---- the tiles on their way: item pi, tile pt of [.., p_end), into stage p_stage
+    uint32_t pi = 0, pt = 0, p_end = 0, p_stage = 0;
+    Item pit = item_at(0);
+    if (!pit.valid()) return;
+    {
+        bool d, l;
+        key_range(pit, pt, p_end, d, l);
+    }
+    const uint32_t k_lane = (lane >> 4) * WROWB + 16 * ((lane & 15) ^ (lane >> 4));
+    const uint32_t v_lane = (lane >> 4) * WROWB + 16 * ((lane & 15) ^ v_swizzle(lane >> 4));
+    uint64_t from_k = 0, from_v = 0;
+    uint32_t to_k = 0, run = 0;  // run: further tiles behind this one that continue its rows
+    uint64_t active = 0;  // all lanes where the next tile lies inside the history or inside the new rows: copied part by part
+    // chooses the next tile's source; a tile on the seam of history and new rows, or at the end of these, is copied at once
+    auto next_copy = [&]() __attribute__((always_inline)) {
+        active = 0;
+        if (!pit.valid()) return;
+        to_k = uni(lds_addr0 + p_stage + 4096 * wave);
+        const uint32_t first = pt * BN, total_keys = pit.base + a.seq;
+        const bool in_hist = first + BN <= pit.base, in_new = first >= pit.base && first + BN <= total_keys;
+        if (run > 0) {
+            --run;
+            from_k += TILE_B;
+            from_v += TILE_B;
+            active = ~0ull;
+        } else if (in_hist || in_new) {
+            const uint64_t row0 = (in_hist ? static_cast<uint64_t>(pit.kvhead) * a.cap + first
+                                           : static_cast<uint64_t>(pit.kvhead) * a.seq + (first - pit.base)) + 16 * wave;
+            run = ((in_hist ? pit.base : total_keys) - first) / BN;
+            run = uni((run < p_end - pt ? run : p_end - pt) - 1);
+            const uint64_t k_from[2] = {reinterpret_cast<uint64_t>(Kn), reinterpret_cast<uint64_t>(Kc)};
+            const uint64_t v_from[2] = {reinterpret_cast<uint64_t>(Vn), reinterpret_cast<uint64_t>(Vc)};
+            from_k = (in_hist ? k_from[1] : k_from[0]) + row0 * WROWB;
+            from_v = (in_hist ? v_from[1] : v_from[0]) + row0 * WROWB;
+            active = ~0ull;
+        } else {
+            const uint8_t *kh = Kc + static_cast<uint64_t>(pit.kvhead) * a.cap * WROWB;
+            const uint8_t *vh = Vc + static_cast<uint64_t>(pit.kvhead) * a.cap * WROWB;
+            const uint8_t *kn = Kn + static_cast<uint64_t>(pit.kvhead) * a.seq * WROWB;
+            const uint8_t *vn = Vn + static_cast<uint64_t>(pit.kvhead) * a.seq * WROWB;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t pos = first + 16 * wave + 4 * i + (lane >> 4);
+                pos = pos < total_keys ? pos : total_keys - 1;
+                const bool old = pos < pit.base;
+                const uint32_t row_off = (old ? pos : pos - pit.base) * WROWB;  // within one kv head: below 2^32
+                const uint8_t *ksrc = (old ? kh : kn) + (row_off + 16 * ((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)));
+                const uint8_t *vsrc = (old ? vh : vn) + (row_off + 16 * ((lane & 15) ^ v_swizzle(lane >> 4)));
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(ksrc), "s"(to_k + i * 1024) : "memory", "m0");
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(vsrc), "s"(to_k + TILE_B + i * 1024) : "memory", "m0");
+            }
+        }
+        p_stage = p_stage + WSTAGE == WNS * WSTAGE ? 0 : p_stage + WSTAGE;
+        if (++pt == p_end) {
+            pit = item_at(++pi);
+            bool d, l;
+            if (pit.valid()) key_range(pit, pt, p_end, d, l);
+        }
+    };
+    // (no branch around a copy, which would cost the wavefront more than the copy: where the tile has been copied at once, the
+    // copy is made with no lane active)
+    auto copy_part = [&]<int I>() __attribute__((always_inline)) {  // 0 .. 7
+        constexpr int J = I / 2;
+        const uint64_t from = I % 2 == 0 ? from_k : from_v, lanes = active;
+        const uint32_t at = I % 2 == 0 ? k_lane ^ (64 * J) : v_lane, to = I % 2 == 0 ? to_k : to_k + TILE_B;
+        asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3\n\ts_mov_b64 exec, -1"
+                     :
+                     : "v"(at), "s"(from), "s"(to), "n"(J * 4 * WROWB), "s"(lanes)
+                     : "memory", "m0");
+    };
+    auto copy_parts = [&]<int FROM, int TO>() __attribute__((always_inline)) {
+        [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+            (copy_part.template operator()<FROM + I>(), ...);
+        }(std::make_integer_sequence<int, TO - FROM>{});
+    };
+
+    // ---- query rows of an item in B-operand layout: lane holds row l32 of a sub-tile, d = 16 kk + 8 half .. + 7
+    Frag q[2][KSTEPS];
+    auto head_of = [&](const Item &it) __attribute__((always_inline)) -> uint32_t {
+        const uint32_t h = it.hc * HW + wave;
+        return h < plan.group ? h : plan.group - 1;
+    };
+    auto first_row = [&](const Item &it) __attribute__((always_inline)) -> uint32_t { return it.qt * ROWS; };
+    auto load_q = [&](const Item &it) __attribute__((always_inline)) {
+        const uint8_t *qh = Q + static_cast<uint64_t>(uni(it.kvhead * plan.group + head_of(it))) * a.seq * WROWB;
+        // whole rows: chunk lane % 16 of rows 4 i + lane / 16 of a sub-tile
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint32_t row = first_row(it) + 32 * s + 4 * i + (lane >> 4);
+                row = row < a.seq ? row : a.seq - 1;
+                q[s][i] = *reinterpret_cast<const Frag *>(qh + (row * WROWB + 16 * (lane & 15)));  // within one head: below 2^32
+            }
+    };
+    // ... and from there through LDS of the wavefront's own into operand layout (chunk c of row r at c ^ (r & 15))
+    uint8_t *const own = lds + WNS * WSTAGE + 32 * WROWB * wave;
+    auto place_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t r = 4 * i + (lane >> 4);
+                *reinterpret_cast<Frag *>(own + r * WROWB + 16 * ((lane & 15) ^ (r & 15))) = q[s][i];
+            }
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk)
+                q[s][kk] = *reinterpret_cast<const Frag *>(own + l32 * WROWB + 16 * ((2 * kk + half) ^ (l32 & 15)));
+        }
+    };
+
+    const uint32_t k_off = l32 * WROWB + 16 * (half ^ (l32 & 15));
+    const uint32_t s16 = lane & 15, v_r = s16 >> 2, v_cl = 2 * ((lane >> 4) & 1) + ((s16 & 3) >> 1);
+    const uint32_t v_off = TILE_B + (4 * half + v_r) * WROWB + 16 * (v_cl ^ v_swizzle(v_r)) + 8 * (s16 & 1);
+    Frag kf[KSTEPS], vf[2 * DBLK];
+    auto read_k = [&](uint32_t block_at, int kk) __attribute__((always_inline)) {  // block_at: stage + 32 kb rows
+        kf[kk] = *reinterpret_cast<const Frag *>(lds + block_at + (k_off ^ (32 * kk)));
+    };
+    auto read_v = [&](uint32_t block_at, int i) __attribute__((always_inline)) {
+        const uint8_t *vp = lds + block_at + 16 * (i / DBLK) * WROWB + (v_off ^ (64 * (i % DBLK)));
+        typedef uint32_t Pair __attribute__((ext_vector_type(2)));
+        const Pair lo = __builtin_bit_cast(Pair, read_tr16(vp)), hi = __builtin_bit_cast(Pair, read_tr16(vp + 8 * WROWB));
+        vf[i] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3);
+    };
+
+    // ---- state of the item being worked on
+    f16v o[2][DBLK], sc[2];
+    Frag pf[2][2];
+    float m[2], l[2], over = 0.f;
+    float raise_at[2], lowest[2];  // the reference is raised where a score exceeds it by raise_at, to lowest at least
+    uint32_t qlim = 0;   // first key that this lane's row of sub-tile 0 does not see
+    uint32_t pos0 = 0;   // position of the wavefront's first row
+    bool mask_all = false;
+    // Sixteenth I of the softmax of sub-tile Y against the 32 keys from `key0`: scores scaled (slots 1-3), masked where the
+    // block reaches past the sub-tile's first row, maximum (4-6), reference raised if need be, probabilities (7-15).
+    auto softmax_part = [&]<int Y, int I>(uint32_t key0) __attribute__((always_inline)) {
+        if constexpr (I == 0) {
+        } else if constexpr (I < 4) {
+            constexpr int from = I == 1 ? 0 : I == 2 ? 6 : 11, to = I == 1 ? 6 : I == 2 ? 11 : 16;
+#pragma unroll
+            for (int e = from; e < to; ++e) sc[Y][e] = fmaf(sc[Y][e], c_log2e, -m[Y]);
+            if constexpr (I == 3) {
+                if (__builtin_expect(key0 + 31 > pos0 + 32 * Y || (SPLIT && mask_all), 0)) {  // wave-uniform
+                    const uint32_t lim = mask_all ? 0u : qlim + 32 * Y;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        if (key0 + 8 * (e / 4) + 4 * half + (e % 4) >= lim) sc[Y][e] = -__builtin_inff();
+                }
+            }
+        } else if constexpr (I < 6) {
+            constexpr int from = I == 4 ? 0 : 8;
+            if constexpr (I == 4) over = -__builtin_inff();
+#pragma unroll
+            for (int e = from; e < from + 8; ++e) over = fmaxf(over, sc[Y][e]);
+        } else if constexpr (I == 6) {
+            over = half_max(over);
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(over > raise_at[Y]) != 0, 0)) {
+                // (the first block, where raise_at is -inf and lowest -1e30, sets the reference to its maximum, if lower than 0 too)
+                const float up = fmaxf(over, lowest[Y]), alpha = __builtin_amdgcn_exp2f(-up);
+                if (lowest[Y] == 0.f) {  // (else there is nothing yet)
+                    l[Y] *= alpha;
+#pragma unroll
+                    for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) o[Y][db][e] *= alpha;
+                }
+                m[Y] += up;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) sc[Y][e] -= up;
+                raise_at[Y] = kSlack;
+                lowest[Y] = 0.f;
+            }
+        } else {
+            // probabilities from .. to - 1 of the block, each pair packed once its second half is there
+            constexpr int from = 16 * (I - 7) / 9, to = 16 * (I - 6) / 9;
+#pragma unroll
+            for (int e = from; e < to; ++e) {
+                float p = __builtin_amdgcn_exp2f(sc[Y][e]);
+                asm volatile("" : "+v"(p));  // (stays here: otherwise it sinks behind the branch of the next copy)
+                sc[Y][e] = p;
+                if (e % 2 == 1) {
+                    uint32_t w = Ops<T>::pack2(sc[Y][e - 1], sc[Y][e]);
+                    asm volatile("" : "+v"(w));
+                    pf[Y][e / 8][(e % 8) / 2] = w;
+                    float sum = Ops<T>::add_pair(l[Y], w, sc[Y][e - 1], sc[Y][e]);
+                    asm volatile("" : "+v"(sum));
+                    l[Y] = sum;
+                }
+            }
+        }
+    };
+    // Phase X of a block: its products (S^T and O^T in turn) beside the softmax of the other sub-tile (keys from key0).
+    // NEXT: S^T of the next block exists.  Phase 1 refills the fragments behind their last use: K two blocks on (k_at), V
+    // one (v_at).  A result of the products is read by the vector ALU no sooner than three products after it (a product
+    // occupies the matrix pipe for 8 passes, its result takes 11 wait states), an operand that the ALU writes no sooner than
+    // two instructions before its product; where there are no products in between, s_nop stands for them.
+    auto phase = [&]<int X, bool NEXT, bool SOFT, int COPY>(uint32_t key0, uint32_t k_at, uint32_t v_at) __attribute__((always_inline)) {
+        if constexpr (!NEXT) asm volatile("s_nop 7" ::: "memory");
+        auto slot = [&]<int I>() __attribute__((always_inline)) {
+            constexpr int i = I / 2;
+            if constexpr (I % 2 == 0) {
+                if constexpr (NEXT) {
+                    if constexpr (i == 0) OpsAsm<T>::scores_first(sc[X], kf[i], q[X][i]);
+                    else OpsAsm<T>::scores(sc[X], kf[i], q[X][i]);
+                    if constexpr (X == 1) read_k(k_at, i);
+                }
+            } else {
+                OpsAsm<T>::output(o[X][i % DBLK], vf[i], pf[X][i / DBLK]);
+                if constexpr (X == 1 && NEXT) read_v(v_at, i);
+            }
+            if constexpr (SOFT) softmax_part.template operator()<1 - X, I>(key0);
+            if constexpr (COPY >= 0 && I % 8 == 4) copy_part.template operator()<COPY + I / 8>();
+            RG_SCHED_FENCE();
+        };
+        [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+            (slot.template operator()<I>(), ...);
+        }(std::make_integer_sequence<int, 16>{});
+        if constexpr (!NEXT) asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    };
+
+    // ---- the item goes out: O normalised (SPLIT: partial results), the item's own new rows into the caches
+    auto finish = [&](const Item &it, bool last_range) __attribute__((always_inline)) {
+        const uint32_t rows_end = (it.qt + 1) * ROWS < a.seq ? (it.qt + 1) * ROWS : a.seq;
+        const bool append = Kc && it.hc == 0 && last_range;
+        const uint64_t new0 = static_cast<uint64_t>(it.kvhead) * a.seq * WROWB, old0 = (static_cast<uint64_t>(it.kvhead) * a.cap + it.base) * WROWB;
+        Frag ak[4], av[4];
+        // 16-byte chunk tid % 16 of rows tid / 16 + 16 j of a group of 64
+        auto fetch_rows = [&](uint32_t row0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t row = row0 + (tid >> 4) + 16 * j;
+                row = row < rows_end ? row : rows_end - 1;
+                const uint32_t off = row * WROWB + 16 * (tid & 15);
+                ak[j] = *reinterpret_cast<const Frag *>(Kn + new0 + off);
+                av[j] = *reinterpret_cast<const Frag *>(Vn + new0 + off);
+            }
+        };
+        auto store_new = [&](uint32_t row0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t row = row0 + (tid >> 4) + 16 * j, off = row * WROWB + 16 * (tid & 15);
+                if (row < rows_end) {
+                    *reinterpret_cast<Frag *>(Kc + old0 + off) = ak[j];
+                    *reinterpret_cast<Frag *>(Vc + old0 + off) = av[j];
+                }
+            }
+        };
+        if (append) fetch_rows(it.qt * ROWS);
+        const bool head_ok = it.hc * HW + wave < plan.group;  // else a repeated head: nothing to store
+        const uint64_t bh = uni(it.kvhead * plan.group + head_of(it));
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const uint32_t row = first_row(it) + 32 * s;
+            if (row >= a.seq || !head_ok) continue;  // wave-uniform
+            if constexpr (SPLIT) {
+                const uint32_t stream = it.kvhead * plan.head_chunks + it.hc;
+                float *rec = plan.part + (static_cast<uint64_t>((stream * plan.q_tiles + it.qt) * 2 + s) * plan.splits + it.ks) * part_floats(128);
+#pragma unroll
+                for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) rec[(db * 16 + e) * 256 + tid] = o[s][db][e];
+                rec[(DBLK * 16) * 256 + tid] = lowest[s] != 0.f ? kMinusBig : m[s];
+                rec[(DBLK * 16 + 1) * 256 + tid] = l[s];
+            } else {
+                const float inv = 1.f / half_sum(l[s]);
+                uint8_t *out = static_cast<uint8_t *>(a.o) + (bh * a.seq + row) * WROWB;
+                // through LDS of the wavefront's own (chunk c of row r at c ^ (r & 15)), so that a store covers four whole rows
+#pragma unroll
+                for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        // registers 4 g .. 4 g + 3 of a block: d = 32 db + 8 g + 4 half + 0..3 of row l32
+                        const f16v &v = o[s][db];
+                        const uint2 x = make_uint2(Ops<T>::pack2(v[4 * g] * inv, v[4 * g + 1] * inv), Ops<T>::pack2(v[4 * g + 2] * inv, v[4 * g + 3] * inv));
+                        *reinterpret_cast<uint2 *>(own + l32 * WROWB + 16 * ((4 * db + g) ^ (l32 & 15)) + 8 * half) = x;
+                    }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t r = 4 * i + (lane >> 4), c = lane & 15;
+                    const Frag x = *reinterpret_cast<const Frag *>(own + r * WROWB + 16 * (c ^ (r & 15)));
+                    if (row + r < a.seq) *reinterpret_cast<Frag *>(out + r * WROWB + 16 * c) = x;
+                }
+            }
+        }
+        if (append) store_new(it.qt * ROWS);
+    };
+
+    // ---- the walk
+    uint32_t ci = 0;
+    Item cur = item_at(0);
+    load_q(cur);
+#pragma unroll 1
+    for (int s = 0; s < WNS - 1; ++s) {
+        next_copy();
+        copy_parts.template operator()<0, 8>();
+    }
+    if (pit.valid()) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((WNS - 2) * 8) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    uint32_t stage = 0;
+    for (;;) {
+        uint32_t t, t_end;
+        bool last_range;
+        key_range(cur, t, t_end, mask_all, last_range);
+        const uint32_t r0 = first_row(cur);
+        pos0 = cur.base + r0;
+        qlim = pos0 + l32 + 1;
+        const Item nxt = item_at(++ci);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+#pragma unroll
+            for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o[s][db][e] = 0.f;
+            m[s] = l[s] = 0.f;
+            raise_at[s] = -__builtin_inff();
+            lowest[s] = kMinusBig;
+        }
+        place_q();
+        {  // the first block's S^T of both sub-tiles, and the softmax of the first one
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk) read_k(stage, kk);
+#pragma unroll
+            for (int i = 0; i < 2 * DBLK; ++i) read_v(stage, i);
+            RG_SCHED_FENCE();
+            [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+                ([&] {
+                    if constexpr (I == 0) {
+                        OpsAsm<T>::scores_first(sc[0], kf[I], q[0][I]);
+                        OpsAsm<T>::scores_first(sc[1], kf[I], q[1][I]);
+                    } else {
+                        OpsAsm<T>::scores(sc[0], kf[I], q[0][I]);
+                        OpsAsm<T>::scores(sc[1], kf[I], q[1][I]);
+                    }
+                    read_k(stage + 32 * WROWB, I);
+                    RG_SCHED_FENCE();
+                }(), ...);
+            }(std::make_integer_sequence<int, KSTEPS>{});
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+            RG_SCHED_FENCE();
+            [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+                (softmax_part.template operator()<0, I>(2 * t * 32), ...);
+            }(std::make_integer_sequence<int, 16>{});
+        }
+        auto begin_tile = [&]() __attribute__((always_inline)) {
+            // tile c + 1 has landed (the copies of tile c + 2 may be on their way)
+            if (pit.valid()) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((WNS - 3) * 8) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            next_copy();
+        };
+        for (; t + 1 < t_end; ++t) {
+            const uint32_t next_stage = stage + WSTAGE == WNS * WSTAGE ? 0 : stage + WSTAGE, key = 64 * t;
+            begin_tile();
+            phase.template operator()<0, true, true, 0>(key, 0, 0);
+            phase.template operator()<1, true, true, 2>(key + 32, next_stage, stage + 32 * WROWB);
+            phase.template operator()<0, true, true, 4>(key + 32, 0, 0);
+            phase.template operator()<1, true, true, 6>(key + 64, next_stage + 32 * WROWB, next_stage);
+            stage = next_stage;
+        }
+        begin_tile();
+        phase.template operator()<0, true, true, 0>(64 * t, 0, 0);
+        phase.template operator()<1, true, true, 2>(64 * t + 32, stage, stage + 32 * WROWB);
+        load_q(nxt.valid() ? nxt : cur);  // (after the last item: nobody looks at them)
+        copy_parts.template operator()<4, 8>();
+        phase.template operator()<0, false, true, -1>(64 * t + 32, 0, 0);
+        phase.template operator()<1, false, false, -1>(0, 0, 0);
+        stage = stage + WSTAGE == WNS * WSTAGE ? 0 : stage + WSTAGE;
+        finish(cur, last_range);
+        if (!nxt.valid()) break;
+        cur = nxt;
     }
 }
 
@@ -883,7 +1367,7 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
             const int rc = launch_status();
             if (rc) return rc;
             constexpr unsigned parts = ((DH + 31) / 32) * 16 / kMergeRegs;
-            attn_prefill_merge<T, HW, DH><<<dim3(static_cast<unsigned>(whole_streams * plan.q_tiles), parts), 256, 0, s>>>(a, plan);
+            attn_prefill_merge<T, HW, DH, 1><<<dim3(static_cast<unsigned>(whole_streams * plan.q_tiles), parts), 256, 0, s>>>(a, plan);
             return launch_status();
         }
     }
@@ -892,9 +1376,58 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
     return launch_status();
 }
 
+// The dealing of a launch of attn_prefill_wide: as launch_hw, with one workgroup on a CU.
+template <class T>
+int launch_wide(const PrefillArgs &a, hipStream_t s) {
+    constexpr uint32_t ROWS = 64, HW = 4;
+    const uint64_t cus = resident_prefill_workgroups<T, HW, 128>() / 2;
+    PrefillPlan plan{};
+    plan.group = a.H / a.Hkv;
+    plan.head_chunks = (plan.group + HW - 1) / HW;
+    plan.q_tiles = (a.seq + ROWS - 1) / ROWS;
+    plan.pairs = (plan.q_tiles + 1) / 2;
+    uint64_t streams = static_cast<uint64_t>(a.N) * a.Hkv * plan.head_chunks;
+    if (streams * plan.pairs > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
+    const uint64_t splits = wide_splits(streams * plan.q_tiles, a.cap, cus, a.part ? a.part_bytes / (2 * part_floats(128) * sizeof(float)) : 0);
+    plan.splits = 1;
+    if (splits >= 2 && streams * splits * plan.q_tiles <= 0x7fffffffu) {
+        plan.splits = static_cast<uint32_t>(splits);
+        plan.pairs = plan.q_tiles;
+    }
+    plan.magic_splits = plan.splits > 1 ? static_cast<uint32_t>((1ull << 32) / plan.splits + 1) : 0;
+    plan.part = a.part;
+    const uint64_t whole_streams = streams;
+    streams *= plan.splits;
+    plan.xcds = streams % 8 == 0 ? 8 : 1;
+    plan.spx = static_cast<uint32_t>(streams / plan.xcds);
+    uint32_t groups = static_cast<uint32_t>(cus) / plan.xcds / plan.pairs;
+    if (groups < 1) groups = 1;
+    if (groups > plan.spx) groups = plan.spx;
+    plan.groups = groups;
+    uint64_t widest = plan.head_chunks > a.Hkv ? plan.head_chunks : a.Hkv;
+    if (plan.splits > widest) widest = plan.splits;
+    if (streams * widest >= (1ull << 32)) return RG_HIP_E_UNSUPPORTED;
+    plan.magic_chunks = plan.head_chunks > 1 ? static_cast<uint32_t>((1ull << 32) / plan.head_chunks + 1) : 0;
+    plan.magic_hkv = a.Hkv > 1 ? static_cast<uint32_t>((1ull << 32) / a.Hkv + 1) : 0;
+    const uint32_t grid = plan.xcds * plan.groups * plan.pairs;
+    if (plan.splits == 1) {
+        attn_prefill_wide<T, false><<<grid, 256, 0, s>>>(a, plan);
+        return launch_status();
+    }
+    attn_prefill_wide<T, true><<<grid, 256, 0, s>>>(a, plan);
+    const int rc = launch_status();
+    if (rc) return rc;
+    attn_prefill_merge<T, HW, 128, 2><<<dim3(static_cast<unsigned>(2 * whole_streams * plan.q_tiles), 64 / kMergeRegs), 256, 0, s>>>(a, plan);
+    return launch_status();
+}
+
 template <class T, int DH>
 int launch_d(const PrefillArgs &a, hipStream_t s) {
     const uint32_t group = a.H / a.Hkv;
+    if constexpr (DH == 128) {
+        const uint64_t cus = resident_prefill_workgroups<T, 4, 128>() / 2;
+        if (wide_pays(a.N, a.H, a.Hkv, a.seq, a.cap, cus, a.part ? a.part_bytes / (2 * part_floats(128) * sizeof(float)) : 0)) return launch_wide<T>(a, s);
+    }
     if (group == 1) return launch_hw<T, 1, DH>(a, s);
     if (group == 2) return launch_hw<T, 2, DH>(a, s);
     return launch_hw<T, 4, DH>(a, s);  // chunks of four heads; the last one is short when group % 4 != 0

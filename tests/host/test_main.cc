@@ -265,6 +265,14 @@ static void attentionPlan() {
     EXPECT(tiled(16, 28, 4, 1, 4096, 128)); // three launches on the split kernel
     // without room for records, other head dims: the rule for items that walk all of their keys
     EXPECT(!rg::prefill_pays(1, 32, 8, 4, 4096, 128, false) && !tiled(1, 32, 8, 4, 4096, 96) && tiled(32, 32, 8, 16, 4096, 96));
+    // 64 or 32 query rows a wavefront: N, query heads, kv heads, new rows, capacity (256 CUs, records for 256 items)
+    auto wide = [](size_t n, size_t h, size_t hk, size_t seq, size_t cap) { return rg::wide_pays(n, h, hk, seq, cap, 256, 256); };
+    EXPECT(wide(1, 32, 8, 128, 20480) && !wide(1, 32, 8, 128, 16384) && !wide(1, 32, 8, 80, 20480) && wide(1, 32, 8, 512, 8512));
+    EXPECT(wide(1, 4, 1, 64, 40960) && !wide(1, 4, 1, 64, 40896) && wide(1, 12, 4, 48, 40960) && !wide(1, 12, 4, 47, 40960));
+    EXPECT(wide(8, 32, 8, 1536, 4096) && !wide(8, 32, 8, 1535, 4096) && !wide(5, 32, 8, 1536, 4096));
+    EXPECT(!wide(8, 16, 8, 2048, 4096) && !wide(1, 8, 8, 128, 40960) && wide(1, 192, 64, 1550, 1600) && !wide(32, 32, 8, 512, 4096));
+    EXPECT(rg::wide_splits(16, 20480, 256, 256) == 16 && rg::wide_splits(1, 41024, 256, 256) == 32 && rg::wide_splits(16, 20480, 256, 100) == 6);
+    EXPECT(rg::wide_splits(128, 2600, 256, 256) == 2 && rg::wide_splits(129, 2600, 256, 256) == 1 && rg::wide_splits(2, 512, 256, 0) == 1);
 }
 
 static void shapeDigests() {

@@ -1153,6 +1153,35 @@ def test_attention_long_history_keys_shared_between_workgroups(N, H, Hkv, seq, c
     assert np.array_equal(kc, ref_kc) and np.array_equal(vc, ref_vc)
 
 
+@pytest.mark.parametrize("N,H,Hkv,seq,cap,past,dt,pairs", [
+    (1, 4, 1, 64, 41024, [40001], torch.float16, [(0, 0), (0, 3)]),                # one item, 32 ranges of 20 tiles
+    (1, 12, 4, 50, 41024, [4321], torch.bfloat16, [(0, 0), (0, 11)]),              # group of 3, ragged rows, ranges beyond the keys
+    (4, 32, 8, 256, 2600, [2344, 17, 0, 1003], torch.float16, [(0, 5), (1, 0), (2, 31), (3, 14)]),  # two ranges, one of them empty
+    (2, 16, 1, 199, 20544, [20345, 700], torch.bfloat16, [(0, 15), (1, 2)]),       # group of 16: four chunks of heads
+    (1, 192, 64, 1550, 1600, [37], torch.float16, [(0, 0), (0, 100), (0, 191)]),   # whole items, the seam inside a tile
+    (2, 128, 32, 1536, 1536, [0, 0], torch.bfloat16, [(0, 1), (1, 127)]),          # whole items, even query tiles
+])
+def test_attention_sixty_four_rows_a_wavefront(N, H, Hkv, seq, cap, past, dt, pairs):
+    # the calls that go to attn_prefill_wide; queries four times as large as elsewhere, so that the reference of the
+    # softmax is raised again and again
+    rng = np.random.default_rng(71)
+    mk = lambda *shape: dev(rng.standard_normal(shape, dtype=np.float32)).to(dt)
+    q, k, v, kc, vc = mk(N, H, seq, 128) * 4, mk(N, Hkv, seq, 128), mk(N, Hkv, seq, 128), mk(N, Hkv, cap, 128), mk(N, Hkv, cap, 128)
+    kc0, vc0 = kc.clone(), vc.clone()
+    o = ops.attention_kvcache(q, k, v, kc, vc, dev(np.asarray(past, np.int64)))
+    assert bool(torch.isfinite(o).all())
+    for b, p in enumerate(past):
+        for new, cache, old in ((k, kc, kc0), (v, vc, vc0)):
+            assert torch.equal(cache[b, :, p:p + seq], new[b])
+            assert torch.equal(cache[b, :, :p], old[b, :, :p]) and torch.equal(cache[b, :, p + seq:], old[b, :, p + seq:])
+    f = lambda t: host(t.float())
+    for b, h in pairs:
+        kh, end = h // (H // Hkv), past[b] + seq
+        ref = oracle.attention_head(f(q[b, h]), f(kc[b, kh, :end]), f(vc[b, kh, :end]), past[b], 1 / math.sqrt(128), True)
+        # one rounding of every probability and of the output: outputs are sums of up to |v| < 6 weighted by at most 1
+        assert np.max(np.abs(f(o[b, h]) - ref)) <= (2 * ABS_F16 if dt == torch.float16 else 4e-2), (b, h)
+
+
 def test_attention_prefill_no_cache_tiled():
     rng = np.random.default_rng(21)
     mk = lambda shape: dev(rng.standard_normal(shape).astype(np.float32)).half()
