@@ -1,0 +1,443 @@
+// The calls of ops.py in native code: argument checks, output allocation and the C ABI call of one operator, for tensors that
+// need nothing special.  Each function returns None where an argument is not what it handles (another kind of tensor, shapes that
+// do not fit, a batch to broadcast): ops.py then goes through the same steps in Python and raises what there is to raise.
+//
+// What bounds a decode step of one sequence is this work: seven calls of 8.5 us each in Python against 41 us of kernels (62 us
+// in all, 41 with these; a small row operator 6.5 and 4.1).
+// The functions of librg_hip.so are handed over by address (bind), so that both ways call the same library.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <array>
+#include <cmath>
+#include <cstdint>
+#include <exception>
+
+#include "rg_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+// ---- the library
+#define RG_CALLS(X)                                                                                                             \
+    X(rg_hip_rms_norm) X(rg_hip_softmax) X(rg_hip_rope) X(rg_hip_dequantize_linear) X(rg_hip_dynamic_quantize_linear_workspace)  \
+    X(rg_hip_dynamic_quantize_linear) X(rg_hip_matmul_workspace) X(rg_hip_matmul_ws) X(rg_hip_transpose) X(rg_hip_split)         \
+    X(rg_hip_matmul_integer) X(rg_hip_matmul_integer_dequantize) X(rg_hip_attention_kvcache)
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+    RG_CALLS(X)
+#undef X
+    PyObject *check = nullptr;  // abi.check
+} rg;
+
+// bind(addresses: dict of name -> address, check)
+PyObject *bind(PyObject *, PyObject *args) {
+    PyObject *addresses, *check;
+    if (!PyArg_ParseTuple(args, "O!O", &PyDict_Type, &addresses, &check)) return nullptr;
+#define X(name)                                                                                   \
+    {                                                                                             \
+        PyObject *at = PyDict_GetItemString(addresses, #name);                                    \
+        if (!at) return PyErr_Format(PyExc_KeyError, "%s", #name);                                \
+        void *p = PyLong_AsVoidPtr(at);                                                           \
+        if (!p) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "%s", #name);  \
+        rg.name = reinterpret_cast<decltype(rg.name)>(p);                                         \
+    }
+    RG_CALLS(X)
+#undef X
+    Py_INCREF(check);
+    Py_XDECREF(rg.check);
+    rg.check = check;
+    Py_RETURN_NONE;
+}
+
+// ---- arguments
+struct Decline {};  // the call is left to Python
+
+// A contiguous device tensor of torch's own types, without anything around it that gives its memory another meaning.
+const Tensor &tensor(PyObject *o) {
+    if (!THPVariable_CheckExact(o)) throw Decline{};
+    const Tensor &t = THPVariable_Unpack(o);
+    constexpr c10::DispatchKeySet odd = c10::python_ks | c10::functorch_transforms_ks |
+                                        c10::DispatchKeySet({c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
+                                                             c10::DispatchKey::ZeroTensor, c10::DispatchKey::Functionalize,
+                                                             c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::Batched});
+    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.key_set().has_any(odd) || !t.is_contiguous())
+        throw Decline{};
+    return t;
+}
+const Tensor *optional(PyObject *o) { return o == Py_None ? nullptr : &tensor(o); }
+
+double number(PyObject *o) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) {
+        PyErr_Clear();
+        throw Decline{};
+    }
+    return v;
+}
+int64_t whole(PyObject *o) {
+    if (!PyLong_CheckExact(o)) throw Decline{};
+    const int64_t v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        throw Decline{};
+    }
+    return v;
+}
+bool flag(PyObject *o) {
+    if (o != Py_True && o != Py_False) throw Decline{};
+    return o == Py_True;
+}
+void require(bool ok) {
+    if (!ok) throw Decline{};
+}
+
+int code(const Tensor &t) {
+    switch (t.scalar_type()) {
+        case at::kFloat: return RG_F32;
+        case at::kHalf: return RG_FP16;
+        case at::kBFloat16: return RG_BF16;
+        case at::kDouble: return RG_F64;
+        case at::kByte: return RG_U8;
+        case at::kChar: return RG_I8;
+        case at::kShort: return RG_I16;
+        case at::kInt: return RG_I32;
+        case at::kLong: return RG_I64;
+        case at::kBool: return RG_BOOL;
+        default: throw Decline{};
+    }
+}
+
+void *ptr(const Tensor &t) { return t.data_ptr(); }
+void *ptr(const Tensor *t) { return t ? t->data_ptr() : nullptr; }
+void *stream() { return c10::hip::getCurrentHIPStream(c10::hip::current_device()).stream(); }
+
+PyObject *result(const Tensor &y, int status, const char *what) {
+    if (status != 0) return PyObject_CallFunction(rg.check, "is", status, what);  // raises
+    return THPVariable_Wrap(y);
+}
+
+template <Py_ssize_t COUNT, PyObject *(*CALL)(PyObject *const *)>
+PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t count) {
+    if (count != COUNT || !rg.check) return PyErr_Format(PyExc_TypeError, "%zd arguments after bind()", COUNT);
+    try {
+        return CALL(args);
+    } catch (const Decline &) {
+        Py_RETURN_NONE;
+    } catch (const python_error &e) {
+        const_cast<python_error &>(e).restore();
+    } catch (const c10::OutOfMemoryError &) {
+        Py_RETURN_NONE;  // (Python meets it again and raises it as torch does)
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+// ---- operators
+PyObject *rms_norm(PyObject *const *p) {  // x, w, eps
+    const Tensor &x = tensor(p[0]), &w = tensor(p[1]);
+    const float eps = static_cast<float>(number(p[2]));
+    require(x.dim() > 0 && x.numel() > 0);
+    const int64_t cols = x.size(-1);
+    const int type = code(x);
+    Tensor y = at::empty_like(x);
+    return result(y, rg.rg_hip_rms_norm(ptr(y), ptr(x), ptr(w), x.numel() / cols, cols, eps, type, stream()), "rg_hip_rms_norm");
+}
+
+PyObject *softmax(PyObject *const *p) {  // x, axis, causal
+    const Tensor &x = tensor(p[0]);
+    int64_t axis = whole(p[1]);
+    const bool causal = flag(p[2]);
+    require(axis >= -x.dim() && axis < x.dim() && (!causal || x.dim() >= 2));
+    if (axis < 0) axis += x.dim();
+    size_t pre = 1, post = 1;
+    for (int64_t i = 0; i < axis; ++i) pre *= x.size(i);
+    for (int64_t i = axis + 1; i < x.dim(); ++i) post *= x.size(i);
+    const int type = code(x);
+    Tensor y = at::empty_like(x);
+    return result(y, rg.rg_hip_softmax(ptr(y), ptr(x), pre, x.size(axis), post, type, causal ? x.size(-2) : 0, stream()), "rg_hip_softmax");
+}
+
+PyObject *rope(PyObject *const *p) {  // x, pos, theta
+    const Tensor &x = tensor(p[0]), &pos = tensor(p[1]);
+    const float theta = static_cast<float>(number(p[2]));
+    require(pos.scalar_type() == at::kLong && x.dim() == 4);
+    const int type = code(x);
+    Tensor y = at::empty_like(x);
+    return result(y, rg.rg_hip_rope(ptr(y), ptr(x), static_cast<const int64_t *>(ptr(pos)), pos.dim() == 2, x.size(0), x.size(1), x.size(2),
+                                    x.size(3), theta, type, stream()), "rg_hip_rope");
+}
+
+PyObject *dequantize_linear(PyObject *const *p) {  // x, scale, zp, axis
+    const Tensor &x = tensor(p[0]), &scale = tensor(p[1]);
+    const Tensor *zp = optional(p[2]);
+    int64_t axis = whole(p[3]);
+    require(scale.scalar_type() == at::kFloat);
+    const bool per_axis = scale.numel() != 1;
+    size_t outer = 1, length = 1, inner = x.numel();
+    if (per_axis) {
+        require(x.dim() > 0);
+        axis = ((axis % x.dim()) + x.dim()) % x.dim();
+        inner = 1;
+        for (int64_t i = 0; i < axis; ++i) outer *= x.size(i);
+        for (int64_t i = axis + 1; i < x.dim(); ++i) inner *= x.size(i);
+        length = x.size(axis);
+        require(scale.numel() == x.size(axis));
+    }
+    const int type = code(x);
+    Tensor y = at::empty_like(x, x.options().dtype(at::kFloat));
+    return result(y, rg.rg_hip_dequantize_linear(static_cast<float *>(ptr(y)), ptr(x), static_cast<const float *>(ptr(scale)), ptr(zp), outer,
+                                                 length, inner, type, per_axis, stream()), "rg_hip_dequantize_linear");
+}
+
+PyObject *dynamic_quantize_linear(PyObject *const *p) {  // x -> (y, scale, zero point)
+    const Tensor &x = tensor(p[0]);
+    require(x.scalar_type() == at::kFloat);
+    const size_t n = x.numel(), bytes = rg.rg_hip_dynamic_quantize_linear_workspace(n);
+    const auto u8 = x.options().dtype(at::kByte);
+    Tensor y = at::empty_like(x, u8), scale = at::empty({1}, x.options()), zp = at::empty({1}, u8);
+    Tensor ws = at::empty({static_cast<int64_t>(bytes)}, u8);
+    const int status = rg.rg_hip_dynamic_quantize_linear(static_cast<uint8_t *>(ptr(y)), static_cast<float *>(ptr(scale)), static_cast<uint8_t *>(ptr(zp)),
+                                                         static_cast<const float *>(ptr(x)), n, ptr(ws), bytes, stream());
+    if (status != 0) return result(y, status, "rg_hip_dynamic_quantize_linear");
+    PyObject *out = PyTuple_New(3);
+    if (!out) return nullptr;
+    PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(y));
+    PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(scale));
+    PyTuple_SET_ITEM(out, 2, THPVariable_Wrap(zp));
+    return out;
+}
+
+// Operands of a product whose batch dimensions are the same ones (or none): output sizes and the number of matrices.
+struct Product {
+    c10::SmallVector<int64_t, 6> sizes;
+    size_t batch = 1, m, k, n;
+};
+Product product(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b) {
+    require(a.dim() >= 2 && a.dim() == b.dim());
+    Product p;
+    for (int64_t i = 0; i < a.dim() - 2; ++i) {
+        require(a.size(i) == b.size(i));
+        p.batch *= a.size(i);
+        p.sizes.push_back(a.size(i));
+    }
+    p.m = a.size(trans_a ? -1 : -2);
+    p.k = a.size(trans_a ? -2 : -1);
+    p.n = b.size(trans_b ? -2 : -1);
+    require(static_cast<int64_t>(p.k) == b.size(trans_b ? -1 : -2));
+    p.sizes.push_back(p.m);
+    p.sizes.push_back(p.n);
+    return p;
+}
+
+// What rg_hip_matmul_workspace says depends on the shape (and the CUs of a device, the same ones for all devices of a box; a
+// workspace too small is not used): the last shapes of a thread are remembered, 64 of them.
+size_t matmul_workspace(int type, int trans_a, int trans_b, const Product &p) {
+    struct Known {
+        std::array<size_t, 5> shape{};
+        size_t bytes = 0;
+        bool set = false;
+    };
+    static thread_local std::array<Known, 64> known;
+    const std::array<size_t, 5> shape{static_cast<size_t>(type * 4 + trans_a * 2 + trans_b), p.batch, p.m, p.k, p.n};
+    Known &slot = known[(p.batch * 31 + p.m * 7 + p.k / 8 * 13 + p.n / 8 * 3 + shape[0]) % known.size()];
+    if (!slot.set || slot.shape != shape) slot = {shape, rg.rg_hip_matmul_workspace(type, trans_a, trans_b, p.batch, p.m, p.k, p.n), true};
+    return slot.bytes;
+}
+
+PyObject *matmul(PyObject *const *p) {  // a, b, c, trans_a, trans_b, alpha, beta
+    const Tensor &a = tensor(p[0]), &b = tensor(p[1]);
+    const Tensor *c = optional(p[2]);
+    const bool trans_a = flag(p[3]), trans_b = flag(p[4]);
+    const float alpha = static_cast<float>(number(p[5])), beta = static_cast<float>(number(p[6]));
+    require(a.scalar_type() == b.scalar_type());
+    const Product s = product(a, b, trans_a, trans_b);
+    size_t sb = 0, sm = 0, sn = 0;
+    if (c) {
+        // strides of the bias: broadcast over leading dimensions of size 1, or one per matrix
+        const int64_t lead = a.dim() - c->dim();
+        require(c->scalar_type() == a.scalar_type() && lead >= 0);
+        auto dim = [&](int64_t i) { return i < lead ? int64_t(1) : c->size(i - lead); };
+        const int64_t rows = dim(a.dim() - 2), cols = dim(a.dim() - 1);
+        bool same = true, ones = true;
+        for (int64_t i = 0; i < a.dim() - 2; ++i) {
+            same &= dim(i) == s.sizes[i];
+            ones &= dim(i) == 1;
+        }
+        if (same && s.batch > 1) sb = rows * cols;
+        else require(ones);
+        require((rows == 1 || rows == static_cast<int64_t>(s.m)) && (cols == 1 || cols == static_cast<int64_t>(s.n)));
+        sm = rows != 1 ? cols : 0;
+        sn = cols == static_cast<int64_t>(s.n) ? 1 : 0;
+    }
+    const int type = code(a);
+    Tensor y = at::empty(s.sizes, a.options());
+    const size_t bytes = matmul_workspace(type, trans_a, trans_b, s);
+    Tensor ws;
+    if (bytes) ws = at::empty({static_cast<int64_t>(bytes)}, a.options().dtype(at::kByte));
+    return result(y, rg.rg_hip_matmul_ws(ptr(y), ptr(a), ptr(b), ptr(c), type, trans_a, trans_b, alpha, beta, s.batch, s.m, s.k, s.n, nullptr, nullptr,
+                                         sb, sm, sn, bytes ? ptr(ws) : nullptr, bytes, stream()), "rg_hip_matmul_ws");
+}
+
+PyObject *matmul_integer(PyObject *const *p) {  // a, b, a_zp, b_zp, dequant_scale
+    const Tensor &a = tensor(p[0]), &b = tensor(p[1]);
+    const Tensor *a_zp = optional(p[2]), *b_zp = optional(p[3]), *scale = optional(p[4]);
+    const Product s = product(a, b, false, false);
+    const unsigned flags = (a_zp && a_zp->numel() == 1 ? RG_MMI_A_ZP_SCALAR : 0u) | (b_zp && b_zp->numel() == 1 ? RG_MMI_B_ZP_SCALAR : 0u);
+    if (scale) require(scale->scalar_type() == at::kFloat && (scale->numel() == 1 || scale->numel() == static_cast<int64_t>(s.n)));
+    Tensor y = at::empty(s.sizes, a.options().dtype(scale ? at::kFloat : at::kInt));
+    if (scale)
+        return result(y, rg.rg_hip_matmul_integer_dequantize(static_cast<float *>(ptr(y)), ptr(a), ptr(b), ptr(a_zp), ptr(b_zp), flags, s.batch, s.m, s.k,
+                                                             s.n, nullptr, nullptr, static_cast<const float *>(ptr(scale)), scale->numel() != 1,
+                                                             nullptr, stream()), "rg_hip_matmul_integer_dequantize");
+    return result(y, rg.rg_hip_matmul_integer(static_cast<int32_t *>(ptr(y)), ptr(a), ptr(b), ptr(a_zp), ptr(b_zp), flags, s.batch, s.m, s.k, s.n,
+                                              nullptr, nullptr, nullptr, stream()), "rg_hip_matmul_integer");
+}
+
+PyObject *transpose(PyObject *const *p) {  // x, perm (tuple)
+    const Tensor &x = tensor(p[0]);
+    constexpr int64_t kMost = 16;
+    const int64_t rank = x.dim();
+    require(PyTuple_CheckExact(p[1]) && PyTuple_GET_SIZE(p[1]) == rank && rank <= kMost);
+    std::array<int64_t, kMost> perm{}, run_of{}, sizes{};
+    c10::SmallVector<int64_t, 6> out;
+    uint32_t seen = 0;
+    for (int64_t i = 0; i < rank; ++i) {
+        perm[i] = whole(PyTuple_GET_ITEM(p[1], i));
+        require(perm[i] >= 0 && perm[i] < rank && !(seen >> perm[i] & 1));
+        seen |= 1u << perm[i];
+        out.push_back(x.size(perm[i]));
+    }
+    // Dimensions of size 1 are dropped and dimensions that stay neighbours in order merged into runs; run_of[r]: the place of
+    // the r-th run of the output among the runs of the input, sizes[place]: its size.
+    std::array<int64_t, kMost> first{}, length{};
+    int64_t runs = 0, last = -2;
+    auto next_kept = [&](int64_t d) {
+        do ++d;
+        while (d < rank && x.size(d) == 1);
+        return d;
+    };
+    for (int64_t i = 0; i < rank; ++i) {
+        if (x.size(perm[i]) == 1) continue;
+        if (runs && last >= 0 && next_kept(last) == perm[i]) {
+            length[runs - 1] *= x.size(perm[i]);
+        } else {
+            first[runs] = perm[i];
+            length[runs++] = x.size(perm[i]);
+        }
+        last = perm[i];
+    }
+    size_t block = x.element_size(), count = x.numel();
+    std::array<uint32_t, kMost> from{}, to{};
+    size_t dims = 1;
+    if (runs <= 1) {
+        from[0] = to[0] = 1;
+        block *= count;
+        count = 1;
+    } else {
+        for (int64_t r = 0; r < runs; ++r) {
+            run_of[r] = 0;
+            for (int64_t q = 0; q < runs; ++q) run_of[r] += first[q] < first[r];
+            sizes[run_of[r]] = length[r];
+        }
+        if (run_of[runs - 1] == runs - 1) {  // the last run stays last: it is the block
+            block *= length[runs - 1];
+            require(length[runs - 1] != 0);
+            count /= length[runs - 1];
+            --runs;
+        }
+        dims = runs;
+        int64_t step = 1;
+        std::array<int64_t, kMost> in_step{};
+        for (int64_t q = runs - 1; q >= 0; --q) {
+            in_step[q] = step;
+            step *= sizes[q];
+        }
+        step = 1;
+        for (int64_t r = runs - 1; r >= 0; --r) {
+            from[r] = static_cast<uint32_t>(in_step[run_of[r]]);
+            to[r] = static_cast<uint32_t>(step);
+            step *= length[r];
+        }
+        require(step <= 0xffffffffll);
+    }
+    Tensor y = at::empty(out, x.options());
+    return result(y, rg.rg_hip_transpose(ptr(y), ptr(x), from.data(), to.data(), dims, block, count, stream()), "rg_hip_transpose");
+}
+
+PyObject *split(PyObject *const *p) {  // x, sizes (list), axis -> list
+    const Tensor &x = tensor(p[0]);
+    constexpr Py_ssize_t kMost = 16;
+    require(PyList_CheckExact(p[1]) && PyList_GET_SIZE(p[1]) >= 1 && PyList_GET_SIZE(p[1]) <= kMost && x.dim() > 0);
+    const Py_ssize_t parts = PyList_GET_SIZE(p[1]);
+    int64_t axis = whole(p[2]);
+    axis = ((axis % x.dim()) + x.dim()) % x.dim();
+    size_t blocks = 1, postfix = x.element_size();
+    for (int64_t i = 0; i < axis; ++i) blocks *= x.size(i);
+    for (int64_t i = axis + 1; i < x.dim(); ++i) postfix *= x.size(i);
+    std::array<uint32_t, kMost> segments{};
+    std::array<int64_t, kMost> size{};
+    size_t total = 0;
+    int64_t sum = 0;
+    for (Py_ssize_t i = 0; i < parts; ++i) {
+        size[i] = whole(PyList_GET_ITEM(p[1], i));
+        require(size[i] >= 0 && size[i] * postfix <= 0xffffffffu);
+        segments[i] = static_cast<uint32_t>(size[i] * postfix);
+        total += segments[i];
+        sum += size[i];
+    }
+    require(sum == x.size(axis));
+    std::array<Tensor, kMost> outs;
+    std::array<void *, kMost> to{};
+    c10::SmallVector<int64_t, 6> shape(x.sizes().begin(), x.sizes().end());
+    for (Py_ssize_t i = 0; i < parts; ++i) {
+        shape[axis] = size[i];
+        outs[i] = at::empty(shape, x.options());
+        to[i] = ptr(outs[i]);
+    }
+    const int status = rg.rg_hip_split(to.data(), ptr(x), segments.data(), parts, blocks, total, stream());
+    if (status != 0) return result(x, status, "rg_hip_split");
+    PyObject *list = PyList_New(parts);
+    if (!list) return nullptr;
+    for (Py_ssize_t i = 0; i < parts; ++i) PyList_SET_ITEM(list, i, THPVariable_Wrap(outs[i]));
+    return list;
+}
+
+PyObject *attention_kvcache(PyObject *const *p) {  // q, k, v, k_cache, v_cache, past_lens, scale, workspace, sync_state
+    const Tensor &q = tensor(p[0]), &k = tensor(p[1]), &v = tensor(p[2]);
+    const Tensor *kc = optional(p[3]), *vc = optional(p[4]), *past = optional(p[5]);
+    const Tensor &ws = tensor(p[7]);
+    const Tensor *state = optional(p[8]);
+    require(q.dim() == 4 && k.dim() == 4 && (!kc || kc->dim() == 4));
+    const int64_t batch = q.size(0);
+    const double scale = p[6] == Py_None ? 1.0 / std::sqrt(static_cast<double>(q.size(3))) : number(p[6]);
+    int per_row = 0;
+    if (past) {
+        require(past->scalar_type() == at::kLong && (past->numel() == 1 || past->numel() == batch));
+        per_row = past->numel() == batch && batch > 1;
+    }
+    const int type = code(q);
+    Tensor o = at::empty_like(q);
+    return result(o, rg.rg_hip_attention_kvcache(ptr(o), ptr(q), ptr(k), ptr(v), ptr(kc), ptr(vc), static_cast<const int64_t *>(ptr(past)), per_row, batch,
+                                                 q.size(1), k.size(1), q.size(2), kc ? kc->size(2) : 0, q.size(3), static_cast<float>(scale), type,
+                                                 ptr(ws), ws.numel(), ptr(state), stream()), "rg_hip_attention_kvcache");
+}
+
+#define ENTRY(name, count) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<count, name>)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {
+    {"bind", bind, METH_VARARGS, nullptr}, ENTRY(rms_norm, 3), ENTRY(softmax, 3), ENTRY(rope, 3), ENTRY(dequantize_linear, 4),
+    ENTRY(dynamic_quantize_linear, 1), ENTRY(matmul, 7), ENTRY(matmul_integer, 5), ENTRY(transpose, 2), ENTRY(split, 3),
+    ENTRY(attention_kvcache, 9), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_rg_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__rg_calls(void) { return PyModule_Create(&module); }

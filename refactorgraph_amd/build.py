@@ -4,6 +4,7 @@
     librg_host.so    C++ host layer mirroring the reference's plugin surface
                      (hardware::Device, runtime::Resources/Routine, kernel::Kernel,
                      collectors); links librg_hip.so
+    _rg_calls.so     the calls of ops.py in native code (binding/calls.cc), a Python extension on torch's headers
     librg_probe.so   measurement aids of bench.py (bench_probes/): ceilings of the matrix pipe
                      and of HBM; not part of the boundary, loaded by the benchmark only
 
@@ -83,6 +84,22 @@ def build_host(jobs=8):
     return out
 
 
+def build_calls():
+    """Host code on torch's headers and libraries; the functions of librg_hip.so reach it by address."""
+    import sysconfig
+
+    import torch
+    torch_dir = os.path.dirname(torch.__file__)
+    out = os.path.join(LIB, "_rg_calls.so")
+    _run(["g++", "-O2", "-std=c++20", "-fPIC", "-Wall", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(f"-I{d}" for d in (os.path.join(torch_dir, "include"), os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+                               "/opt/rocm/include", sysconfig.get_paths()["include"], INCLUDE)),
+          os.path.join(PKG, "binding", "calls.cc"), "-o", out,
+          f"-L{os.path.join(torch_dir, 'lib')}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"])
+    return out
+
+
 def build_probes():
     os.makedirs(OBJ, exist_ok=True)
     out = os.path.join(LIB, "librg_probe.so")
@@ -93,8 +110,9 @@ def build_probes():
 def build_all(jobs=8):
     hip = build_hip(jobs)
     host = build_host(jobs)
+    calls = build_calls()
     probes = build_probes()
-    return hip, host, probes
+    return hip, host, calls, probes
 
 
 if __name__ == "__main__":

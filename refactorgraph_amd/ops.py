@@ -7,7 +7,9 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import importlib.util
 import math
+import os
 
 import numpy as np
 import torch
@@ -26,10 +28,30 @@ for _name, _code in (("uint16", abi.U16), ("uint32", abi.U32), ("uint64", abi.U6
         _T2CODE[getattr(torch, _name)] = _code
 
 
-# A call's host work is what a decode step of one sequence waits for (seven calls of 13 us each against 40 us of kernels
-# before): addresses go to ctypes as integers, what depends on shapes alone (MatMul's workspace: and on the device's CUs, the
-# same for all devices of a box; too small a workspace is not used) is worked out once per shape, in bounded caches,
-# two-dimensional products skip the broadcasting of batches.
+# A call's host work is what a decode step of one sequence waits for (seven calls of 8.5 us each against 41 us of kernels).  So the
+# usual calls go through binding/calls.cc, which checks, allocates and launches in native code (the attention half of a layer, one
+# token 62 -> 41 us, one small row operator 6.5 -> 4.1); what it declines (it then returns
+# None) takes the Python way below, with addresses as integers and what depends on shapes alone worked out once per shape, in
+# bounded caches (MatMul's workspace: and on the device's CUs, the same for all devices of a box; too small a workspace is not used).
+
+class _NotLoaded:
+    """Stands for the native calls until the first of them is looked up."""
+
+    def __getattr__(self, name):
+        global _native
+        path = os.path.join(os.path.dirname(abi.HOST_LIB_PATH), "_rg_calls.so")
+        if not os.path.exists(path):
+            raise abi.RgHipError(f"{path} is missing: build it with `python -m refactorgraph_amd.build`")
+        spec = importlib.util.spec_from_file_location("_rg_calls", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.bind({n: C.cast(getattr(lib(), n), C.c_void_p).value for n in abi.SIGNATURES}, check)
+        _native = module
+        return getattr(module, name)
+
+
+_native = _NotLoaded()
+
 
 def _stream():
     """Address of torch's current stream of the current device."""
@@ -47,6 +69,10 @@ def _need_gpu(*ts):
 
 
 def rms_norm(x, w, eps=1e-5, out=None):
+    if out is None:
+        y = _native.rms_norm(x, w, eps)
+        if y is not None:
+            return y
     _need_gpu(x, w)
     y = torch.empty_like(x) if out is None else out
     cols = x.shape[-1]
@@ -76,6 +102,10 @@ def rms_norm_quantize(x, w, eps=1e-5):
 
 
 def softmax(x, axis=-1, causal=False, out=None):
+    if out is None:
+        y = _native.softmax(x, axis, causal)
+        if y is not None:
+            return y
     _need_gpu(x)
     axis = axis % x.dim()
     pre = math.prod(x.shape[:axis])
@@ -89,6 +119,10 @@ def softmax(x, axis=-1, causal=False, out=None):
 
 
 def rope(x, pos, theta=10000.0, out=None):
+    if out is None:
+        y = _native.rope(x, pos, theta)
+        if y is not None:
+            return y
     _need_gpu(x, pos)
     assert pos.dtype == torch.int64
     batch, seq, heads, dim = x.shape
@@ -100,6 +134,10 @@ def rope(x, pos, theta=10000.0, out=None):
 
 
 def dequantize_linear(x, scale, zp=None, axis=1, out=None):
+    if out is None:
+        y = _native.dequantize_linear(x, scale, zp, axis)
+        if y is not None:
+            return y
     _need_gpu(x, scale, zp)
     assert scale.dtype == torch.float32
     per_axis = int(scale.numel() != 1)
@@ -117,6 +155,10 @@ def dequantize_linear(x, scale, zp=None, axis=1, out=None):
 
 def dynamic_quantize_linear(x, out=None, workspace=None):
     """x float32 (any shape) -> (y uint8 like x, scale float32 [1], zero_point uint8 [1])."""
+    if out is None and workspace is None:
+        y = _native.dynamic_quantize_linear(x)
+        if y is not None:
+            return y
     _need_gpu(x)
     assert x.dtype == torch.float32 and x.is_contiguous()
     n = x.numel()
@@ -164,6 +206,10 @@ def matmul(a, b, c=None, trans_a=False, trans_b=False, alpha=1.0, beta=1.0, out=
     """Y = alpha * op(A) @ op(B) + beta * C.  a [..., m, k] ([..., k, m] when trans_a), b [..., k, n]
     ([..., n, k] when trans_b), batch dimensions broadcast; c broadcasts to [m, n] (any leading
     dimensions of size 1) or has the output's full shape.  float32/float64/float16/bfloat16."""
+    if out is None and workspace is None:
+        y = _native.matmul(a, b, c, trans_a, trans_b, alpha, beta)
+        if y is not None:
+            return y
     _need_gpu(a, b, c)
     assert a.dtype == b.dtype and a.is_contiguous() and b.is_contiguous()
     m, k = (a.shape[-1], a.shape[-2]) if trans_a else (a.shape[-2], a.shape[-1])
@@ -233,6 +279,10 @@ def transpose_info(shape, perm, itemsize):
 
 def transpose(x, perm, out=None):
     """Contiguous x with its dimensions permuted (any dtype: bytes are moved)."""
+    if out is None:
+        y = _native.transpose(x, perm)
+        if y is not None:
+            return y
     _need_gpu(x)
     assert x.is_contiguous() and sorted(perm) == list(range(x.dim()))
     rank, si, so, block, count = _transpose_digest(tuple(x.shape), tuple(perm), x.element_size())
@@ -262,6 +312,10 @@ def _pointer_array(tensors):
 
 def split(x, sizes, axis, outs=None):
     """The parts of x along `axis` with the given sizes, each contiguous (any dtype: bytes are moved)."""
+    if outs is None:
+        y = _native.split(x, sizes, axis)
+        if y is not None:
+            return y
     _need_gpu(x)
     axis %= x.dim()
     assert sum(sizes) == x.shape[axis]
@@ -373,6 +427,10 @@ def matmul_integer(a, b, a_zp=None, b_zp=None, out=None, dequant_scale=None):
     """a [..., m, k], b [..., k, n] (uint8/int8).  Zero points: None, one element, or one per
     (batch, row) of the operand as the reference's CPU kernel reads them.  dequant_scale (float32,
     one element or n): the result leaves as float32 = float(sum) * scale instead of int32."""
+    if out is None:
+        y = _native.matmul_integer(a, b, a_zp, b_zp, dequant_scale)
+        if y is not None:
+            return y
     _need_gpu(a, b, a_zp, b_zp, dequant_scale)
     m, k = a.shape[-2:]
     k2, n = b.shape[-2:]
@@ -427,6 +485,10 @@ def attention_kvcache(q, k, v, k_cache=None, v_cache=None, past_lens=None, scale
                       workspace=None, sync_state=None):
     """q [N,H,seq,D]; k, v [N,Hkv,seq,D]; caches [N,Hkv,cap,D] are updated in place;
     past_lens: int64 device tensor with 1 or N elements (None = 0)."""
+    if out is None and workspace is not None:
+        o = _native.attention_kvcache(q, k, v, k_cache, v_cache, past_lens, scale, workspace, sync_state)
+        if o is not None:
+            return o
     _need_gpu(q, k, v, k_cache, v_cache, past_lens)
     N, H, seq, D = q.shape
     Hkv = k.shape[1]

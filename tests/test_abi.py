@@ -69,3 +69,17 @@ def test_product_package_does_not_touch_the_oracle():
                 src = open(os.path.join(dirpath, f)).read()
                 assert not re.search(r"^\s*(import|from)\s+oracle\b", src, flags=re.M), f
                 assert "liboracle" not in src and "oracle.h" not in src, f
+
+
+def test_native_calls_leave_what_they_do_not_handle_to_python():
+    import torch
+
+    from refactorgraph_amd import ops
+    x, w = torch.ones(4, 8), torch.ones(8)
+    calls = ops._native  # (host tensors, no tensors at all, wrong kinds of arguments: None, and nothing is called)
+    assert calls.rms_norm(x, w, 1e-5) is None and calls.rms_norm(None, w, 1e-5) is None
+    assert calls.matmul(x, x, None, False, True, 1.0, 1.0) is None and calls.transpose(x, (1, 0)) is None
+    assert calls.split(x, [1, 3], 0) is None and calls.softmax(x, -1, False) is None
+    assert calls.attention_kvcache(x, x, x, None, None, None, None, x, None) is None
+    with pytest.raises(TypeError):
+        calls.rms_norm(x, w)

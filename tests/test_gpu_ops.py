@@ -4,6 +4,7 @@ Bars: bit-exact for MatMulInteger / DequantizeLinear; <= 1e-5 relative for fp32 
 and fp32 Softmax; <= 2e-3 absolute for fp16 paths (oracle in fp32 on up-cast inputs).
 """
 import ctypes as C
+import itertools
 import json
 import math
 import os
@@ -1897,3 +1898,87 @@ def test_matmul_one_to_four_rows_matrix_vector(m, k, n, dt):
     want = ai.astype(np.int64) @ wi.astype(np.int64).T
     if np.max(np.abs(want)) < (2048 if name == "fp16" else 256):
         assert np.array_equal(f(ops.matmul(dev(ai).to(dt), dev(wi).to(dt), trans_b=True)), want.astype(np.float32))
+
+
+# ------------------------------------------------------------------ the calls in native code
+
+class _InPython:
+    """Takes the place of the native calls: declines every one of them."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _calls_both_ways():
+    g = torch.Generator(device=DEV).manual_seed(91)
+    r = lambda *shape, dt=torch.float16: torch.randn(*shape, generator=g, device=DEV).to(dt)
+    u = lambda *shape, dt=torch.uint8: torch.randint(0, 120, shape, generator=g, device=DEV).to(dt)
+    x, w = r(3, 5, 64), r(64)
+    for t in (x, x.float(), x.bfloat16()):
+        yield "rms_norm", (t, w.to(t.dtype)), {}
+        yield "softmax", (t,), {}
+        yield "softmax", (t, 1), {}
+        yield "softmax", (t, -1, True), {}
+        yield "softmax", (t, -4), {}
+    yield "rope", (r(2, 3, 4, 64), torch.arange(6, device=DEV).view(2, 3)), {}
+    yield "rope", (r(2, 3, 4, 64), torch.arange(3, device=DEV), 500.0), {}
+    for zp in (None, u(7, dt=torch.int8)):
+        yield "dequantize_linear", (u(3, 7, 5, dt=torch.int8), r(7, dt=torch.float32), zp), {"axis": -2}
+    yield "dequantize_linear", (u(9), r(1, dt=torch.float32)), {}
+    yield "dynamic_quantize_linear", (r(3, 77, dt=torch.float32),), {}
+    a, b = r(2, 6, 64), r(2, 64, 32)
+    for c in (None, r(32), r(6, 1), r(6, 32), r(1, 1, 32), r(2, 6, 32), r(2, 1, 1), torch.ones((), device=DEV).half(), r(1, 6, 1)):
+        yield "matmul", (a, b, c), {"alpha": 0.5, "beta": 2}
+    yield "matmul", (a[0], b[0], r(6, 32)), {}
+    yield "matmul", (a[0].t().contiguous(), b[0].t().contiguous()), {"trans_a": True, "trans_b": True}
+    yield "matmul", (a, b[0]), {}                       # one matrix for all of a batch: left to Python
+    yield "matmul", (a.view(2, 1, 6, 64), b.view(1, 2, 64, 32)), {}
+    yield "matmul", (r(1, 4096), r(4096, 512)), {}      # with a workspace
+    yield "matmul", (r(4, 64, dt=torch.float64), r(64, 32, dt=torch.float64)), {}
+    yield "matmul", (a, b), {"trans_a": 0}
+    ia, ib = u(2, 6, 64), u(2, 64, 32, dt=torch.int8)
+    for az, bz in ((None, None), (u(1), u(1, dt=torch.int8)), (u(12), u(128, dt=torch.int8))):
+        yield "matmul_integer", (ia, ib, az, bz), {}
+        yield "matmul_integer", (ia, ib, az, bz), {"dequant_scale": r(32, dt=torch.float32)}
+    yield "matmul_integer", (ia, ib[0]), {"dequant_scale": r(1, dt=torch.float32)}
+    for shape in ((2, 3, 4, 5), (1, 3, 1, 5), (7, 1, 2), (4, 1, 1), (6,), (1,), ()):
+        for perm in itertools.permutations(range(len(shape))):
+            for dt in (torch.float16, torch.int64, torch.bool):
+                yield "transpose", (r(*shape).to(dt) if shape else r(1).to(dt)[0], perm), {}
+    yield "transpose", (x, [2, 0, 1]), {}
+    yield "split", (x, [2, 1, 2], 1), {}
+    yield "split", (x, [64], -1), {}
+    yield "split", (x, (1, 2), 0), {}
+
+
+def test_native_calls_do_what_the_python_ones_do(monkeypatch):
+    native = ops._native
+    for name, args, kw in _calls_both_ways():
+        monkeypatch.setattr(ops, "_native", native)
+        got = getattr(ops, name)(*args, **kw)
+        monkeypatch.setattr(ops, "_native", _InPython())
+        want = getattr(ops, name)(*args, **kw)
+        pairs = [(got, want)] if isinstance(want, torch.Tensor) else list(zip(got, want, strict=True))
+        assert type(got) is type(want), name
+        for x, y in pairs:
+            where = (name, [tuple(t.shape) if isinstance(t, torch.Tensor) else t for t in args], kw)
+            assert x.shape == y.shape and x.stride() == y.stride() and x.dtype == y.dtype and x.device == y.device, where
+            assert torch.equal(x, y), where
+
+
+def test_native_calls_refuse_what_the_python_ones_refuse(monkeypatch):
+    x, w = torch.randn(4, 64, device=DEV).half(), torch.randn(64, 8, device=DEV).half()
+    calls = [("rms_norm", (x.cpu(), w)), ("rms_norm", (x.t(), w)), ("rms_norm", (x.to(torch.complex64), w)), ("softmax", (x[:, ::2],)),
+             ("matmul", (x, w.float())), ("matmul", (x, x)), ("matmul", (x, w, x)), ("matmul", (x, w, w.t())),
+             ("transpose", (x, (0, 0))), ("transpose", (x, (1,))), ("split", (x, [3, 2], 0)), ("rope", (x, x)),
+             ("dequantize_linear", (x, x[0].float()[:3])), ("dynamic_quantize_linear", (x,)), ("matmul_integer", (x.byte(), x.byte())),
+             ("rms_norm", (None, w)), ("rms_norm", (x.byte(), w))]
+    native = ops._native
+    for name, args in calls:
+        raised = []
+        for way in (native, _InPython()):
+            monkeypatch.setattr(ops, "_native", way)
+            with pytest.raises(Exception) as e:
+                getattr(ops, name)(*args)
+            raised.append((e.type, str(e.value)))
+        assert raised[0] == raised[1], name
