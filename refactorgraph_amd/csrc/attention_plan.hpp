@@ -46,6 +46,22 @@ inline bool prefill_pays(size_t N, size_t n_head, size_t n_kv_head, size_t seq, 
 constexpr uint64_t kSplitMinTiles = 8;  // key tiles (of 64) of the capacity per range of shared keys, at least
 constexpr uint64_t kSplitMax = 32;      // ranges per item, at most
 
+// Ranges per item of a launch of attn_prefill: as many as bring it to the `resident` workgroups (two a CU), or one.  A workgroup
+// takes about 1.7 us a tile alone on its CU and 3 us beside another one, the records and their merge 10 us together ([1, 1000
+// rows, 32/8 heads] 33 us in two ranges, 29 unshared; [4, 128 rows] 19 and 8; [2, 300 rows] 16 either way).  Half of the capacity
+// behind the new rows stands for the history.
+inline uint64_t tiled_splits(uint64_t items, uint64_t seq, uint64_t cap, uint64_t resident, uint64_t room) {
+    uint64_t splits = items ? resident / items : 1;
+    const uint64_t by_tiles = (cap + 63) / 64 / kSplitMinTiles, by_room = items ? room / items : 0;
+    if (splits > by_tiles) splits = by_tiles;
+    if (splits > kSplitMax) splits = kSplitMax;
+    if (splits > by_room) splits = by_room;
+    if (splits < 2) return 1;
+    const double tiles = static_cast<double>(seq + (cap > seq ? cap - seq : 0) / 2) / 64 + 1;
+    const double shared = 10 + tiles / static_cast<double>(splits) * (2 * items * splits > resident ? 3.0 : 1.7);
+    return shared < 1.7 * tiles ? splits : 1;
+}
+
 // Ranges per item of a launch of attn_prefill_wide: as many as bring it to a workgroup per CU, while the records (`room` of
 // them, of an item and range) fit the workspace.
 inline uint64_t wide_splits(uint64_t items, uint64_t cap, uint64_t cus, uint64_t room) {

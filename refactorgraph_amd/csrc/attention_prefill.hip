@@ -156,7 +156,7 @@ struct PrefillPlan {
     uint32_t group;        // query heads per kv head
     uint32_t head_chunks;  // group / HW
     uint32_t q_tiles;      // query tiles (of ROWS rows) per stream
-    uint32_t pairs;        // (q_tiles + 1) / 2, SPLIT: q_tiles: workgroups that share a stream
+    uint32_t pairs;        // (q_tiles + 1) / 2, SPLIT and `one`: q_tiles: workgroups that share a stream
     uint32_t xcds;         // 8 when the streams divide evenly over the XCDs, else 1
     uint32_t spx;          // streams per XCD
     uint32_t groups;       // sets of `pairs` workgroups per XCD; set g walks streams g, g + groups, ...
@@ -165,6 +165,7 @@ struct PrefillPlan {
     uint32_t magic_chunks, magic_hkv;
     // key ranges per item (SPLIT instances): the streams above are then (stream, range) pairs, range fastest
     uint32_t splits, magic_splits;
+    uint32_t one;  // a workgroup takes one query tile of a stream, not a pair (SPLIT: always)
     float *part;  // partial results of the ranges, kPartFloats(DH) per item and range
 };
 
@@ -242,17 +243,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
         raw_past = 0;
         while (en_k < plan.spx) {
             const uint32_t heavy = plan.q_tiles - 1 - pj;
-            // (SPLIT: one query tile a stream, every other set from the other end, so that the two workgroups of a CU
+            // (SPLIT, plan.one: one query tile a stream, every other set from the other end, so that the two workgroups of a CU
             // get a long and a short one under a causal prompt)
-            const uint32_t qt = SPLIT ? ((set & 1) ? heavy : pj) : en_sub == 0 ? heavy : pj;
-            const bool ok = SPLIT || en_sub == 0 || pj != heavy;
+            const bool one = SPLIT || plan.one;
+            const uint32_t qt = one ? ((set & 1) ? heavy : pj) : en_sub == 0 ? heavy : pj;
+            const bool ok = one || en_sub == 0 || pj != heavy;
             uint32_t stream = en_k * plan.xcds + xcd;
             if constexpr (SPLIT) {
                 const uint32_t whole = div_magic(stream, plan.magic_splits);
                 it.ks = stream - whole * plan.splits;
                 stream = whole;
             }
-            if (!SPLIT && en_sub == 0) {
+            if (!one && en_sub == 0) {
                 en_sub = 1;
             } else {
                 en_sub = 0;
@@ -1323,26 +1325,16 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
     plan.pairs = (plan.q_tiles + 1) / 2;
     uint64_t streams = static_cast<uint64_t>(a.N) * a.Hkv * plan.head_chunks;
     if (streams * plan.pairs > 0x7fffffffu) return RG_HIP_E_UNSUPPORTED;
-    // Few items and room for a long history: the keys of an item are shared between workgroups, as many as bring
-    // the launch to the workgroups that are resident together, each with at least kSplitMinTiles tiles of the
-    // capacity, while the records fit the workspace (head dims 64 and 128)
+    // Few items: the keys of an item are shared between workgroups where that is expected to pay (head dims 64 and 128), or each
+    // has a workgroup, on a CU, of its own (with pairs of a heavy and a light one half of the CUs had none)
     plan.splits = 1;
-    const uint64_t items = streams * plan.q_tiles;
+    const uint64_t items = streams * plan.q_tiles, resident = resident_prefill_workgroups<T, HW, DH>();
     if constexpr (DH == 64 || DH == 128) {
-        const uint64_t resident = resident_prefill_workgroups<T, HW, DH>();
-        const uint64_t cap_tiles = (static_cast<uint64_t>(a.cap) + BN - 1) / BN;
-        uint64_t splits = items ? resident / items : 1;
-        if (splits > cap_tiles / kSplitMinTiles) splits = cap_tiles / kSplitMinTiles;
-        if (splits > kSplitMax) splits = kSplitMax;
-        const uint64_t room = a.part ? a.part_bytes / (items * part_floats(DH) * sizeof(float)) : 0;
-        if (splits > room) splits = room;
-        if (splits >= 2 && streams * splits * plan.q_tiles <= 0x7fffffffu) {
-            plan.splits = static_cast<uint32_t>(splits);
-            // a query tile per workgroup: with a pair each only half of the resident workgroups were launched, one
-            // wavefront on a SIMD (128 new rows behind 16384, 32 heads: 64.7 -> 50.2 us, 690 TFLOP/s)
-            plan.pairs = plan.q_tiles;
-        }
+        const uint64_t room = a.part ? a.part_bytes / (part_floats(DH) * sizeof(float)) : 0;
+        plan.splits = static_cast<uint32_t>(tiled_splits(items, a.seq, a.cap, resident, room));
     }
+    plan.one = plan.splits == 1 && 2 * items <= resident;
+    if (plan.splits > 1 || plan.one) plan.pairs = plan.q_tiles;
     plan.magic_splits = plan.splits > 1 ? static_cast<uint32_t>((1ull << 32) / plan.splits + 1) : 0;
     plan.part = a.part;
     const uint64_t whole_streams = streams;
