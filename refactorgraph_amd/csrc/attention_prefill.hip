@@ -165,7 +165,8 @@ struct PrefillPlan {
     uint32_t magic_chunks, magic_hkv;
     // key ranges per item (SPLIT instances): the streams above are then (stream, range) pairs, range fastest
     uint32_t splits, magic_splits;
-    uint32_t one;  // a workgroup takes one query tile of a stream, not a pair (SPLIT: always)
+    uint32_t one;        // 1: a workgroup takes one query tile of a stream, the second one of a pair (SPLIT: 0)
+    uint32_t last_tile;  // the first of a pair is last_tile - the second: q_tiles - 1, far from any second one if `one`
     float *part;  // partial results of the ranges, kPartFloats(DH) per item and range
 };
 
@@ -235,29 +236,28 @@ __global__ __launch_bounds__(256, 2) void attn_prefill(const PrefillArgs a, cons
     // tiles q_tiles - 1 - j and j of each of them (the heavy one first; SPLIT: one of the two).
     const uint32_t xcd = uni(blockIdx.x % plan.xcds), lw = uni(blockIdx.x / plan.xcds);
     const uint32_t pj = uni(lw % plan.pairs), set = uni(lw / plan.pairs);
-    uint32_t en_k = set, en_sub = 0;
+    uint32_t en_k = set, en_sub = plan.one;
     // The history length of an item's batch row is read when the item is enumerated and clamped
     // when the item becomes the current one (an item later), so that nobody waits for the load.
     auto next_item = [&](uint64_t &raw_past) __attribute__((always_inline)) -> Item {
         Item it{0, 0, kNoItem, 0, 0};
         raw_past = 0;
         while (en_k < plan.spx) {
-            const uint32_t heavy = plan.q_tiles - 1 - pj;
-            // (SPLIT, plan.one: one query tile a stream, every other set from the other end, so that the two workgroups of a CU
+            const uint32_t heavy = plan.last_tile - pj;
+            // (SPLIT: one query tile a stream, every other set from the other end, so that the two workgroups of a CU
             // get a long and a short one under a causal prompt)
-            const bool one = SPLIT || plan.one;
-            const uint32_t qt = one ? ((set & 1) ? heavy : pj) : en_sub == 0 ? heavy : pj;
-            const bool ok = one || en_sub == 0 || pj != heavy;
+            const uint32_t qt = SPLIT ? ((set & 1) ? heavy : pj) : en_sub == 0 ? heavy : pj;
+            const bool ok = SPLIT || en_sub == 0 || pj != heavy;
             uint32_t stream = en_k * plan.xcds + xcd;
             if constexpr (SPLIT) {
                 const uint32_t whole = div_magic(stream, plan.magic_splits);
                 it.ks = stream - whole * plan.splits;
                 stream = whole;
             }
-            if (!one && en_sub == 0) {
+            if (!SPLIT && en_sub == 0) {
                 en_sub = 1;
             } else {
-                en_sub = 0;
+                en_sub = plan.one;
                 en_k += plan.groups;
             }
             if (!ok) continue;
@@ -1335,6 +1335,7 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
     }
     plan.one = plan.splits == 1 && 2 * items <= resident;
     if (plan.splits > 1 || plan.one) plan.pairs = plan.q_tiles;
+    plan.last_tile = plan.one ? 0x7fffffffu : plan.q_tiles - 1;
     plan.magic_splits = plan.splits > 1 ? static_cast<uint32_t>((1ull << 32) / plan.splits + 1) : 0;
     plan.part = a.part;
     const uint64_t whole_streams = streams;
