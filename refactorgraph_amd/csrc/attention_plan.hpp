@@ -47,10 +47,11 @@ constexpr uint64_t kSplitMinTiles = 8;  // key tiles (of 64) of the capacity per
 constexpr uint64_t kSplitMax = 32;      // ranges per item, at most
 
 // Ranges per item of a launch of attn_prefill: as many as bring it to the `resident` workgroups (two a CU), or one.  A workgroup
-// takes about 1.7 us a tile alone on its CU and 3 us beside another one, the records and their merge 10 us together ([1, 1000
-// rows, 32/8 heads] 33 us in two ranges, 29 unshared; [4, 128 rows] 19 and 8; [2, 300 rows] 16 either way).  Half of the capacity
-// behind the new rows stands for the history.
-inline uint64_t tiled_splits(uint64_t items, uint64_t seq, uint64_t cap, uint64_t resident, uint64_t room) {
+// takes about 1.7 us a tile alone on its CU and 3 us beside another one, the records and their merge 9 us together; at head dim 64
+// 1.25, 2.2 and 5.  In two ranges and unshared: [1, 1000 rows, 32/8 heads] 34 and 29 us, [4, 128] 19 and 8, [1, 300] 16 and 12;
+// head dim 64, [3, 55 rows, 24/8 heads] behind 914 positions 17 and 22.  Half of the capacity behind the new rows stands for the
+// history, which is device data.
+inline uint64_t tiled_splits(uint64_t items, uint64_t seq, uint64_t cap, uint64_t resident, uint64_t room, uint64_t dim) {
     uint64_t splits = items ? resident / items : 1;
     const uint64_t by_tiles = (cap + 63) / 64 / kSplitMinTiles, by_room = items ? room / items : 0;
     if (splits > by_tiles) splits = by_tiles;
@@ -58,8 +59,8 @@ inline uint64_t tiled_splits(uint64_t items, uint64_t seq, uint64_t cap, uint64_
     if (splits > by_room) splits = by_room;
     if (splits < 2) return 1;
     const double tiles = static_cast<double>(seq + (cap > seq ? cap - seq : 0) / 2) / 64 + 1;
-    const double shared = 10 + tiles / static_cast<double>(splits) * (2 * items * splits > resident ? 3.0 : 1.7);
-    return shared < 1.7 * tiles ? splits : 1;
+    const double alone = dim <= 64 ? 1.25 : 1.7, beside = dim <= 64 ? 2.2 : 3.0, merge = dim <= 64 ? 5 : 9;
+    return merge + tiles / static_cast<double>(splits) * (2 * items * splits > resident ? beside : alone) < alone * tiles ? splits : 1;
 }
 
 // Ranges per item of a launch of attn_prefill_wide: as many as bring it to a workgroup per CU, while the records (`room` of

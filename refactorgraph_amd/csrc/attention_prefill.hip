@@ -1331,7 +1331,7 @@ int launch_hw(const PrefillArgs &a, hipStream_t s) {
     const uint64_t items = streams * plan.q_tiles, resident = resident_prefill_workgroups<T, HW, DH>();
     if constexpr (DH == 64 || DH == 128) {
         const uint64_t room = a.part ? a.part_bytes / (part_floats(DH) * sizeof(float)) : 0;
-        plan.splits = static_cast<uint32_t>(tiled_splits(items, a.seq, a.cap, resident, room));
+        plan.splits = static_cast<uint32_t>(tiled_splits(items, a.seq, a.cap, resident, room, DH));
     }
     plan.one = plan.splits == 1 && 2 * items <= resident;
     if (plan.splits > 1 || plan.one) plan.pairs = plan.q_tiles;
